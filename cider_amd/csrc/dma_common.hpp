@@ -58,6 +58,16 @@ __device__ __forceinline__ void dma16s_nt(const void* base, uint32_t off, uint32
       : "memory", "m0");
 }
 
+// 4 bytes per lane from base + off to LDS at lds_base + 4 * lane.
+__device__ __forceinline__ void dma4s(const void* base, uint32_t off, uint32_t lds_base) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "global_load_lds_dword %0, %1"
+      :
+      : "v"(off), "s"(base), "s"(lds_base)
+      : "memory", "m0");
+}
+
 // Waits until at most N vector-memory loads of this wave are outstanding
 // (they complete in order).
 template <int N>

@@ -542,13 +542,9 @@ hipError_t pick_tile(const GemmArgs& a, hipStream_t s) {
   // N=10240 K=2560: 33.5 vs 35.8 us; int4: M=1024 N=10240 K=2560: 38.6 vs
   // 42.8 us).  The mixed grid below reads candidates 0 and 1.
   struct Cand { int bm, bn; double rate; };
-  static const Cand c8[] = {{256, 256, 1.0},   {128, 256, 0.87}, {128, 128, 0.75},
-                            {128, 64, 0.517},  {64, 128, 0.508}, {64, 64, 0.40},
-                            {192, 256, 0.90}};
-  static const Cand c4[] = {{256, 256, 1.0},   {128, 256, 0.77}, {128, 128, 0.60},
+  static const Cand cands[] = {{256, 256, 1.0},   {128, 256, 0.77}, {128, 128, 0.60},
                             {128, 64, 0.41},   {64, 128, 0.40},  {64, 64, 0.32},
                             {192, 256, 0.92}};
-  const Cand* cands = WF == W_I4 ? c4 : c8;
   const int cus = num_cus();
   int best = 0;
   double best_cost = 1e300;
@@ -594,6 +590,64 @@ hipError_t pick_tile(const GemmArgs& a, hipStream_t s) {
   if (bm == 128) return run_dma<128, 64, 128, EPI, WF>(a, s);
   if (bn == 128) return run_dma<64, 128, 128, EPI, WF>(a, s);
   return run_dma<64, 64, 128, EPI, WF>(a, s);
+}
+
+// Time (us) of a grid of small tiles, fitted as plan_cost in gemm_pp.hip is,
+// to the same shapes (rms error 2-7 %): the rounds of
+// tiles one after the other, or the chip's rate, in the fourth-power mean.
+struct TileCost {
+  int bm, bn;
+  double stage, fill, full, launch;
+};
+
+double tile_cost(const TileCost& c, int M, int N, int nk, int cus) {
+  const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+  const double crit = (double)((tiles + cus - 1) / cus) * (nk * c.stage + c.fill);
+  const double work = (double)tiles / cus * c.bm * c.bn / 65536.0;
+  const double power = work * nk * c.full + c.launch;
+  const double c2 = crit * crit, p2 = power * power;
+  return sqrt(sqrt(c2 * c2 + p2 * p2));
+}
+
+// int8 weights: the ping-pong kernel (gemm_pp.hip) against the tiles that
+// serve few rows or columns, by estimated time.  Over 108 measured shapes (M =
+// 65 .. 2048) the choice is within 1 % of the best of all candidates.  128 x
+// 256 tiles are a candidate where they make one round only (M=300 N=12288
+// K=4096: 24.6 us against 28.8 in ping-pong tiles of 64 rows); in more rounds
+// the ping-pong kernel was ahead everywhere.  The measured operands stayed in
+// the caches between calls; on weights that do not, the deeper rings of the
+// other tiles gain some 3 % on the ping-pong kernel (M=512 N=12288 K=2048
+// inside a model layer), hence the margin.
+template <int EPI>
+hipError_t pick_tile_i8(const GemmArgs& a, hipStream_t s) {
+  static const TileCost cands[] = {{128, 256, 0.545, 3.30, 1.685, 7.53},
+                                   {128, 128, 0.326, 5.73, 2.164, 1.74},
+                                   {128, 64, 0.286, 3.60, 2.427, 2.79},
+                                   {64, 128, 0.301, 3.96, 3.171, 1.63},
+                                   {64, 64, 0.197, 2.85, 2.468, 3.36}};
+  const int cus = num_cus();
+  int best = 0;
+  double best_cost = 1e300;
+  for (int i = 0; i < 5; ++i) {
+    if (i == 0 && (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus) continue;
+    const double cost = tile_cost(cands[i], a.M, a.N, a.K / 128, cus);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = i;
+    }
+  }
+  if (pp_supported(a, EPI, W_I8)) {
+    PpPlan pl;
+    if (pp_plan(a.M, a.N, a.K, W_I8, pl) < 0.96 * best_cost)
+      return launch_gemm_pp(a, EPI, W_I8, pl, s);
+  }
+  switch (best) {
+    case 0: return run_dma<128, 256, 128, EPI>(a, s);
+    case 1: return run_dma<128, 128, 128, EPI>(a, s);
+    case 2: return run_dma<128, 64, 128, EPI>(a, s);
+    case 3: return run_dma<64, 128, 128, EPI>(a, s);
+    default: return run_dma<64, 64, 128, EPI>(a, s);
+  }
 }
 
 }  // namespace
@@ -713,8 +767,8 @@ hipError_t launch_gemm_splitk(const GemmArgs& a, int S, int32_t* part, hipStream
 // K % 128 == 0, N % 8 == 0, 16-byte aligned operands (launch_gemm checks).
 hipError_t launch_gemm_dma(const GemmArgs& a, int epi, int wf, hipStream_t s) {
   if (wf == W_I4) return pick_tile<EPI_PC, W_I4>(a, s);
-  if (epi == EPI_I32) return pick_tile<EPI_I32, W_I8>(a, s);
-  return pick_tile<EPI_PC, W_I8>(a, s);
+  if (epi == EPI_I32) return pick_tile_i8<EPI_I32>(a, s);
+  return pick_tile_i8<EPI_PC>(a, s);
 }
 
 }  // namespace cider

@@ -42,6 +42,18 @@ hipError_t launch_skinny_dma(const GemmArgs& a, int wf, int epi, int gs, hipStre
 hipError_t launch_skinny(const GemmArgs& a, int wf, int epi, bool sw_half, int gs,
                          hipStream_t s);
 hipError_t launch_gemm_dma(const GemmArgs& a, int epi, int wf, hipStream_t s);
+// Persistent ping-pong GEMM (gemm_pp.hip): big tiles of 64 mb x 256 over rows
+// [0, m_split) and columns [0, n_split), small ones of 64 ms x 256 over the
+// rest (rows below m_split or columns right of n_split), the small ones on
+// workgroups s0 .. grid - 1.
+struct PpPlan {
+  int mb, ms, nbig, nsmall, m_split, n_split, s0, grid;
+};
+// Shapes and alignments it takes, the best plan for a shape (returns its
+// estimated time in us), and the launch.
+bool pp_supported(const GemmArgs& a, int epi, int wf);
+double pp_plan(int M, int N, int K, int wf, PpPlan& best);
+hipError_t launch_gemm_pp(const GemmArgs& a, int epi, int wf, const PpPlan& pl, hipStream_t s);
 // Split-K per-channel GEMM for shapes with few tiles (gemm_dma.hip): K slices
 // (1 = no split), the int32 partial bytes they need, and the launch (split
 // tiles into `part`, then the summing dequant into a.y).

@@ -1,0 +1,73 @@
+"""The ping-pong GEMM (cider_amd/csrc/gemm_pp.hip) at the sizes where its
+tiling can go wrong: one, one and a partial, and several rounds of tiles of
+each height, tiles moved inside at ragged rows and columns, rows and columns
+left to small tiles, even and odd numbers of k-stages, the shortest K.
+
+Bit-exact: the integer accumulators come from float64 products (exact below
+2^53), and the epilogue's three binary32 operations are done one by one.
+"""
+
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    import cider_amd as C
+
+DEV = "cuda"
+
+# (M, N, K); on 256 compute units, tile rows (big, small):
+SHAPES = [
+    (64, 256, 512),       # one tile of 64 rows
+    (100, 520, 640),      # 64 rows, the last tile row and column moved inside
+    (193, 2056, 1152),
+    (1000, 6152, 512),    # 128 rows
+    (1334, 6152, 640),    # 192 rows, one round
+    (3455, 6152, 512),    # 192 rows, several rounds
+    (1000, 12296, 640),   # 256 rows, one round
+    (2500, 10248, 1152),  # 256 rows, several rounds
+    (4096, 2056, 640),    # 192, then 64 for the last rows
+    (1601, 6152, 640),    # 192, then 128
+    (1601, 12296, 512),   # the same in two rounds
+    (2049, 6152, 640),    # 256, then 64
+    (2049, 12296, 512),
+    (3455, 12288, 640),   # 256, then 128
+    (4096, 12296, 640),   # 256 rows, the last columns in tiles of 128 rows
+]
+
+
+def ints(shape, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randint(-128, 128, shape, dtype=torch.int8, device=DEV, generator=g)
+
+
+def exact_product(a, b):
+    return a.double() @ b.double().t().contiguous()
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_int32_product(M, N, K):
+    a, b = ints((M, K), 1), ints((N, K), 2)
+    a[0], b[-1] = -128, -128  # the largest sums
+    out = C.int8_matmul_int32(a, b)
+    assert torch.equal(out.double(), exact_product(a, b))
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_perchannel_epilogue(M, N, K, bias):
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, w = ints((M, K), 4), ints((N, K), 5)
+    sa = torch.rand(M, device=DEV, generator=g) * 0.02 + 1e-3
+    sw = torch.rand(N, device=DEV, generator=g) * 1e-2 + 1e-4
+    sa[M - 1] = float("inf")  # an infinite row: inf, and NaN where the sum is 0
+    b = torch.randn(N, device=DEV, generator=g).half() if bias else None
+    y = C.perchannel_gemm(q, sa, w, sw, b)
+    e = exact_product(q, w).float() * sa[:, None]
+    e = e * sw
+    if bias:
+        e = e + b.float()
+    e = e.half()
+    assert torch.equal(y.view(torch.int16)[~e.isnan()], e.view(torch.int16)[~e.isnan()])
+    assert torch.equal(y.isnan(), e.isnan())

@@ -113,11 +113,11 @@ bool try_fused_gemv(const char* fn, const void* x, const cider::GemmArgs& g, int
 
 // Quantizes x into the workspace; returns q and sa pointers.
 int quantize_into_ws(const char* fn, const void* x, void* ws, int64_t M, int64_t K,
-                     hipStream_t s, int8_t** q, float** sa) {
+                     hipStream_t s, int8_t** q, float** sa, bool il = false) {
   *q = reinterpret_cast<int8_t*>(ws);
   *sa = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + align256((size_t)M * (size_t)K));
   return hip_status(cider::launch_quantize(reinterpret_cast<const uint16_t*>(x), *q, *sa,
-                                           (int)M, (int)K, s),
+                                           (int)M, (int)K, s, il),
                     fn);
 }
 
@@ -383,8 +383,9 @@ int cider_w4a8_linear(const void* x_f16, const uint8_t* w4_nk, const float* sw, 
   if (try_fused_gemv(fn, x_f16, gf, cider::W_I4, cider::EPI_PC, 0, s, &rc)) return rc;
   int8_t* q;
   float* sa;
-  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa));
-  cider::GemmArgs g{q, w4_nk, sa, sw, nullptr, y_f16, (int)M, (int)N, (int)K};
+  const bool il = aligned16(x_f16) && cider::w4_wants_il(gf);
+  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, il));
+  cider::GemmArgs g{q, w4_nk, sa, sw, nullptr, y_f16, (int)M, (int)N, (int)K, il};
   return hip_status(cider::launch_gemm(g, cider::W_I4, cider::EPI_PC, false, 0, s), fn);
 }
 

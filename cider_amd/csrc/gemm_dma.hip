@@ -1,8 +1,9 @@
-// Tiled int8 GEMM, main path for int8 weights (int32 and per-channel
-// epilogues) and int4 weights (per-channel, the reference W4A8) with
-// K % 128 == 0 and N % 8 == 0: operands stream global -> LDS by gfx950's
-// 16-byte LDS-DMA loads through a ring of k-stages, the MFMAs are
-// v_mfma_i32_32x32x32_i8, and the fp16 tile is staged through LDS so the
+// Tiled int8 GEMM for shapes with few rows or columns, where the 256-column
+// tiles of the ping-pong kernel (gemm_pp.hip) would leave CUs idle: int8
+// weights (int32 and per-channel epilogues) and int4 weights (per-channel, the
+// reference W4A8) with K % 128 == 0 and N % 8 == 0.  Operands stream global ->
+// LDS by gfx950's 16-byte LDS-DMA loads through a ring of k-stages, the MFMAs
+// are v_mfma_i32_32x32x32_i8, and the fp16 tile is staged through LDS so the
 // output is written in whole rows.
 //
 // Reference semantics are those of gemm.hip (same epilogues, same fp32
@@ -16,26 +17,17 @@
 // kernel does not take run the register-staged kernel of gemm.hip.)
 //
 // MI355X design
-//   * One workgroup per CU; tile BM (m) x BN (n) from {256 x 256, 192 x 256,
-//     128 x 256, 128 x 128, 128 x 64, 64 x 128, 64 x 64}, picked per shape by
-//     measured rate and the rounds the grid needs on the 256 CUs.  Waves: 2
-//     along m and NWV / 2 along n.  The 256-column tiles run NWV = 8 waves,
-//     two per SIMD: at 256 x 256 each wave owns 128 x 64 = 4 x 2 blocks of
-//     32 x 32 (16 int32 accumulators per lane per block, 128 registers), and
-//     while one wave of a SIMD waits on its DMA issue, fragment reads or
-//     epilogue, the other's MFMAs run.  That costs 1.5x the fragment reads of
-//     four 128 x 128 waves (LDS ~126 B/clk per CU at the full MFMA rate,
-//     against ~128 delivered) and measured faster anyway: uniform 256 x 256 at
-//     M=4096 N=10240 K=2560 113.8 -> 105.9 us, the mixed grid 104.4 -> 99.8
-//     us, M=8192 199.6 -> 188.0 us, int4 N=12288 K=4096 199.9 -> 190.3 us;
-//     192 x 256 and 128 x 256 4-10 %; N=2560 K=10240 level.  The smaller
-//     tiles keep four waves (2 x 2).  Weights are the MFMA A operand,
-//     activations the B operand.  A spill reload is a vector-memory load, and
-//     waiting for it waits for every DMA load in flight (one spilled build ran
-//     15 % slower).
+//   * One workgroup per CU; tile BM (m) x BN (n) from {128 x 256 (int8), 128 x
+//     128, 128 x 64, 64 x 128, 64 x 64}, picked per shape by a fitted time.
+//     Waves: 2 along m and NWV / 2 along n; 128 x 256 runs eight, two per
+//     SIMD (while one waits on its DMA issue, fragment reads or epilogue, the
+//     other's MFMAs run: 4-10 % over four), the smaller tiles four (2 x 2).
+//     Weights are the MFMA A operand, activations the B operand.  A spill
+//     reload is a vector-memory load, and waiting for it waits for every DMA
+//     load in flight (one spilled build ran 15 % slower).
 //   * K advances BK bytes per stage (128; 64 is kept for tuning); stage s
 //     lives in ring slot s % NS, NS = as many stages as fit the 160 KB LDS
-//     (2 at 256 x 256 x 128, 3 at 128 x 256, up to 8 for small tiles).  Each
+//     (3 at 128 x 256, up to 8 for small tiles).  Each
 //     wave moves its share of a stage with global_load_lds_dwordx4 (one
 //     instruction = 1 KB, written contiguously to LDS at M0): no VGPR
 //     staging, no ds_write.  The
@@ -49,15 +41,10 @@
 //     consumed, and this wave's share of DMA loads spread over the MFMAs.
 //     Left to itself, the compiler regroups the reads next to the MFMAs that
 //     consume them and exposes LDS latency at every sub-step.
-//   * With three or more ring slots, a stage's DMA loads are spread over
-//     SUBS sub-steps (the last of stage kt and the first ones of stage kt+1)
-//     instead of one: the CU's vector-memory path accepts one 1 KB load per
-//     ~23 cycles, and a whole stage's loads inside one sub-step stalled the
-//     issuing waves for ~440 of its 512 MFMA cycles (measured at 256 x 256).
-//     Two slots (int8 256 x 256) split a stage in two parts only: the second
-//     part, issued in the first sub-step of stage kt+1, must land by that
-//     stage's barrier.  int4 weights at 256 x 256 (three slots) issue a
-//     stage whole: 4 parts measured 25-40 % slower, 2 parts level.
+//   * A stage's DMA loads are spread over SUBS sub-steps (the last of stage kt
+//     and the first ones of stage kt+1) instead of one: the CU's vector-memory
+//     path accepts one 1 KB load per ~23 cycles, and a whole stage's loads
+//     inside one sub-step stall the issuing waves.
 //   * The one barrier per stage sits before its last sub-step: it publishes
 //     stage kt + 1 and frees the slot of stage kt, which then receives stage
 //     kt + NS.
@@ -72,8 +59,7 @@
 //     fp16 into a BM x BN LDS tile (rows padded by 16 bytes),
 //     then the workgroup stores whole 2*BN-byte rows with 16-byte lanes, so
 //     HBM sees full 128-byte lines instead of 32-byte row fragments.
-//   * int4 weights: a k-stage of a weight row is 64 bytes of nibbles (the ring
-//     then holds 3 stages at 256 x 256).  One ds_read_b128 per W block brings
+//   * int4 weights: a k-stage of a weight row is 64 bytes of nibbles.  One ds_read_b128 per W block brings
 //     the 32 nibbles of a pair of sub-steps; each sub-step's 16 are unpacked
 //     to int8 in registers (sign extension by xor/sub, byte permute) one
 //     sub-step ahead of their MFMAs.  The k mapping of a pair puts lane half h
@@ -112,7 +98,7 @@ struct DmaCfg {
   static constexpr int EPI_BYTES = OUT + SCL;
   static constexpr int SMEM = RING > EPI_BYTES ? RING : EPI_BYTES;
   static_assert(WI >= 1 && XI >= 1, "tile too small for the DMA split");
-  static_assert(NS >= 2, "ring needs two slots");
+  static_assert(NS >= 3, "ring slots");
   static_assert(SMEM <= kLdsBytes, "LDS budget");
   static_assert((NS - 2) * PS <= 63 && (NS - 1) * PS <= 63, "vmcnt range");
 };
@@ -137,9 +123,7 @@ using icst = std::integral_constant<int, V>;
 template <int BM, int BN, int BK, int EPI, int WF = W_I8, int NWV = 4>
 __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const int n0,
                                          int8_t* __restrict__ smem, const int kloop = 0) {
-  static_assert((BM == 64 || BM == 128 || BM == 192 || BM == 256) &&
-                    (BN == 64 || BN == 128 || BN == 256),
-                "tile shape");
+  static_assert((BM == 64 || BM == 128) && (BN == 64 || BN == 128 || BN == 256), "tile shape");
   static_assert(BK == 64 || BK == 128, "k stage");
   static_assert(WF == W_I8 || BK == 128, "int4 weights use 128-byte k-stages");
   using C = DmaCfg<BM, BN, BK, WF, NWV>;
@@ -230,12 +214,8 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
   // (PS per wave inside one sub-step) outrun what the CU's vector-memory path
   // accepts (one 1 KB load per ~23 cycles) and stall the issuing waves.  Every
   // part is out before the next barrier, so the counts waited for are as if
-  // the stage were issued at once.  With two slots (int8 256 x 256) the parts
-  // issued in stage kt+1 have only the sub-steps before its barrier to land:
-  // two parts measured 4-11% faster than one, four parts no faster than one.
-  // Exception, measured: int4 weights at 256 x 256 (three slots) ran 25-40%
-  // slower in 4 parts than whole, and level in 2.
-  constexpr int DS = (W4 && BM == 256) ? 1 : NS >= 3 ? SUBS : 2;
+  // the stage were issued at once.
+  constexpr int DS = SUBS;
 
   // One k sub-step in a fixed instruction order (sched_barrier): the TN*TM
   // MFMAs on fragments (wc, xc); between them the operands of the next
@@ -446,8 +426,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
             for (int r = 0; r < 4; ++r) {
               // The volatile asm keeps each path's int -> float conversions
               // inside that path: hoisted above the bias test, the converted
-              // accumulators were parked back in AGPRs and the 256 x 256 tile
-              // spilled.
+              // accumulators were parked back in AGPRs.
               int iv = acc[a][b][4 * g + r];
               asm volatile("" : "+v"(iv));
               float v = (float)iv * sam[b];
@@ -489,36 +468,6 @@ __global__ __launch_bounds__(64 * NWV, 1) void gemm_dma_kernel(const GemmArgs p)
   dma_tile<BM, BN, BK, EPI, WF, NWV>(p, m0, n0, smem);
 }
 
-// Two tile sizes in one grid, so that the last round of workgroups is not
-// half empty: the big workgroups take 256 x 256 tiles of columns [0, nsplit),
-// the small ones 128 x 256 tiles of columns [nsplit, N), twice as many tiles
-// of half the work.  Workgroups start in index order: [0, s1) small tiles
-// 0 .. s1-1, [s1, s1 + nbig) the big tiles, the rest the other small tiles.
-// With s1 = half the small tiles, half the CUs start on a small tile and run
-// half a tile out of phase with the other half from then on, so the tile
-// epilogues' output stores (a 256 x 256 tile writes 128 KB, a round of
-// tiles 32 MB at once, for about 4.6 us at M=4096 N=10240 K=2560) meet the
-// other half's k-loops instead of each other (that shape: 102.0 -> 95.9 us,
-// bit-identical).  Each region keeps its own XCD remap; s1 and nbig are
-// multiples of 8, so a region's index keeps the XCD of its workgroup.
-template <int EPI, int WF, int NWV = 4>
-__global__ __launch_bounds__(64 * NWV, 1) void gemm_dma_mixed_kernel(const GemmArgs p, int nbig,
-                                                                     int nsplit, int s1) {
-  constexpr int S1 = DmaCfg<256, 256, 128, WF, NWV>::SMEM,
-                S2 = DmaCfg<128, 256, 128, WF, NWV>::SMEM;
-  __shared__ __attribute__((aligned(1024))) int8_t smem[S1 > S2 ? S1 : S2];
-  const int b = blockIdx.x;
-  int m0, n0;
-  if (b >= s1 && b < s1 + nbig) {
-    tile_coords<256, 256>(xcd_remap(b - s1, nbig), p.M, 0, nsplit, m0, n0);
-    dma_tile<256, 256, 128, EPI, WF, NWV>(p, m0, n0, smem);
-  } else {
-    const int bs = b < s1 ? b : b - nbig;
-    tile_coords<128, 256>(xcd_remap(bs, gridDim.x - nbig), p.M, nsplit, p.N, m0, n0);
-    dma_tile<128, 256, 128, EPI, WF, NWV>(p, m0, n0, smem);
-  }
-}
-
 namespace {
 
 // 256-column tiles run eight waves (two per SIMD), the smaller tiles four.
@@ -528,68 +477,6 @@ hipError_t run_dma(const GemmArgs& a, hipStream_t s) {
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
   gemm_dma_kernel<BM, BN, BK, EPI, WF, NWV><<<tiles, 64 * NWV, 0, s>>>(a);
   return hipGetLastError();
-}
-
-template <int EPI, int WF>
-hipError_t pick_tile(const GemmArgs& a, hipStream_t s) {
-  // Estimated time = rounds x tile area / tile rate.  Rates are throughputs
-  // measured on MI355X relative to a 256 x 256 tile (= 1), with back-to-back
-  // launches, over M = 128 .. 8192 and (N, K) from (10240, 2560) to
-  // (4096, 12288).  A last round only partly full runs with less contention:
-  // it counts 0.6 + 0.4 x its occupancy.  Ties go to the earlier candidate.
-  // 192 x 256 (waves of 96 x 128) serves grids whose 256 x 256 tiles make one
-  // partial round (int8: M=4096 N=2560 K=10240: 97.3 vs 105.8 us; M=1024
-  // N=10240 K=2560: 33.5 vs 35.8 us; int4: M=1024 N=10240 K=2560: 38.6 vs
-  // 42.8 us).  The mixed grid below reads candidates 0 and 1.
-  struct Cand { int bm, bn; double rate; };
-  static const Cand cands[] = {{256, 256, 1.0},   {128, 256, 0.77}, {128, 128, 0.60},
-                            {128, 64, 0.41},   {64, 128, 0.40},  {64, 64, 0.32},
-                            {192, 256, 0.92}};
-  const int cus = num_cus();
-  int best = 0;
-  double best_cost = 1e300;
-  for (int i = 0; i < 7; ++i) {
-    const int64_t tiles =
-        (int64_t)((a.M + cands[i].bm - 1) / cands[i].bm) * ((a.N + cands[i].bn - 1) / cands[i].bn);
-    const int64_t full = tiles / cus, rest = tiles % cus;
-    const double rounds = (double)full + (rest ? 0.6 + 0.4 * (double)rest / cus : 0.0);
-    const double cost = rounds * cands[i].bm * cands[i].bn / cands[i].rate;
-    if (cost < best_cost * 0.999) {
-      best_cost = cost;
-      best = i;
-    }
-  }
-  // Mixed grid: when the 256 x 256 tiles leave a last round at most half
-  // full, made of whole tile columns, those columns can run as twice as many
-  // 128 x 256 tiles of half the length, so the last round is full and half
-  // as long.
-  {
-    const int tm = (a.M + 255) / 256, tn = (a.N + 255) / 256;
-    const int64_t T = (int64_t)tm * tn;
-    const int R = (int)(T % cus);
-    if (T > cus && R > 0 && 2 * R <= cus && R % tm == 0) {
-      const double tail = (0.6 + 0.4 * 2.0 * R / cus) * 128 * 256 / cands[1].rate;
-      if ((double)(T / cus) * 256 * 256 / cands[0].rate + tail < best_cost * 0.999) {
-        const int tail_cols = R / tm;
-        const int nsplit = (tn - tail_cols) * 256;
-        const int nbig = (int)(T - R);
-        const int nsmall = ((a.M + 127) / 128) * tail_cols;
-        // half the small tiles first (a multiple of 8), when the big region
-        // starts on an XCD boundary; otherwise all of them last
-        const int s1 = nbig % 8 == 0 ? nsmall / 2 / 8 * 8 : 0;
-        gemm_dma_mixed_kernel<EPI, WF, 8><<<nbig + nsmall, 512, 0, s>>>(a, nbig, nsplit, s1);
-        return hipGetLastError();
-      }
-    }
-  }
-  const int bm = cands[best].bm, bn = cands[best].bn;
-  if (bm == 256) return run_dma<256, 256, 128, EPI, WF>(a, s);
-  if (bm == 192) return run_dma<192, 256, 128, EPI, WF>(a, s);
-  if (bm == 128 && bn == 256) return run_dma<128, 256, 128, EPI, WF>(a, s);
-  if (bm == 128 && bn == 128) return run_dma<128, 128, 128, EPI, WF>(a, s);
-  if (bm == 128) return run_dma<128, 64, 128, EPI, WF>(a, s);
-  if (bn == 128) return run_dma<64, 128, 128, EPI, WF>(a, s);
-  return run_dma<64, 64, 128, EPI, WF>(a, s);
 }
 
 // Time (us) of a grid of small tiles, fitted as plan_cost in gemm_pp.hip is,
@@ -618,36 +505,60 @@ double tile_cost(const TileCost& c, int M, int N, int nk, int cus) {
 // the caches between calls; on weights that do not, the deeper rings of the
 // other tiles gain some 3 % on the ping-pong kernel (M=512 N=12288 K=2048
 // inside a model layer), hence the margin.
-template <int EPI>
-hipError_t pick_tile_i8(const GemmArgs& a, hipStream_t s) {
-  static const TileCost cands[] = {{128, 256, 0.545, 3.30, 1.685, 7.53},
-                                   {128, 128, 0.326, 5.73, 2.164, 1.74},
-                                   {128, 64, 0.286, 3.60, 2.427, 2.79},
-                                   {64, 128, 0.301, 3.96, 3.171, 1.63},
-                                   {64, 64, 0.197, 2.85, 2.468, 3.36}};
+constexpr TileCost kTilesI8[] = {{128, 256, 0.545, 3.30, 1.685, 7.53},
+                                 {128, 128, 0.326, 5.73, 2.164, 1.74},
+                                 {128, 64, 0.286, 3.60, 2.427, 2.79},
+                                 {64, 128, 0.301, 3.96, 3.171, 1.63},
+                                 {64, 64, 0.197, 2.85, 2.468, 3.36}};
+
+// int4 weights: the same rule; over 190 measured shapes 0.2 % off the best in
+// the geometric mean.  128 x 256 tiles were not ahead anywhere.
+constexpr TileCost kTilesI4[] = {{128, 128, 0.655, 4.75, 2.328, 4.35},
+                                 {128, 64, 0.373, 3.48, 2.612, 3.63},
+                                 {64, 128, 0.484, 3.40, 3.137, 4.08},
+                                 {64, 64, 0.348, 2.62, 3.034, 3.98}};
+
+// The best small tile and, where the ping-pong kernel takes the operands and
+// is ahead, its plan (returns true).
+template <int N>
+bool pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N], const TileCost** best,
+          PpPlan* pl) {
   const int cus = num_cus();
-  int best = 0;
   double best_cost = 1e300;
-  for (int i = 0; i < 5; ++i) {
-    if (i == 0 && (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus) continue;
-    const double cost = tile_cost(cands[i], a.M, a.N, a.K / 128, cus);
+  *best = nullptr;
+  for (const TileCost& c : cands) {
+    if (c.bn == 256 && (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus) continue;
+    const double cost = tile_cost(c, a.M, a.N, a.K / 128, cus);
     if (cost < best_cost) {
       best_cost = cost;
-      best = i;
+      *best = &c;
     }
   }
-  if (pp_supported(a, EPI, W_I8)) {
-    PpPlan pl;
-    if (pp_plan(a.M, a.N, a.K, W_I8, pl) < 0.96 * best_cost)
-      return launch_gemm_pp(a, EPI, W_I8, pl, s);
-  }
-  switch (best) {
-    case 0: return run_dma<128, 256, 128, EPI>(a, s);
-    case 1: return run_dma<128, 128, 128, EPI>(a, s);
-    case 2: return run_dma<128, 64, 128, EPI>(a, s);
-    case 3: return run_dma<64, 128, 128, EPI>(a, s);
-    default: return run_dma<64, 64, 128, EPI>(a, s);
-  }
+  return pp_supported(a, epi, wf) && pp_plan(a.M, a.N, a.K, wf, *pl) < 0.96 * best_cost;
+}
+
+template <int EPI>
+hipError_t launch_i8(const GemmArgs& a, hipStream_t s) {
+  const TileCost* c;
+  PpPlan pl;
+  if (pick(a, EPI, W_I8, kTilesI8, &c, &pl)) return launch_gemm_pp(a, EPI, W_I8, pl, s);
+  if (c->bn == 256) return run_dma<128, 256, 128, EPI>(a, s);
+  if (c->bm == 128 && c->bn == 128) return run_dma<128, 128, 128, EPI>(a, s);
+  if (c->bm == 128) return run_dma<128, 64, 128, EPI>(a, s);
+  if (c->bn == 128) return run_dma<64, 128, 128, EPI>(a, s);
+  return run_dma<64, 64, 128, EPI>(a, s);
+}
+
+// x_il says that w4_wants_il chose the ping-pong kernel for this call.
+hipError_t launch_i4(const GemmArgs& a, hipStream_t s) {
+  const TileCost* c;
+  PpPlan pl;
+  const bool pp = pick(a, EPI_PC, W_I4, kTilesI4, &c, &pl);
+  if (a.x_il) return pp ? launch_gemm_pp(a, EPI_PC, W_I4, pl, s) : hipErrorInvalidValue;
+  if (c->bm == 128 && c->bn == 128) return run_dma<128, 128, 128, EPI_PC, W_I4>(a, s);
+  if (c->bm == 128) return run_dma<128, 64, 128, EPI_PC, W_I4>(a, s);
+  if (c->bn == 128) return run_dma<64, 128, 128, EPI_PC, W_I4>(a, s);
+  return run_dma<64, 64, 128, EPI_PC, W_I4>(a, s);
 }
 
 }  // namespace
@@ -763,12 +674,22 @@ hipError_t launch_gemm_splitk(const GemmArgs& a, int S, int32_t* part, hipStream
   return hipGetLastError();
 }
 
+bool w4_wants_il(const GemmArgs& a) {
+  const TileCost* c;
+  PpPlan pl;
+  // launch_gemm's conditions for the LDS-DMA kernels, above its M <= 64 rules
+  if (a.M <= 64 || a.K % 128 != 0 || a.N % 8 != 0 || (int64_t)a.K * 256 >= ((int64_t)1 << 32) ||
+      (((uintptr_t)a.w | (uintptr_t)a.y | (uintptr_t)a.sw) & 15) != 0)
+    return false;
+  return pick(a, EPI_PC, W_I4, kTilesI4, &c, &pl);
+}
+
 // Eligible: EPI_I32 or EPI_PC with int8 weights, EPI_PC with int4 weights;
 // K % 128 == 0, N % 8 == 0, 16-byte aligned operands (launch_gemm checks).
 hipError_t launch_gemm_dma(const GemmArgs& a, int epi, int wf, hipStream_t s) {
-  if (wf == W_I4) return pick_tile<EPI_PC, W_I4>(a, s);
-  if (epi == EPI_I32) return pick_tile_i8<EPI_I32>(a, s);
-  return pick_tile_i8<EPI_PC>(a, s);
+  if (wf == W_I4) return launch_i4(a, s);
+  if (epi == EPI_I32) return launch_i8<EPI_I32>(a, s);
+  return launch_i8<EPI_PC>(a, s);
 }
 
 }  // namespace cider

@@ -445,6 +445,8 @@ struct PpCost {
 };
 constexpr PpCost kCostI8 = {{0, 0.559, 0.597, 0.776, 1.033}, {0, 2.32, 5.25, 7.52, 9.0},
                             1.281, 0.374, 6.4};
+constexpr PpCost kCostI4 = {{0, 0.645, 0.696, 0.828, 1.014}, {0, 4.04, 5.79, 7.51, 9.0},
+                            1.243, 0.551, 5.4};
 
 double plan_cost(const PpCost& c, const PpPlan& pl, int nk, int cus) {
   const double tb = nk * c.stage[pl.mb] + c.fill[pl.mb];
@@ -464,9 +466,9 @@ double plan_cost(const PpCost& c, const PpPlan& pl, int nk, int cus) {
 
 bool pp_supported(const GemmArgs& a, int epi, int wf) {
   // 32-bit element offsets within a tile of the output; the DMA of the bias
-  // moves 16 bytes per lane
+  // moves 16 bytes per lane; 16 times the int4 weights' sums fit int32
   return a.M >= 64 && a.N >= 256 && a.N % 8 == 0 && a.N <= (1 << 22) && a.K >= 512 &&
-         a.K % 128 == 0 && epi != EPI_PG && wf == W_I8 &&
+         a.K % 128 == 0 && (wf == W_I8 ? epi != EPI_PG : epi == EPI_PC && a.K < (1 << 17)) &&
          (a.bias == nullptr || ((uintptr_t)a.bias & 15) == 0);
 }
 
@@ -474,7 +476,7 @@ bool pp_supported(const GemmArgs& a, int epi, int wf) {
 // big tile in small ones; and as many whole tile columns of big tiles as fill
 // whole rounds of the CUs, the columns right of them in small ones.
 double pp_plan(int M, int N, int K, int wf, PpPlan& best) {
-  const PpCost& c = kCostI8;
+  const PpCost& c = wf == W_I4 ? kCostI4 : kCostI8;
   const int cus = num_cus(), nk = K / 128, tn = (N + 255) / 256;
   auto ceil_div = [](int x, int y) { return (x + y - 1) / y; };
   double best_cost = 1e300;
@@ -508,7 +510,7 @@ double pp_plan(int M, int N, int K, int wf, PpPlan& best) {
 }
 
 hipError_t launch_gemm_pp(const GemmArgs& a, int epi, int wf, const PpPlan& pl, hipStream_t s) {
-  (void)wf;
+  if (wf == W_I4) return run_pp<EPI_PC, W_I4>(a, pl, s);
   if (epi == EPI_I32) return run_pp<EPI_I32, W_I8>(a, pl, s);
   return run_pp<EPI_PC, W_I8>(a, pl, s);
 }

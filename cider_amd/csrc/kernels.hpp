@@ -19,10 +19,15 @@ struct GemmArgs {
   const uint16_t* bias;   // fp16 [N] or nullptr (no add)
   void* y;                // fp16 [M, N] (PC, PG) or int32 [M, N] (I32)
   int M, N, K;
+  // x holds every 32 consecutive k as the 16 even ones, then the 16 odd ones:
+  // the ping-pong kernel's order for int4 weights (w4_wants_il), no other's
+  bool x_il = false;
 };
 
+// il: every 32 consecutive k of q in the order GemmArgs::x_il describes (K %
+// 32 == 0, vectorizable x and q).
 hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
-                           int K, hipStream_t s);
+                           int K, hipStream_t s, bool il = false);
 
 // C = epilogue(x . w^T).  wf: W_I8 / W_I4; epi: Epilogue; sw_half: PG scales
 // are fp16; gs: group size (PG only).
@@ -49,6 +54,9 @@ hipError_t launch_gemm_dma(const GemmArgs& a, int epi, int wf, hipStream_t s);
 struct PpPlan {
   int mb, ms, nbig, nsmall, m_split, n_split, s0, grid;
 };
+// Whether the per-channel int4 GEMM of a runs the ping-pong kernel, so that its
+// x has to be quantized with il (a.x need not hold anything yet).
+bool w4_wants_il(const GemmArgs& a);
 // Shapes and alignments it takes, the best plan for a shape (returns its
 // estimated time in us), and the launch.
 bool pp_supported(const GemmArgs& a, int epi, int wf);

@@ -19,12 +19,29 @@
 
 namespace cider {
 
+namespace {
+
+// Vector e (8 elements) of a quantized row.  il: every 32 consecutive elements
+// are stored as the 16 of even index, then the 16 of odd index (K % 32 == 0),
+// the order the ping-pong GEMM takes for int4 weights (gemm_pp.hip).
+__device__ __forceinline__ void store_q8(int8_t* qr, int e, i32x2 v, int il) {
+  if (!il) {
+    *reinterpret_cast<i32x2*>(qr + 8 * e) = v;
+    return;
+  }
+  int32_t* const d = reinterpret_cast<int32_t*>(qr + 32 * (e >> 2) + 4 * (e & 3));
+  d[0] = (int32_t)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x06040200u);
+  d[4] = (int32_t)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x07050301u);
+}
+
+}  // namespace
+
 // Vectorized rows: K % 8 == 0, x 16-byte and q 8-byte aligned.  NV > 0 keeps
 // NV 16-byte vectors per lane in registers; NV == 0 streams the row twice.
 template <int NV>
 __global__ __launch_bounds__(256) void quantize_vec_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
-    float* __restrict__ sa, int M, int K) {
+    float* __restrict__ sa, int M, int K, int il) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= M) return;  // uniform per wave
@@ -49,7 +66,7 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int e = lane + i * kWave;
-      if (e < nvec) *reinterpret_cast<i32x2*>(qr + 8 * e) = quant8(v[i], inv);
+      if (e < nvec) store_q8(qr, e, quant8(v[i], inv), il);
     }
   } else {
     for (int e = lane; e < nvec; e += kWave) amax = absmax8(ld16(xr + 8 * e), amax);
@@ -58,7 +75,7 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(
     const float inv = 1.0f / s;
     if (lane == 0) sa[row] = s;
     for (int e = lane; e < nvec; e += kWave)
-      *reinterpret_cast<i32x2*>(qr + 8 * e) = quant8(ld16(xr + 8 * e), inv);
+      store_q8(qr, e, quant8(ld16(xr + 8 * e), inv), il);
   }
 }
 
@@ -70,7 +87,7 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(
 template <int NV, int NT = 1024>
 __global__ __launch_bounds__(NT) void quantize_row_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
-    float* __restrict__ sa, int K) {
+    float* __restrict__ sa, int K, int il) {
   constexpr int NWV = NT / 64;
   __shared__ float red[NWV];
   const int tid = threadIdx.x;
@@ -98,7 +115,7 @@ __global__ __launch_bounds__(NT) void quantize_row_kernel(
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int e = tid + i * NT;
-    if (e < nvec) *reinterpret_cast<i32x2*>(qr + 8 * e) = quant8(v[i], inv);
+    if (e < nvec) store_q8(qr, e, quant8(v[i], inv), il);
   }
 }
 
@@ -121,11 +138,12 @@ __global__ __launch_bounds__(256) void quantize_scalar_kernel(
 }
 
 hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
-                           int K, hipStream_t s) {
+                           int K, hipStream_t s, bool il) {
   const dim3 grid((M + 3) / 4), block(256);
   const bool vec = (K % 8 == 0) && (((uintptr_t)x & 15) == 0) &&
                    (((uintptr_t)q & 7) == 0);
   if (!vec) {
+    if (il) return hipErrorInvalidValue;
     quantize_scalar_kernel<<<grid, block, 0, s>>>(x, q, sa, M, K);
     return hipGetLastError();
   }
@@ -134,13 +152,13 @@ hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
     // a row per 1024-thread workgroup (max(a, b) is exact, so the absmax does
     // not depend on how the row is split)
     if (nvec <= 1024)
-      quantize_row_kernel<1><<<M, 1024, 0, s>>>(x, q, sa, K);
+      quantize_row_kernel<1><<<M, 1024, 0, s>>>(x, q, sa, K, il);
     else if (nvec <= 2048)
-      quantize_row_kernel<2><<<M, 1024, 0, s>>>(x, q, sa, K);
+      quantize_row_kernel<2><<<M, 1024, 0, s>>>(x, q, sa, K, il);
     else if (nvec <= 4096)
-      quantize_row_kernel<4><<<M, 1024, 0, s>>>(x, q, sa, K);
+      quantize_row_kernel<4><<<M, 1024, 0, s>>>(x, q, sa, K, il);
     else
-      quantize_row_kernel<8><<<M, 1024, 0, s>>>(x, q, sa, K);
+      quantize_row_kernel<8><<<M, 1024, 0, s>>>(x, q, sa, K, il);
     return hipGetLastError();
   }
   const int per_lane = (nvec + kWave - 1) / kWave;
@@ -155,32 +173,32 @@ hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
     // to 32 16-byte vectors per lane and ran at few waves per SIMD (4096 x
     // 10240: 36.3 -> 21.7 us; 4096 x 4096: 10.8 -> 9.7 us).
     const int nv = (nvec + 255) / 256;
-    if (nv <= 2) quantize_row_kernel<2, 256><<<M, 256, 0, s>>>(x, q, sa, K);
-    else if (nv <= 3) quantize_row_kernel<3, 256><<<M, 256, 0, s>>>(x, q, sa, K);
-    else if (nv <= 4) quantize_row_kernel<4, 256><<<M, 256, 0, s>>>(x, q, sa, K);
-    else if (nv <= 5) quantize_row_kernel<5, 256><<<M, 256, 0, s>>>(x, q, sa, K);
-    else if (nv <= 6) quantize_row_kernel<6, 256><<<M, 256, 0, s>>>(x, q, sa, K);
-    else quantize_row_kernel<8, 256><<<M, 256, 0, s>>>(x, q, sa, K);
+    if (nv <= 2) quantize_row_kernel<2, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
+    else if (nv <= 3) quantize_row_kernel<3, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
+    else if (nv <= 4) quantize_row_kernel<4, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
+    else if (nv <= 5) quantize_row_kernel<5, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
+    else if (nv <= 6) quantize_row_kernel<6, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
+    else quantize_row_kernel<8, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
     return hipGetLastError();
   }
   if (per_lane <= 1)
-    quantize_vec_kernel<1><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<1><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else if (per_lane <= 2)
-    quantize_vec_kernel<2><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<2><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else if (per_lane <= 4)
-    quantize_vec_kernel<4><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<4><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else if (per_lane <= 5)
-    quantize_vec_kernel<5><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<5><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else if (per_lane <= 6)
-    quantize_vec_kernel<6><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<6><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else if (per_lane <= 8)
-    quantize_vec_kernel<8><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<8><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else if (per_lane <= 16)
-    quantize_vec_kernel<16><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<16><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else if (per_lane <= 32)
-    quantize_vec_kernel<32><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<32><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   else
-    quantize_vec_kernel<0><<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_vec_kernel<0><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
   return hipGetLastError();
 }
 

@@ -71,3 +71,21 @@ def test_perchannel_epilogue(M, N, K, bias):
     e = e.half()
     assert torch.equal(y.view(torch.int16)[~e.isnan()], e.view(torch.int16)[~e.isnan()])
     assert torch.equal(y.isnan(), e.isnan())
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES + [(65, 256, 512), (777, 4104, 4096)])
+def test_int4_weights(M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(6)
+    x = torch.randn(M, K, device=DEV, generator=g).half()
+    x[0] *= 1e-5   # a row of fp16 subnormals: the smallest scales
+    x[M - 1] = 0
+    w = torch.randint(-8, 8, (N, K), dtype=torch.int8, device=DEV, generator=g)
+    w[N - 1] = -8
+    sw = torch.rand(N, device=DEV, generator=g) * 0.1 + 1e-3
+    u = w.to(torch.uint8) & 15
+    packed = (u[:, 0::2] | (u[:, 1::2] << 4)).contiguous()
+    y = C.w4a8_linear_packed(x, packed, sw)
+    q, sa = C.quantize_per_token(x)  # pinned to the oracle elsewhere
+    e = exact_product(q, w).float() * sa[:, None]
+    e = (e * sw).half()
+    assert torch.equal(y.view(torch.int16), e.view(torch.int16))

@@ -20,6 +20,7 @@
 #include <string>
 
 #include "cider_hip.h"
+#include "cider_hip_bf16.h"
 #include "kernels.hpp"
 
 namespace {
@@ -100,9 +101,10 @@ int check_ws(const char* fn, const void* ws, size_t ws_bytes, size_t needed) {
 // it saves: N=10240 K=2560 M=2 ran 13.3 us fused against 10.8 us as quantize
 // + GEMV, M=4 24.9 against 13.3 us (W4A8 gs 128, N=12288 K=4096 M=4: 22.5
 // against 15.0 us).  Returns true and the launch status in *rc if it ran.
-bool try_fused_gemv(const char* fn, const void* x, const cider::GemmArgs& g, int wf, int epi,
+bool try_fused_gemv(const char* fn, const void* x, const cider::GemmArgs& ga, int wf, int epi,
                     int gs, hipStream_t s, int* rc) {
-  cider::GemmArgs t = g;
+  cider::GemmArgs g = ga, t = ga;
+  g.x_bf16 = ga.y_bf16;
   t.x = reinterpret_cast<const int8_t*>(x);
   if (!cider::gemv_q_supported(t, wf, true)) return false;
   if (g.M > 1 && (int64_t)((g.N + 15) / 16) * g.M * g.K > ((int64_t)1 << 20)) return false;
@@ -113,11 +115,11 @@ bool try_fused_gemv(const char* fn, const void* x, const cider::GemmArgs& g, int
 
 // Quantizes x into the workspace; returns q and sa pointers.
 int quantize_into_ws(const char* fn, const void* x, void* ws, int64_t M, int64_t K,
-                     hipStream_t s, int8_t** q, float** sa, bool il = false) {
+                     hipStream_t s, int8_t** q, float** sa, bool bf, bool il = false) {
   *q = reinterpret_cast<int8_t*>(ws);
   *sa = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + align256((size_t)M * (size_t)K));
   return hip_status(cider::launch_quantize(reinterpret_cast<const uint16_t*>(x), *q, *sa,
-                                           (int)M, (int)K, s, il),
+                                           (int)M, (int)K, s, il, bf),
                     fn);
 }
 
@@ -237,7 +239,7 @@ int cider_perchannel_gemm(const int8_t* q, const float* sa, const int8_t* w_nk, 
                     fn);
 }
 
-int cider_perchannel_linear(const void* x_f16, const int8_t* w_nk, const float* sw,
+static int linear_pc(bool bf, const void* x_f16, const int8_t* w_nk, const float* sw,
                             const void* bias_f16, void* y_f16, void* ws, size_t ws_bytes,
                             int64_t M, int64_t N, int64_t K, void* stream) {
   static const char* fn = "cider_perchannel_linear";
@@ -249,18 +251,23 @@ int cider_perchannel_linear(const void* x_f16, const int8_t* w_nk, const float* 
   CIDER_TRY(need(fn, y_f16, "y", true));
   const hipStream_t s = (hipStream_t)stream;
   const uint16_t* bias = reinterpret_cast<const uint16_t*>(bias_f16);
+  if (M == 1 && bf && !cider::mv_stream_supported(x_f16, w_nk, sw, (int)K, 0))
+    return fail(CIDER_E_UNSUPPORTED, "%s: no bf16 MV for K=%lld", fn, (long long)K);
   if (M == 1)
     return hip_status(cider::launch_mv(reinterpret_cast<const uint16_t*>(x_f16), w_nk, sw, bias,
-                                       reinterpret_cast<uint16_t*>(y_f16), (int)N, (int)K, 0, s),
+                                       reinterpret_cast<uint16_t*>(y_f16), (int)N, (int)K, 0, s,
+                                       bf),
                       fn);
   CIDER_TRY(check_ws(fn, ws, ws_bytes, quant_ws_bytes(M, K)));
   int rc;
-  const cider::GemmArgs gf{nullptr, w_nk, nullptr, sw, bias, y_f16, (int)M, (int)N, (int)K};
+  cider::GemmArgs gf{nullptr, w_nk, nullptr, sw, bias, y_f16, (int)M, (int)N, (int)K};
+  gf.y_bf16 = bf;
   if (try_fused_gemv(fn, x_f16, gf, cider::W_I8, cider::EPI_PC, 0, s, &rc)) return rc;
   int8_t* q;
   float* sa;
-  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa));
+  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, bf));
   cider::GemmArgs g{q, w_nk, sa, sw, bias, y_f16, (int)M, (int)N, (int)K};
+  g.y_bf16 = bf;
   // Split-K where the shape takes it and the workspace holds the partial sums
   // (a workspace sized for the quantized activations alone runs one pass)
   const int S = cider::splitk_ways((int)M, (int)N, (int)K);
@@ -271,6 +278,12 @@ int cider_perchannel_linear(const void* x_f16, const int8_t* w_nk, const float* 
     return hip_status(cider::launch_gemm_splitk(g, S, part, s), fn);
   }
   return hip_status(cider::launch_gemm(g, cider::W_I8, cider::EPI_PC, false, 0, s), fn);
+}
+
+int cider_perchannel_linear(const void* x_f16, const int8_t* w_nk, const float* sw,
+                            const void* bias_f16, void* y_f16, void* ws, size_t ws_bytes,
+                            int64_t M, int64_t N, int64_t K, void* stream) {
+  return linear_pc(false, x_f16, w_nk, sw, bias_f16, y_f16, ws, ws_bytes, M, N, K, stream);
 }
 
 int cider_perchannel_linear_noalloc(const void* x_f16, const int8_t* w_nk, const float* sw,
@@ -309,7 +322,7 @@ float* pg_splitk_part(const cider::GemmArgs& g, void* ws, size_t ws_bytes, int g
 
 }  // namespace
 
-int cider_pergroup_linear(const void* x_f16, const int8_t* w_nk, const float* sw_gn,
+static int linear_pg(bool bf, const void* x_f16, const int8_t* w_nk, const float* sw_gn,
                           const void* bias_f16, void* y_f16, void* ws, size_t ws_bytes,
                           int64_t M, int64_t N, int64_t K, int group_size, void* stream) {
   static const char* fn = "cider_pergroup_linear";
@@ -327,19 +340,23 @@ int cider_pergroup_linear(const void* x_f16, const int8_t* w_nk, const float* sw
   CIDER_TRY(need(fn, y_f16, "y", true));
   const hipStream_t s = (hipStream_t)stream;
   const uint16_t* bias = reinterpret_cast<const uint16_t*>(bias_f16);
+  if (M == 1 && bf && !cider::mv_stream_supported(x_f16, w_nk, sw_gn, (int)K, group_size))
+    return fail(CIDER_E_UNSUPPORTED, "%s: no bf16 MV for K=%lld", fn, (long long)K);
   if (M == 1)
     return hip_status(cider::launch_mv(reinterpret_cast<const uint16_t*>(x_f16), w_nk, sw_gn,
                                        bias, reinterpret_cast<uint16_t*>(y_f16), (int)N, (int)K,
-                                       group_size, s),
+                                       group_size, s, bf),
                       fn);
   CIDER_TRY(check_ws(fn, ws, ws_bytes, quant_ws_bytes(M, K)));
   int rc;
-  const cider::GemmArgs gf{nullptr, w_nk, nullptr, sw_gn, bias, y_f16, (int)M, (int)N, (int)K};
+  cider::GemmArgs gf{nullptr, w_nk, nullptr, sw_gn, bias, y_f16, (int)M, (int)N, (int)K};
+  gf.y_bf16 = bf;
   if (try_fused_gemv(fn, x_f16, gf, cider::W_I8, cider::EPI_PG, group_size, s, &rc)) return rc;
   int8_t* q;
   float* sa;
-  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa));
+  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, bf));
   cider::GemmArgs g{q, w_nk, sa, sw_gn, bias, y_f16, (int)M, (int)N, (int)K};
+  g.y_bf16 = bf;
   float* part = pg_splitk_part(g, ws, ws_bytes, group_size);
   if (part)
     return hip_status(cider::launch_gemm_pg_splitk(g, group_size, false, cider::W_I8,
@@ -348,6 +365,13 @@ int cider_pergroup_linear(const void* x_f16, const int8_t* w_nk, const float* sw
                                                    part, s),
                       fn);
   return hip_status(cider::launch_gemm(g, cider::W_I8, cider::EPI_PG, false, group_size, s), fn);
+}
+
+int cider_pergroup_linear(const void* x_f16, const int8_t* w_nk, const float* sw_gn,
+                          const void* bias_f16, void* y_f16, void* ws, size_t ws_bytes,
+                          int64_t M, int64_t N, int64_t K, int group_size, void* stream) {
+  return linear_pg(false, x_f16, w_nk, sw_gn, bias_f16, y_f16, ws, ws_bytes, M, N, K, group_size,
+                   stream);
 }
 
 int cider_w4_repack_ref(const uint8_t* src_kn, uint8_t* dst_nk, int64_t N, int64_t K,
@@ -364,7 +388,7 @@ int cider_w4_repack_ref(const uint8_t* src_kn, uint8_t* dst_nk, int64_t N, int64
                     fn);
 }
 
-int cider_w4a8_linear(const void* x_f16, const uint8_t* w4_nk, const float* sw, void* y_f16,
+static int linear_w4(bool bf, const void* x_f16, const uint8_t* w4_nk, const float* sw, void* y_f16,
                       void* ws, size_t ws_bytes, int64_t M, int64_t N, int64_t K,
                       void* stream) {
   static const char* fn = "cider_w4a8_linear";
@@ -379,14 +403,22 @@ int cider_w4a8_linear(const void* x_f16, const uint8_t* w4_nk, const float* sw, 
   const hipStream_t s = (hipStream_t)stream;
   CIDER_TRY(check_ws(fn, ws, ws_bytes, quant_ws_bytes(M, K)));
   int rc;
-  const cider::GemmArgs gf{nullptr, w4_nk, nullptr, sw, nullptr, y_f16, (int)M, (int)N, (int)K};
+  cider::GemmArgs gf{nullptr, w4_nk, nullptr, sw, nullptr, y_f16, (int)M, (int)N, (int)K};
+  gf.y_bf16 = bf;
   if (try_fused_gemv(fn, x_f16, gf, cider::W_I4, cider::EPI_PC, 0, s, &rc)) return rc;
   int8_t* q;
   float* sa;
   const bool il = aligned16(x_f16) && cider::w4_wants_il(gf);
-  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, il));
+  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, bf, il));
   cider::GemmArgs g{q, w4_nk, sa, sw, nullptr, y_f16, (int)M, (int)N, (int)K, il};
+  g.y_bf16 = bf;
   return hip_status(cider::launch_gemm(g, cider::W_I4, cider::EPI_PC, false, 0, s), fn);
+}
+
+int cider_w4a8_linear(const void* x_f16, const uint8_t* w4_nk, const float* sw, void* y_f16,
+                      void* ws, size_t ws_bytes, int64_t M, int64_t N, int64_t K,
+                      void* stream) {
+  return linear_w4(false, x_f16, w4_nk, sw, y_f16, ws, ws_bytes, M, N, K, stream);
 }
 
 int cider_w4a8_linear_ref(const void* x_f16, const uint8_t* packed_kn, const float* sw,
@@ -412,7 +444,7 @@ int cider_w4a8_linear_ref(const void* x_f16, const uint8_t* packed_kn, const flo
   return cider_w4a8_linear(x_f16, w4_nk, sw, y_f16, ws, qbytes, M, N, K, stream);
 }
 
-int cider_w4a8_pergroup_linear(const void* x_f16, const uint8_t* w4_nk,
+static int linear_w4pg(bool bf, const void* x_f16, const uint8_t* w4_nk,
                                const void* scale_gn_f16, const void* bias_f16, void* y_f16,
                                void* ws, size_t ws_bytes, int64_t M, int64_t N, int64_t K,
                                int group_size, void* stream) {
@@ -431,15 +463,17 @@ int cider_w4a8_pergroup_linear(const void* x_f16, const uint8_t* w4_nk,
   const hipStream_t s = (hipStream_t)stream;
   CIDER_TRY(check_ws(fn, ws, ws_bytes, quant_ws_bytes(M, K)));
   int rc;
-  const cider::GemmArgs gf{nullptr, w4_nk, nullptr, scale_gn_f16,
+  cider::GemmArgs gf{nullptr, w4_nk, nullptr, scale_gn_f16,
                            reinterpret_cast<const uint16_t*>(bias_f16), y_f16, (int)M, (int)N,
                            (int)K};
+  gf.y_bf16 = bf;
   if (try_fused_gemv(fn, x_f16, gf, cider::W_I4, cider::EPI_PG, group_size, s, &rc)) return rc;
   int8_t* q;
   float* sa;
-  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa));
+  CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, bf));
   cider::GemmArgs g{q, w4_nk, sa, scale_gn_f16, reinterpret_cast<const uint16_t*>(bias_f16),
                     y_f16, (int)M, (int)N, (int)K};
+  g.y_bf16 = bf;
   float* part = pg_splitk_part(g, ws, ws_bytes, group_size);
   if (part)
     return hip_status(cider::launch_gemm_pg_splitk(g, group_size, true, cider::W_I4,
@@ -448,6 +482,38 @@ int cider_w4a8_pergroup_linear(const void* x_f16, const uint8_t* w4_nk,
                                                    part, s),
                       fn);
   return hip_status(cider::launch_gemm(g, cider::W_I4, cider::EPI_PG, true, group_size, s), fn);
+}
+
+int cider_w4a8_pergroup_linear(const void* x_f16, const uint8_t* w4_nk,
+                               const void* scale_gn_f16, const void* bias_f16, void* y_f16,
+                               void* ws, size_t ws_bytes, int64_t M, int64_t N, int64_t K,
+                               int group_size, void* stream) {
+  return linear_w4pg(false, x_f16, w4_nk, scale_gn_f16, bias_f16, y_f16, ws, ws_bytes, M, N, K,
+                     group_size, stream);
+}
+
+int cider_linear_bf16(int op, const void* x_bf16, const void* w, const void* scale,
+                      const void* bias_f16, void* y_bf16, void* ws, size_t ws_bytes, int64_t M,
+                      int64_t N, int64_t K, int group_size, void* stream) {
+  const float* sw = reinterpret_cast<const float*>(scale);
+  switch (op) {
+    case CIDER_OP_PERCHANNEL:
+      return linear_pc(true, x_bf16, reinterpret_cast<const int8_t*>(w), sw, bias_f16, y_bf16, ws,
+                       ws_bytes, M, N, K, stream);
+    case CIDER_OP_PERGROUP:
+      return linear_pg(true, x_bf16, reinterpret_cast<const int8_t*>(w), sw, bias_f16, y_bf16, ws,
+                       ws_bytes, M, N, K, group_size, stream);
+    case CIDER_OP_W4A8:
+      if (bias_f16 != nullptr)
+        return fail(CIDER_E_INVALID, "cider_linear_bf16: the per-channel W4A8 linear has no bias");
+      return linear_w4(true, x_bf16, reinterpret_cast<const uint8_t*>(w), sw, y_bf16, ws,
+                       ws_bytes, M, N, K, stream);
+    case CIDER_OP_W4A8_PERGROUP:
+      return linear_w4pg(true, x_bf16, reinterpret_cast<const uint8_t*>(w), scale, bias_f16,
+                         y_bf16, ws, ws_bytes, M, N, K, group_size, stream);
+    default:
+      return fail(CIDER_E_INVALID, "cider_linear_bf16: unknown op %d", op);
+  }
 }
 
 // ---- producers of the linear's input and the decode attention -------------

@@ -45,6 +45,45 @@ __device__ __forceinline__ uint32_t f2h2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
 }
 
+// Eight bf16 (two per word) rounded to fp16, as a cast of the tensor rounds
+// them: exact in binary32, then RNE (out of range: infinity).
+__device__ __forceinline__ i32x4 bf16x8_to_f16(i32x4 v) {
+  i32x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t w = (uint32_t)v[j];
+    o[j] = (int32_t)f2h2(__builtin_bit_cast(float, w << 16),
+                         __builtin_bit_cast(float, w & 0xffff0000u));
+  }
+  return o;
+}
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// Output values of the linears: fp16, or with bf (wave-uniform) the fp16 value
+// rounded to bf16, as a cast of the fp16 result rounds it.
+__device__ __forceinline__ uint32_t h2_to_bf2(uint32_t h) {
+  const f32x2 f = __builtin_convertvector(__builtin_bit_cast(f16x2, h), f32x2);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+}
+__device__ __forceinline__ uint32_t f2o2(float a, float b, bool bf) {
+  const uint32_t h = f2h2(a, b);
+  return bf ? h2_to_bf2(h) : h;
+}
+__device__ __forceinline__ uint16_t f2o(float f, bool bf) {
+  const uint16_t h = f2h(f);
+  return bf ? (uint16_t)h2_to_bf2(h) : h;
+}
+
+// Eight fp16 outputs staged in LDS, as they are stored.
+__device__ __forceinline__ i32x4 out8(i32x4 v, bool bf) {
+  if (bf) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (int32_t)h2_to_bf2((uint32_t)v[j]);
+  }
+  return v;
+}
+
 // 16x16x64 int8 MFMA: C[i][j] += sum_k A[i][k] * B[k][j].
 // Operand layout (64 lanes, 16 bytes each): lane l holds row i = l % 16 of A
 // (column j = l % 16 of B) and one 16-byte slice of K selected by l / 16; the

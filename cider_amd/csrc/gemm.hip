@@ -326,7 +326,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const GemmArgs p) {
           }
           if (p.bias) v[r] = v[r] + bv[r];
         }
-        const uint32_t o01 = f2h2(v[0], v[1]), o23 = f2h2(v[2], v[3]);
+        const uint32_t o01 = f2o2(v[0], v[1], p.y_bf16), o23 = f2o2(v[2], v[3], p.y_bf16);
         uint16_t* yp = reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + n;
         if (vec_n) {
           *reinterpret_cast<i32x2*>(yp) = i32x2{(int)o01, (int)o23};

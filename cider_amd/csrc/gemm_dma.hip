@@ -395,8 +395,8 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         swv[a][g] = *reinterpret_cast<const f32x4*>(ssw + wn * WN + a * 32 + 8 * g + 4 * h);
-    auto convert = [&](auto biasc) {
-      constexpr bool BIAS = decltype(biasc)::value != 0;
+    auto convert = [&](auto biasc, auto bfc) {
+      constexpr bool BIAS = decltype(biasc)::value != 0, BF = decltype(bfc)::value != 0;
       i32x2 bbv[TN][4];
       if constexpr (BIAS) {
 #pragma unroll
@@ -435,15 +435,21 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
               o[r] = v;
             }
             *reinterpret_cast<i32x2*>(smem + ml * C::OUT_LD + nl * 2) =
-                i32x2{(int)f2h2(o[0], o[1]), (int)f2h2(o[2], o[3])};
+                i32x2{(int)f2o2(o[0], o[1], BF), (int)f2o2(o[2], o[3], BF)};
           }
         }
       }
     };
-    if (p.bias)
-      convert(icst<1>{});
-    else
-      convert(icst<0>{});
+    if (p.y_bf16) {
+      if (p.bias)
+        convert(icst<1>{}, icst<1>{});
+      else
+        convert(icst<0>{}, icst<1>{});
+    } else if (p.bias) {
+      convert(icst<1>{}, icst<0>{});
+    } else {
+      convert(icst<0>{}, icst<0>{});
+    }
     __syncthreads();
     // whole rows: BN / 8 lanes x 16 bytes per row, 512 / BN rows per store
     constexpr int LPR = BN / 8, RPS = 64 / LPR;
@@ -622,7 +628,7 @@ __global__ __launch_bounds__(256) void splitk_dequant_kernel(const GemmArgs p,
     o[r] = v;
   }
   *reinterpret_cast<i32x2*>(reinterpret_cast<uint16_t*>(p.y) + e) =
-      i32x2{(int)f2h2(o[0], o[1]), (int)f2h2(o[2], o[3])};
+      i32x2{(int)f2o2(o[0], o[1], p.y_bf16), (int)f2o2(o[2], o[3], p.y_bf16)};
 }
 
 // K slices for a per-channel int8 shape (1 = no split): only where the

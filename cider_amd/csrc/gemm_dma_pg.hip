@@ -219,7 +219,7 @@ __device__ __forceinline__ void pg_exact_tile(const GemmArgs& p, int m0, int n0,
     } else {
       float v = acc * p.sa[m];
       if (p.bias) v = v + h2f(p.bias[n]);
-      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2h(v);
+      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
     }
   }
 }
@@ -793,7 +793,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_dma_pg_kernel(const 
     const int m = m0 + rr;
     if (m < M && n < N)
       *reinterpret_cast<i32x4*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + n) =
-          *reinterpret_cast<const i32x4*>(smem + rr * PG_OUT_LD + cl * 2);
+          out8(*reinterpret_cast<const i32x4*>(smem + rr * PG_OUT_LD + cl * 2), p.y_bf16);
   }
 }
 
@@ -1191,7 +1191,7 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_pg16_kernel(const GemmArgs pi
       const int m = m0 + rr;
       if (m < M && n < N)
         *reinterpret_cast<i32x4*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + n) =
-            *reinterpret_cast<const i32x4*>(smem + rr * OUT_LD + cl * 2);
+            out8(*reinterpret_cast<const i32x4*>(smem + rr * OUT_LD + cl * 2), p.y_bf16);
     }
   };
   // split-K slice: the chain's fp32 sums, 4 consecutive columns per store
@@ -1268,7 +1268,7 @@ __global__ __launch_bounds__(256) void pg_splitk_sum_kernel(const GemmArgs p,
     o[r] = v;
   }
   *reinterpret_cast<i32x2*>(reinterpret_cast<uint16_t*>(p.y) + e) =
-      i32x2{(int)f2h2(o[0], o[1]), (int)f2h2(o[2], o[3])};
+      i32x2{(int)f2o2(o[0], o[1], p.y_bf16), (int)f2o2(o[2], o[3], p.y_bf16)};
 }
 
 // Tile of the split-K slices, with the workgroups one CU holds and the

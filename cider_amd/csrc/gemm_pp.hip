@@ -328,8 +328,8 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
       for (int h = 0; h < 2; ++h) {
         const f32x4 s0 = *reinterpret_cast<const f32x4*>(ssw + 32 * h);
         const f32x4 s1 = *reinterpret_cast<const f32x4*>(ssw + 32 * h + 4);
-        auto convert = [&](auto biasc) {
-          constexpr bool BIAS = decltype(biasc)::value;
+        auto convert = [&](auto biasc, auto bfc) {
+          constexpr bool BIAS = decltype(biasc)::value, BF = decltype(bfc)::value;
           float bv[8];
           if constexpr (BIAS) {
             const i32x4 bb = *reinterpret_cast<const i32x4*>(sbi + 32 * h);
@@ -347,7 +347,7 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
             float o[8];
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
-              // opaque: the conversions stay inside this bias path
+              // opaque: the conversions stay inside this path
               int iv = acc[2 * h + r / 4][q][r % 4];
               asm volatile("" : "+v"(iv));
               float v = (float)iv * sa;
@@ -356,14 +356,20 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
               o[r] = v;
             }
             *reinterpret_cast<i32x4*>(yb + (uint32_t)((er + ro) * N + ec + 32 * h)) =
-                i32x4{(int)f2h2(o[0], o[1]), (int)f2h2(o[2], o[3]), (int)f2h2(o[4], o[5]),
-                      (int)f2h2(o[6], o[7])};
+                i32x4{(int)f2o2(o[0], o[1], BF), (int)f2o2(o[2], o[3], BF),
+                      (int)f2o2(o[4], o[5], BF), (int)f2o2(o[6], o[7], BF)};
           }
         };
-        if (p.bias)
-          convert(std::true_type{});
-        else
-          convert(std::false_type{});
+        if (p.y_bf16) {
+          if (p.bias)
+            convert(std::true_type{}, std::true_type{});
+          else
+            convert(std::false_type{}, std::true_type{});
+        } else if (p.bias) {
+          convert(std::true_type{}, std::false_type{});
+        } else {
+          convert(std::false_type{}, std::false_type{});
+        }
       }
     } else {
       int32_t* const yb = reinterpret_cast<int32_t*>(p.y) + (int64_t)m0 * N + n0;

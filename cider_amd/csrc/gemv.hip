@@ -528,9 +528,13 @@ hipError_t launch_mv_producer(int xm, const uint16_t* x, const uint16_t* add, ui
 
 hipError_t launch_mv(const uint16_t* x, const int8_t* w, const float* sw,
                      const uint16_t* bias, uint16_t* y, int N, int K, int gs,
-                     hipStream_t s) {
-  if (mv_stream_supported(x, w, sw, K, gs))
-    return launch_mv_stream(XM_PLAIN, x, w, sw, bias, y, N, K, gs, MvProducer{}, s);
+                     hipStream_t s, bool bf) {
+  if (mv_stream_supported(x, w, sw, K, gs)) {
+    MvProducer pp;
+    pp.bf16 = bf;
+    return launch_mv_stream(XM_PLAIN, x, w, sw, bias, y, N, K, gs, pp, s);
+  }
+  if (bf) return hipErrorNotSupported;
   return launch_mv_lanes(x, w, sw, bias, y, N, K, gs, s);
 }
 

@@ -86,6 +86,7 @@ __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
       for (int i = 0; i < QV; ++i) {
         const int e = tid + 1024 * i;
         xv[m][i] = (m < M && e < nv8) ? ld16(x16 + (size_t)m * K + 8 * e) : i32x4{0, 0, 0, 0};
+        if (p.x_bf16) xv[m][i] = bf16x8_to_f16(xv[m][i]);
         am[m] = absmax8(xv[m][i], am[m]);
       }
       am[m] = wave_max(am[m]);
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
       for (; g < G; ++g) chain = chain + tm[g];
       float v = chain * (FQ ? srow[m] : p.sa[m]);
       if (p.bias) v = v + h2f(p.bias[n]);
-      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2h(v);
+      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
     }
   } else {
 #pragma unroll
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
           float v = (float)acc[m] * (FQ ? srow[m] : p.sa[m]);
           v = v * reinterpret_cast<const float*>(p.sw)[n];
           if (p.bias) v = v + h2f(p.bias[n]);
-          reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2h(v);
+          reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
         }
       }
     }
@@ -296,7 +297,8 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
                                                           const uint8_t* __restrict__ w,
                                                           const void* __restrict__ sw_,
                                                           const uint16_t* __restrict__ bias,
-                                                          uint16_t* __restrict__ y, int N) {
+                                                          uint16_t* __restrict__ y, int N,
+                                                          bool bf) {
   constexpr bool PG = GS > 0;
   constexpr int NT = 64 * NW;
   constexpr int RB = 1024 * C / R, K = 2 * RB;  // bytes per weight row, k per row
@@ -337,7 +339,11 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
   }
   __builtin_amdgcn_sched_barrier(0);
 
-  // per-token quantization of x (one row)
+  // per-token quantization of x (one row; bf16 is rounded to fp16 first)
+  if (bf) {
+#pragma unroll
+    for (int q = 0; q < XV; ++q) xv[q] = bf16x8_to_f16(xv[q]);
+  }
   float am = 0.0f;
 #pragma unroll
   for (int q = 0; q < XV; ++q)
@@ -410,7 +416,7 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
       float v = (float)av * sa;
       v = v * reinterpret_cast<const float*>(sw_)[n0 + lane];
       if (bias) v = v + h2f(bias[n0 + lane]);
-      y[n0 + lane] = f2h(v);
+      y[n0 + lane] = f2o(v, bf);
     }
     return;
   }
@@ -425,7 +431,7 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
     for (int g = 0; g < G; ++g) chain = chain + tm[g];
     float v = chain * sa;
     if (bias) v = v + h2f(bias[n0 + lane]);
-    y[n0 + lane] = f2h(v);
+    y[n0 + lane] = f2o(v, bf);
   }
 }
 
@@ -443,7 +449,7 @@ hipError_t run_gemv1_w4(const uint16_t* x, const GemmArgs& a, hipStream_t s) {
 #define CIDER_G1(RR, CC, NWW)                                                                 \
   case 1024 * (CC) / (RR) * 2:                                                                \
     gemv1_w4_kernel<RR, CC, GS, NWW><<<(a.N + (NWW) * (RR) - 1) / ((NWW) * (RR)), 64 * (NWW), \
-                                       0, s>>>(x, w, a.sw, a.bias, y, a.N);                   \
+                                       0, s>>>(x, w, a.sw, a.bias, y, a.N, a.x_bf16);         \
     return hipGetLastError();
   switch (a.K) {
     CIDER_G1(4, 4, 4)   // 2048

@@ -22,12 +22,16 @@ struct GemmArgs {
   // x holds every 32 consecutive k as the 16 even ones, then the 16 odd ones:
   // the ping-pong kernel's order for int4 weights (w4_wants_il), no other's
   bool x_il = false;
+  // y (PC, PG) is bf16: the fp16 result rounded once more.  x of the GEMVs that
+  // quantize it themselves is bf16, rounded to fp16 first.
+  bool y_bf16 = false, x_bf16 = false;
 };
 
 // il: every 32 consecutive k of q in the order GemmArgs::x_il describes (K %
 // 32 == 0, vectorizable x and q).
+// bf: x is bf16, rounded to fp16 first.
 hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
-                           int K, hipStream_t s, bool il = false);
+                           int K, hipStream_t s, bool il = false, bool bf = false);
 
 // C = epilogue(x . w^T).  wf: W_I8 / W_I4; epi: Epilogue; sw_half: PG scales
 // are fp16; gs: group size (PG only).
@@ -96,6 +100,7 @@ struct MvProducer {
   uint16_t* hsum = nullptr;       // XM_ADDNORM: h = x + add
   const uint16_t* nw = nullptr;   // XM_NORM / XM_ADDNORM
   float eps = 0.0f;
+  bool bf16 = false;              // XM_PLAIN: x and y are bf16 (x rounded to fp16)
 };
 // Streaming MV (mv_stream.hip): K in its table (1024 <= K <= 16384,
 // K % 256 == 0), 16-byte aligned x and w, gs % 16 == 0.
@@ -113,9 +118,10 @@ bool mv_producer_supported(const void* x, const void* w, int K);
 hipError_t launch_mv_producer(int xm, const uint16_t* x, const uint16_t* add, uint16_t* hsum,
                               const uint16_t* nw, float eps, const int8_t* w, const float* sw,
                               const uint16_t* bias, uint16_t* y, int N, int K, hipStream_t s);
+// bf: x and y are bf16 (only shapes mv_stream_supported takes).
 hipError_t launch_mv(const uint16_t* x, const int8_t* w, const float* sw,
                      const uint16_t* bias, uint16_t* y, int N, int K, int gs,
-                     hipStream_t s);
+                     hipStream_t s, bool bf = false);
 
 // Producer kernels (fused.hip): RMSNorm (+ residual add) and SwiGLU, each
 // optionally ending in the per-token quantization; per-head q/k RMSNorm +

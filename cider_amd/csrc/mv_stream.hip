@@ -155,6 +155,8 @@ __global__ __launch_bounds__(kWpg * 64) void mv_stream_kernel(
   for (int q = 0; q < XR; ++q) {
     if constexpr (XM == XM_SWIGLU) xr[q] = swiglu8(xr[q], xu[q]);
     if constexpr (XM == XM_ADDNORM) xr[q] = add8(xr[q], xu[q]);
+    if constexpr (XM == XM_PLAIN)
+      if (pp.bf16) xr[q] = bf16x8_to_f16(xr[q]);
   }
   if constexpr (kNorm) {
     float ss = 0.0f;
@@ -225,7 +227,7 @@ __global__ __launch_bounds__(kWpg * 64) void mv_stream_kernel(
     for (int r = 1; r < R; ++r) a = lane == r ? acc[r] : a;
     float v = PG ? a : s_row * a;
     if (bias) v = v + b_row;
-    y[n0 + lane] = f2h(v);
+    y[n0 + lane] = f2o(v, XM == XM_PLAIN && pp.bf16);
   }
 }
 
@@ -308,6 +310,12 @@ __global__ __launch_bounds__(KS * 64) void mv_ksplit_kernel(const uint16_t* __re
 #pragma unroll
     for (int q = 0; q < XR; ++q) xr[q] = swiglu8(xr[q], xu[q]);
   }
+  if constexpr (XM == XM_PLAIN) {
+    if (pp.bf16) {
+#pragma unroll
+      for (int q = 0; q < XR; ++q) xr[q] = bf16x8_to_f16(xr[q]);
+    }
+  }
   if constexpr (kNorm) {
     // the statistic as the producer kernels take it: thread t's chunks t,
     // t + 256, ... (threads 0..255), then the sum over waves 0..3
@@ -378,7 +386,7 @@ __global__ __launch_bounds__(KS * 64) void mv_ksplit_kernel(const uint16_t* __re
     for (int v = 1; v < KS; ++v) a = a + part[v][lane];
     float o = s_row * a;
     if (bias) o = o + b_row;
-    y[n0 + lane] = f2h(o);
+    y[n0 + lane] = f2o(o, XM == XM_PLAIN && pp.bf16);
   }
 }
 

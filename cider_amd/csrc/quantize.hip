@@ -36,12 +36,15 @@ __device__ __forceinline__ void store_q8(int8_t* qr, int e, i32x2 v, int il) {
 
 }  // namespace
 
+// bf: x is bf16, rounded to fp16 first (three VALU operations per two
+// elements, instead of a cast kernel that reads and writes x).
+//
 // Vectorized rows: K % 8 == 0, x 16-byte and q 8-byte aligned.  NV > 0 keeps
 // NV 16-byte vectors per lane in registers; NV == 0 streams the row twice.
 template <int NV>
 __global__ __launch_bounds__(256) void quantize_vec_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
-    float* __restrict__ sa, int M, int K, int il) {
+    float* __restrict__ sa, int M, int K, int il, int bf) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= M) return;  // uniform per wave
@@ -57,6 +60,10 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(
     i32x4 v[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) v[i] = ld16(xr + 8 * min(lane + i * kWave, nvec - 1));
+    if (bf) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) v[i] = bf16x8_to_f16(v[i]);
+    }
 #pragma unroll
     for (int i = 0; i < NV; ++i) amax = absmax8(v[i], amax);
     amax = wave_max(amax);
@@ -69,13 +76,17 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(
       if (e < nvec) store_q8(qr, e, quant8(v[i], inv), il);
     }
   } else {
-    for (int e = lane; e < nvec; e += kWave) amax = absmax8(ld16(xr + 8 * e), amax);
+    auto ldv = [&](int e) {
+      const i32x4 v = ld16(xr + 8 * e);
+      return bf ? bf16x8_to_f16(v) : v;
+    };
+    for (int e = lane; e < nvec; e += kWave) amax = absmax8(ldv(e), amax);
     amax = wave_max(amax);
     const float s = row_scale(amax);
     const float inv = 1.0f / s;
     if (lane == 0) sa[row] = s;
     for (int e = lane; e < nvec; e += kWave)
-      store_q8(qr, e, quant8(ld16(xr + 8 * e), inv), il);
+      store_q8(qr, e, quant8(ldv(e), inv), il);
   }
 }
 
@@ -87,7 +98,7 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(
 template <int NV, int NT = 1024>
 __global__ __launch_bounds__(NT) void quantize_row_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
-    float* __restrict__ sa, int K, int il) {
+    float* __restrict__ sa, int K, int il, int bf) {
   constexpr int NWV = NT / 64;
   __shared__ float red[NWV];
   const int tid = threadIdx.x;
@@ -101,8 +112,13 @@ __global__ __launch_bounds__(NT) void quantize_row_kernel(
   for (int i = 0; i < NV; ++i) {
     const int e = tid + i * NT;
     v[i] = e < nvec ? ld16(xr + 8 * e) : i32x4{0, 0, 0, 0};
-    amax = absmax8(v[i], amax);
   }
+  if (bf) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = bf16x8_to_f16(v[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) amax = absmax8(v[i], amax);
   amax = wave_max(amax);
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
@@ -122,29 +138,33 @@ __global__ __launch_bounds__(NT) void quantize_row_kernel(
 // Any K and alignment: element-wise, two passes.
 __global__ __launch_bounds__(256) void quantize_scalar_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
-    float* __restrict__ sa, int M, int K) {
+    float* __restrict__ sa, int M, int K, int bf) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= M) return;
   const uint16_t* xr = x + row * K;
   int8_t* qr = q + row * K;
+  auto ldx = [&](int k) {
+    if (!bf) return h2f(xr[k]);
+    return h2f(f2h(__builtin_bit_cast(float, (uint32_t)xr[k] << 16)));
+  };
   float amax = 0.0f;
-  for (int k = lane; k < K; k += kWave) amax = fmaxf(amax, fabsf(h2f(xr[k])));
+  for (int k = lane; k < K; k += kWave) amax = fmaxf(amax, fabsf(ldx(k)));
   amax = wave_max(amax);
   const float s = row_scale(amax);
   const float inv = 1.0f / s;
   if (lane == 0) sa[row] = s;
-  for (int k = lane; k < K; k += kWave) qr[k] = quant1(h2f(xr[k]), inv);
+  for (int k = lane; k < K; k += kWave) qr[k] = quant1(ldx(k), inv);
 }
 
 hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
-                           int K, hipStream_t s, bool il) {
+                           int K, hipStream_t s, bool il, bool bf) {
   const dim3 grid((M + 3) / 4), block(256);
   const bool vec = (K % 8 == 0) && (((uintptr_t)x & 15) == 0) &&
                    (((uintptr_t)q & 7) == 0);
   if (!vec) {
     if (il) return hipErrorInvalidValue;
-    quantize_scalar_kernel<<<grid, block, 0, s>>>(x, q, sa, M, K);
+    quantize_scalar_kernel<<<grid, block, 0, s>>>(x, q, sa, M, K, bf);
     return hipGetLastError();
   }
   const int nvec = K >> 3;
@@ -152,13 +172,13 @@ hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
     // a row per 1024-thread workgroup (max(a, b) is exact, so the absmax does
     // not depend on how the row is split)
     if (nvec <= 1024)
-      quantize_row_kernel<1><<<M, 1024, 0, s>>>(x, q, sa, K, il);
+      quantize_row_kernel<1><<<M, 1024, 0, s>>>(x, q, sa, K, il, bf);
     else if (nvec <= 2048)
-      quantize_row_kernel<2><<<M, 1024, 0, s>>>(x, q, sa, K, il);
+      quantize_row_kernel<2><<<M, 1024, 0, s>>>(x, q, sa, K, il, bf);
     else if (nvec <= 4096)
-      quantize_row_kernel<4><<<M, 1024, 0, s>>>(x, q, sa, K, il);
+      quantize_row_kernel<4><<<M, 1024, 0, s>>>(x, q, sa, K, il, bf);
     else
-      quantize_row_kernel<8><<<M, 1024, 0, s>>>(x, q, sa, K, il);
+      quantize_row_kernel<8><<<M, 1024, 0, s>>>(x, q, sa, K, il, bf);
     return hipGetLastError();
   }
   const int per_lane = (nvec + kWave - 1) / kWave;
@@ -173,32 +193,32 @@ hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
     // to 32 16-byte vectors per lane and ran at few waves per SIMD (4096 x
     // 10240: 36.3 -> 21.7 us; 4096 x 4096: 10.8 -> 9.7 us).
     const int nv = (nvec + 255) / 256;
-    if (nv <= 2) quantize_row_kernel<2, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
-    else if (nv <= 3) quantize_row_kernel<3, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
-    else if (nv <= 4) quantize_row_kernel<4, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
-    else if (nv <= 5) quantize_row_kernel<5, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
-    else if (nv <= 6) quantize_row_kernel<6, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
-    else quantize_row_kernel<8, 256><<<M, 256, 0, s>>>(x, q, sa, K, il);
+    if (nv <= 2) quantize_row_kernel<2, 256><<<M, 256, 0, s>>>(x, q, sa, K, il, bf);
+    else if (nv <= 3) quantize_row_kernel<3, 256><<<M, 256, 0, s>>>(x, q, sa, K, il, bf);
+    else if (nv <= 4) quantize_row_kernel<4, 256><<<M, 256, 0, s>>>(x, q, sa, K, il, bf);
+    else if (nv <= 5) quantize_row_kernel<5, 256><<<M, 256, 0, s>>>(x, q, sa, K, il, bf);
+    else if (nv <= 6) quantize_row_kernel<6, 256><<<M, 256, 0, s>>>(x, q, sa, K, il, bf);
+    else quantize_row_kernel<8, 256><<<M, 256, 0, s>>>(x, q, sa, K, il, bf);
     return hipGetLastError();
   }
   if (per_lane <= 1)
-    quantize_vec_kernel<1><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<1><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else if (per_lane <= 2)
-    quantize_vec_kernel<2><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<2><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else if (per_lane <= 4)
-    quantize_vec_kernel<4><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<4><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else if (per_lane <= 5)
-    quantize_vec_kernel<5><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<5><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else if (per_lane <= 6)
-    quantize_vec_kernel<6><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<6><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else if (per_lane <= 8)
-    quantize_vec_kernel<8><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<8><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else if (per_lane <= 16)
-    quantize_vec_kernel<16><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<16><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else if (per_lane <= 32)
-    quantize_vec_kernel<32><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<32><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   else
-    quantize_vec_kernel<0><<<grid, block, 0, s>>>(x, q, sa, M, K, il);
+    quantize_vec_kernel<0><<<grid, block, 0, s>>>(x, q, sa, M, K, il, bf);
   return hipGetLastError();
 }
 

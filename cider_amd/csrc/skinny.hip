@@ -174,7 +174,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_kernel(const GemmArgs p) {
         v[r] = v[r] * swn;
         if (p.bias) v[r] = v[r] + (n < N ? h2f(p.bias[n]) : 0.0f);
       }
-      const uint32_t o01 = f2h2(v[0], v[1]), o23 = f2h2(v[2], v[3]);
+      const uint32_t o01 = f2o2(v[0], v[1], p.y_bf16), o23 = f2o2(v[2], v[3], p.y_bf16);
       uint16_t* yp = reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + ncol;
       if (VEC) {
         *reinterpret_cast<i32x2*>(yp) = i32x2{(int)o01, (int)o23};
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_pg_kernel(const GemmArgs p) {
     if (m >= M || n >= N) continue;
     float v = facc[o] * p.sa[m];
     if (p.bias) v = v + h2f(p.bias[n]);
-    reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2h(v);
+    reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
   }
 }
 

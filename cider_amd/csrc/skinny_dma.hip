@@ -259,7 +259,7 @@ __global__ __launch_bounds__((EPI == EPI_PG ? kSdKW + kSdCW : kSdKW) * 64) void 
         if (p.bias) v[r] = v[r] + h2f(e_b[r]);
       }
       *reinterpret_cast<i32x2*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + ncol) =
-          i32x2{(int)f2h2(v[0], v[1]), (int)f2h2(v[2], v[3])};
+          i32x2{(int)f2o2(v[0], v[1], p.y_bf16), (int)f2o2(v[2], v[3], p.y_bf16)};
     }
   } else {
     // ---- per-group.  Parts of a stage (int32 sums in LDS, [part][output],
@@ -352,7 +352,7 @@ __global__ __launch_bounds__((EPI == EPI_PG ? kSdKW + kSdCW : kSdKW) * 64) void 
       if (m >= M || n >= N) continue;
       float v = facc[o] * p.sa[m];
       if (p.bias) v = v + h2f(p.bias[n]);
-      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2h(v);
+      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
     }
   }
 }

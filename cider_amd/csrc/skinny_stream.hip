@@ -218,7 +218,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_stream_kernel(const GemmArgs p
             if (p.bias) v[r] = v[r] + h2f(p.bias[ncol + r]);
           }
           *reinterpret_cast<i32x2*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + ncol) =
-              i32x2{(int)f2h2(v[0], v[1]), (int)f2h2(v[2], v[3])};
+              i32x2{(int)f2o2(v[0], v[1], p.y_bf16), (int)f2o2(v[2], v[3], p.y_bf16)};
         }
       }
     }
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_stream_kernel(const GemmArgs p
       if (m >= M || n >= N) continue;
       float v = facc[o] * p.sa[m];
       if (p.bias) v = v + h2f(p.bias[n]);
-      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2h(v);
+      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
     }
   }
 }

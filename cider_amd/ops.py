@@ -218,6 +218,23 @@ def _cast_out(y: torch.Tensor, dtype) -> torch.Tensor:
     return y if dtype == torch.float16 else y.to(dtype)
 
 
+def _linear_bf16(op: int, x, w, scale, bias, M: int, N: int, K: int, gs: int, dev,
+                 stream) -> Optional[torch.Tensor]:
+    """A linear on bfloat16 x with a bfloat16 result in one library call (the
+    values of casting around the fp16 entry, without the cast kernels); None
+    where the library has no such path (some M == 1 shapes)."""
+    xb = x.contiguous()
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    ws = _workspace(op, M, N, K, gs, dev)
+    rc = _lib.load().cider_linear_bf16(op, _ptr(xb), _ptr(w), _ptr(scale), _ptr(bias), _ptr(y),
+                                       _ptr(ws), _nbytes(ws), M, N, K, gs,
+                                       _stream_ptr(dev, stream))
+    if rc == _lib.CIDER_E_UNSUPPORTED:
+        return None
+    _lib.check(rc)
+    return y
+
+
 # --------------------------------------------------------------------------
 # primitive API (reference surface)
 # --------------------------------------------------------------------------
@@ -268,11 +285,15 @@ def perchannel_linear(x: torch.Tensor, w: torch.Tensor, scale_w: torch.Tensor,
     out_dtype = x.dtype
     lib = _lib.load()
     with _on_stream(dev, stream):
-        xh = _as(x, torch.float16)
         wq = _as(w, torch.int8)
         sw = _as(scale_w.reshape(-1), torch.float32)
         b = (torch.zeros(N, dtype=torch.float16, device=dev) if bias is None
              else _as(bias.reshape(-1), torch.float16))
+        if out_dtype == torch.bfloat16:
+            y = _linear_bf16(_lib.CIDER_OP_PERCHANNEL, x, wq, sw, b, M, N, K, 0, dev, stream)
+            if y is not None:
+                return y
+        xh = _as(x, torch.float16)
         y = torch.empty((M, N), dtype=torch.float16, device=dev)
         ws = _workspace(_lib.CIDER_OP_PERCHANNEL, M, N, K, 0, dev)
         _lib.check(lib.cider_perchannel_linear(
@@ -343,11 +364,16 @@ def pergroup_linear(x: torch.Tensor, w: torch.Tensor, scale_w: torch.Tensor,
     out_dtype = x.dtype
     lib = _lib.load()
     with _on_stream(dev, stream):
-        xh = _as(x, torch.float16)
         wq = _as(w, torch.int8)
         sw = _as(scale_w, torch.float32)
         b = (torch.zeros(N, dtype=torch.float16, device=dev) if bias is None
              else _as(bias.reshape(-1), torch.float16))
+        if out_dtype == torch.bfloat16:
+            y = _linear_bf16(_lib.CIDER_OP_PERGROUP, x, wq, sw, b, M, N, K, group_size, dev,
+                             stream)
+            if y is not None:
+                return y
+        xh = _as(x, torch.float16)
         y = torch.empty((M, N), dtype=torch.float16, device=dev)
         ws = _workspace(_lib.CIDER_OP_PERGROUP, M, N, K, group_size, dev)
         _lib.check(lib.cider_pergroup_linear(
@@ -456,8 +482,12 @@ def w4a8_linear_packed(x: torch.Tensor, w4_nk: torch.Tensor, scale_w: torch.Tens
     out_dtype = x.dtype
     lib = _lib.load()
     with _on_stream(dev, stream):
-        xh = _as(x, torch.float16)
         sw = _as(scale_w.reshape(-1), torch.float32)
+        if out_dtype == torch.bfloat16:
+            y = _linear_bf16(_lib.CIDER_OP_W4A8, x, w4_nk, sw, None, M, N, K, 0, dev, stream)
+            if y is not None:
+                return y
+        xh = _as(x, torch.float16)
         y = torch.empty((M, N), dtype=torch.float16, device=dev)
         ws = _workspace(_lib.CIDER_OP_W4A8, M, N, K, 0, dev)
         _lib.check(lib.cider_w4a8_linear(_ptr(xh), _ptr(w4_nk), _ptr(sw), _ptr(y), _ptr(ws),
@@ -505,10 +535,15 @@ def w4a8_pergroup_linear(x: torch.Tensor, w4_nk: torch.Tensor, scales: torch.Ten
     out_dtype = x.dtype
     lib = _lib.load()
     with _on_stream(dev, stream):
-        xh = _as(x, torch.float16)
         w4 = _as(w4_nk, torch.uint8)
         sc = _as(scales, torch.float16)
         b = None if bias is None else _as(bias.reshape(-1), torch.float16)
+        if out_dtype == torch.bfloat16:
+            y = _linear_bf16(_lib.CIDER_OP_W4A8_PERGROUP, x, w4, sc, b, M, N, K, group_size, dev,
+                             stream)
+            if y is not None:
+                return y
+        xh = _as(x, torch.float16)
         y = torch.empty((M, N), dtype=torch.float16, device=dev)
         ws = _workspace(_lib.CIDER_OP_W4A8_PERGROUP, M, N, K, group_size, dev)
         _lib.check(lib.cider_w4a8_pergroup_linear(

@@ -6,9 +6,10 @@
 // with both caches [KV, T, D] (position-major, 256 bytes per position); n,
 // the number of valid positions, is read from device memory so a captured
 // decode step replays unchanged while the sequence grows.  All arithmetic is
-// fp32 (the reference's models call MLX's fused SDPA here, whose
-// accumulation order is not specified; parity is against an fp32 softmax
-// attention, within a tolerance).
+// fp32: fp16 products are exact and accumulate in fp32 (v_dot2_f32_f16), P.V
+// is one fused multiply-add per term (the reference's models call MLX's fused
+// SDPA here, whose accumulation order is not specified; parity is against an
+// fp32 softmax attention, within a tolerance).
 //
 // MI355X design (split-K "flash decoding"):
 //   * the cache is cut into chunks of 128 positions; workgroup (chunk c, KV
@@ -19,6 +20,11 @@
 //   * scores: a thread owns 8 consecutive positions and 8 of the 128
 //     dimensions (one 16-byte K load per position); the 16 dimension slices
 //     are summed through LDS.
+//     What bounds a chunk once its loads are in is VALU issue at one wave per
+//     SIMD, so both products take as few operations as fp32 allows: two terms
+//     per v_dot2_f32_f16 for the scores, and v_fma_mix_f32 (the fp16 operand
+//     widened in place) for P.V, instead of a widening, a multiply and an add
+//     per term.
 //   * P.V: a thread owns 8 dimensions (one 16-byte V load per position) and
 //     8 positions; the 16 position slices are summed through LDS.
 //   * the grid covers the cache capacity T; chunks at or past n exit at once
@@ -47,12 +53,13 @@ __device__ __forceinline__ float wave_sum_f(float v) {
   return v;
 }
 
-__device__ __forceinline__ void unpack8(i32x4 v, float (&f)[8]) {
+// s + the 8 products of two vectors of 8 fp16
+__device__ __forceinline__ float dot8(i32x4 a, i32x4 b, float s) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    f[2 * j] = h2f((uint16_t)((uint32_t)v[j] & 0xffffu));
-    f[2 * j + 1] = h2f((uint16_t)((uint32_t)v[j] >> 16));
-  }
+  for (int j = 0; j < 4; ++j)
+    s = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, (uint32_t)a[j]),
+                               __builtin_bit_cast(f16x2, (uint32_t)b[j]), s, false);
+  return s;
 }
 
 // A workgroup serves G query heads of one KV head (G <= 4: the LDS slices
@@ -64,7 +71,7 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, const int64_t* __restrict__ n_ptr, float scale,
     float* __restrict__ ws, int64_t T, int nchunk) {
-  __shared__ float qs[G][kD];
+  __shared__ __attribute__((aligned(16))) uint16_t qs[G][kD];
   __shared__ float part[16][G][kChunk];  // dimension / position slices
   __shared__ float ps[G][kChunk];        // scores, then probabilities
   __shared__ float ml[G][2];
@@ -91,7 +98,7 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) vv[i] = ld16(vp + (int64_t)i * kD);
   }
-  for (int e = tid; e < G * kD; e += 256) qs[e / kD][e % kD] = h2f(q[(int64_t)y * G * kD + e]);
+  for (int e = tid; e < G * kD; e += 256) qs[e / kD][e % kD] = q[(int64_t)y * G * kD + e];
   __syncthreads();
 
   // ---- scores: thread (dq, tq) sums dimensions 8dq..8dq+7 for positions
@@ -100,20 +107,10 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
     const int64_t t0 = tk0;
     float acc[G][8];
 #pragma unroll
-    for (int r = 0; r < G; ++r)
+    for (int r = 0; r < G; ++r) {
+      const i32x4 qv = *reinterpret_cast<const i32x4*>(&qs[r][8 * dq]);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[r][i] = 0.0f;
-    if (t0 < n) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float kf[8];  // dimensions 8dq .. 8dq + 7 of position t0 + i
-        unpack8(kv[i], kf);
-#pragma unroll
-        for (int r = 0; r < G; ++r) {
-#pragma unroll
-          for (int jd = 0; jd < 8; ++jd) acc[r][i] = acc[r][i] + qs[r][8 * dq + jd] * kf[jd];
-        }
-      }
+      for (int i = 0; i < 8; ++i) acc[r][i] = t0 < n ? dot8(kv[i], qv, 0.0f) : 0.0f;
     }
 #pragma unroll
     for (int r = 0; r < G; ++r)
@@ -161,13 +158,15 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         if (t0 + i >= n) break;  // invalid positions may hold anything
-        float vf[8];
-        unpack8(vv[i], vf);
 #pragma unroll
         for (int r = 0; r < G; ++r) {
           const float p = ps[r][8 * ts + i];
 #pragma unroll
-          for (int d = 0; d < 8; ++d) acc[r][d] = acc[r][d] + p * vf[d];
+          for (int d = 0; d < 8; ++d) {
+            const uint32_t w = (uint32_t)vv[i][d / 2];
+            acc[r][d] = __builtin_fmaf(p, h2f((uint16_t)(d & 1 ? w >> 16 : w & 0xffffu)),
+                                       acc[r][d]);
+          }
         }
       }
     }

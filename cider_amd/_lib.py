@@ -74,8 +74,9 @@ SIGNATURES = {
     "cider_swiglu_mv": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _P]),
 }
 
-# the symbol of include/cider_hip_bf16.h
-SIGNATURES_BF16 = {
+# the symbols of include/cider_hip_ext.h
+SIGNATURES_EXT = {
+    "cider_gate_up_mv": (_I, [_P, _P, _P, _P, _F, _P, _P, _P, _P, _I64, _I64, _P]),
     "cider_linear_bf16": (_I, [_I, _P, _P, _P, _P, _P, _P, _SZ, _I64, _I64, _I64, _I, _P]),
 }
 
@@ -100,7 +101,7 @@ def load():
             lib = ctypes.CDLL(LIB_PATH)
         except OSError as e:  # pragma: no cover - depends on the machine
             raise RuntimeError(f"cider_amd HIP extension failed to load: {e}") from e
-        for name, (res, args) in {**SIGNATURES, **SIGNATURES_BF16}.items():
+        for name, (res, args) in {**SIGNATURES, **SIGNATURES_EXT}.items():
             try:
                 fn = getattr(lib, name)
             except AttributeError as e:

@@ -20,7 +20,7 @@
 #include <string>
 
 #include "cider_hip.h"
-#include "cider_hip_bf16.h"
+#include "cider_hip_ext.h"
 #include "kernels.hpp"
 
 namespace {
@@ -611,6 +611,47 @@ int cider_rmsnorm_mv(const void* x_f16, const void* add_f16, void* sum_f16, cons
           reinterpret_cast<const uint16_t*>(norm_w_f16), eps, w, scale_w,
           reinterpret_cast<const uint16_t*>(bias_f16), reinterpret_cast<uint16_t*>(y_f16), (int)N,
           (int)K, (hipStream_t)stream),
+      fn);
+}
+
+int cider_gate_up_mv(const void* x_f16, const void* add_f16, void* sum_f16,
+                     const void* norm_w_f16, float eps, const int8_t* w, const float* scale_w,
+                     const void* bias_f16, void* y_f16, int64_t I, int64_t K, void* stream) {
+  static const char* fn = "cider_gate_up_mv";
+  CIDER_TRY(check_dims(fn, 1, I, K));
+  if (I > kMaxDim / 2) return fail(CIDER_E_INVALID, "%s: I too large", fn);
+  if (I == 0) return ok();
+  CIDER_TRY(need(fn, x_f16, "x", true));
+  CIDER_TRY(need(fn, w, "w", true));
+  CIDER_TRY(need(fn, scale_w, "scale_w", true));
+  CIDER_TRY(need(fn, y_f16, "y", true));
+  if (!cider::mv_pair_supported(x_f16, w, (int)K))
+    return fail(CIDER_E_UNSUPPORTED, "%s: K=%lld or the alignment of x / w is not taken", fn,
+                (long long)K);
+  if ((add_f16 == nullptr) != (sum_f16 == nullptr) || (add_f16 && !norm_w_f16))
+    return fail(CIDER_E_INVALID, "%s: add and sum come together, with norm_w", fn);
+  if (norm_w_f16 && !(eps >= 0.0f)) return fail(CIDER_E_INVALID, "%s: eps must be >= 0", fn);
+  if (!aligned16(add_f16) || !aligned16(sum_f16) || !aligned16(norm_w_f16) ||
+      (((uintptr_t)bias_f16 | (uintptr_t)y_f16) & 1) != 0 || ((uintptr_t)scale_w & 3) != 0)
+    return fail(CIDER_E_INVALID, "%s: add, sum and norm_w must be 16-byte aligned", fn);
+  const size_t row = (size_t)K * 2;
+  if (overlaps(sum_f16, row, x_f16, row) || overlaps(sum_f16, row, add_f16, row))
+    return fail(CIDER_E_INVALID, "%s: sum must not overlap x or add (other workgroups read them)",
+                fn);
+  if (overlaps(y_f16, (size_t)I * 2, x_f16, row) || overlaps(y_f16, (size_t)I * 2, add_f16, row) ||
+      overlaps(y_f16, (size_t)I * 2, sum_f16, row))
+    return fail(CIDER_E_INVALID, "%s: y must not overlap x, add or sum", fn);
+  cider::MvProducer pp;
+  pp.add = reinterpret_cast<const uint16_t*>(add_f16);
+  pp.hsum = reinterpret_cast<uint16_t*>(sum_f16);
+  pp.nw = reinterpret_cast<const uint16_t*>(norm_w_f16);
+  pp.eps = eps;
+  const int xm = add_f16 ? cider::XM_ADDNORM : norm_w_f16 ? cider::XM_NORM : cider::XM_PLAIN;
+  return hip_status(
+      cider::launch_mv_pair(xm, reinterpret_cast<const uint16_t*>(x_f16), w, scale_w,
+                            reinterpret_cast<const uint16_t*>(bias_f16),
+                            reinterpret_cast<uint16_t*>(y_f16), (int)I, (int)K, pp,
+                            (hipStream_t)stream),
       fn);
 }
 

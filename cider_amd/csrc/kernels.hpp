@@ -108,6 +108,12 @@ bool mv_stream_supported(const void* x, const void* w, const void* sw, int K, in
 hipError_t launch_mv_stream(int xm, const uint16_t* x, const int8_t* w, const float* sw,
                             const uint16_t* bias, uint16_t* y, int N, int K, int gs,
                             const MvProducer& pp, hipStream_t s);
+// The streaming MV on a fused gate + up projection w [2N, K] with SwiGLU of its
+// halves as the output y [N]; xm: XM_PLAIN, XM_NORM or XM_ADDNORM.
+bool mv_pair_supported(const void* x, const void* w, int K);
+hipError_t launch_mv_pair(int xm, const uint16_t* x, const int8_t* w, const float* sw,
+                          const uint16_t* bias, uint16_t* y, int N, int K, const MvProducer& pp,
+                          hipStream_t s);
 // The lane-order MV of gemv.hip alone (reproduces the reference's 32-lane
 // order); launch_mv / launch_mv_producer use it where the streaming MV does
 // not apply.

@@ -83,12 +83,20 @@ __device__ __forceinline__ float dot16(i32x4 wv, i32x4 xa, i32x4 xb, float acc) 
 // 16-byte vectors with x and staged in LDS, instead of one scalar load per
 // weight chunk and lane (a group row per lane group, many cache lines per
 // instruction).
-template <int R, int C, bool PG, int XM, bool SS = false>
+//
+// PAIR: the weights are a fused gate + up projection [2N, K] and y [N] is
+// SwiGLU of its two halves: a wave takes R / 2 gate rows from n0 and the R / 2
+// up rows N below them, so the product never leaves the registers.  One launch
+// less than the projection followed by SwiGLU, and half the stores; y is the
+// same bits (the projection's fp16 rounding and swiglu1 are both kept).
+template <int R, int C, bool PG, int XM, bool SS = false, bool PAIR = false>
 __global__ __launch_bounds__(kWpg * 64) void mv_stream_kernel(
     const uint16_t* __restrict__ x, const int8_t* __restrict__ w,
     const float* __restrict__ sw, const uint16_t* __restrict__ bias,
     uint16_t* __restrict__ y, int N, int gs, MvProducer pp) {
   constexpr int K = 1024 * C / R;
+  constexpr int RO = PAIR ? R / 2 : R;  // outputs per wave
+  static_assert(!PAIR || (R % 2 == 0 && !PG), "paired rows");
   constexpr int CPR = K / 16;  // 16-byte chunks per row
   static_assert(R * K == 1024 * C && CPR >= 64, "one wave covers whole rows");
   static_assert(!SS || PG, "staged scales are per-group");
@@ -99,7 +107,12 @@ __global__ __launch_bounds__(kWpg * 64) void mv_stream_kernel(
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = (blockIdx.x * kWpg + wave) * R;
+  const int n0 = (blockIdx.x * kWpg + wave) * RO;
+  // the weight row of the wave's row r (rows past N re-read the last one)
+  auto row_of = [&](int r) {
+    if constexpr (PAIR) return r < RO ? min(n0 + r, N - 1) : N + min(n0 + r - RO, N - 1);
+    return min(n0 + r, N - 1);
+  };
 
   // ---- x (or the producer's inputs) first: the staging then waits for these
   // loads only, and each chunk's products below wait only for that chunk
@@ -131,7 +144,7 @@ __global__ __launch_bounds__(kWpg * 64) void mv_stream_kernel(
   // per-row scale (per-channel) and bias of the row lane l < R writes; the
   // loads are unconditional (clamped row; x stands in for a missing bias), as
   // a load under a lane mask makes the compiler wait for every load before it
-  const int wrow = min(n0 + min(lane, R - 1), N - 1);
+  const int wrow = row_of(min(lane, R - 1));
   const float s_row = PG ? 0.0f : sw[wrow];
   const float b_row = h2f(bias ? bias[wrow] : x[0]);
 
@@ -142,7 +155,7 @@ __global__ __launch_bounds__(kWpg * 64) void mv_stream_kernel(
   for (int j = 0; j < C; ++j) {
     const int c = lane + 64 * j;
     const int r = c / CPR, kc = c - r * CPR;
-    const int row = min(n0 + r, N - 1);
+    const int row = row_of(r);
     wv[j] = ld16_nt(w + (int64_t)row * K + 16 * kc);  // read once: non-temporal
     if constexpr (PG && !SS) sj[j] = sw[(int64_t)((16 * kc) / gs) * N + row];
   }
@@ -221,13 +234,17 @@ __global__ __launch_bounds__(kWpg * 64) void mv_stream_kernel(
   // moves, then the four 16-lane rows)
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r] = wave_sum_dpp(acc[r]);
-  if (lane < R && n0 + lane < N) {
-    float a = acc[0];
+  float a = acc[0];
 #pragma unroll
-    for (int r = 1; r < R; ++r) a = lane == r ? acc[r] : a;
-    float v = PG ? a : s_row * a;
-    if (bias) v = v + b_row;
-    y[n0 + lane] = f2o(v, XM == XM_PLAIN && pp.bf16);
+  for (int r = 1; r < R; ++r) a = lane == r ? acc[r] : a;
+  float v = PG ? a : s_row * a;  // row `lane` (lanes past R hold copies of row 0)
+  if (bias) v = v + b_row;
+  if constexpr (PAIR) {
+    const int h = (int)f2h(v);
+    const int up = __shfl(h, (lane + RO) & 63);
+    if (lane < RO && n0 + lane < N) y[n0 + lane] = swiglu1((uint16_t)h, (uint16_t)up);
+  } else {
+    if (lane < R && n0 + lane < N) y[n0 + lane] = f2o(v, XM == XM_PLAIN && pp.bf16);
   }
 }
 
@@ -420,6 +437,14 @@ template <bool PG, int XM>
 hipError_t pick_stream(int K, const uint16_t* x, const int8_t* w, const float* sw,
                        const uint16_t* bias, uint16_t* y, int N, int gs, const MvProducer& pp,
                        hipStream_t s) {
+  // RMSNorm in the staging: two rows per wave at K = 4096 halve the workgroups
+  // that redo it, where three per CU are left (Qwen3-8B-shaped decode step, N =
+  // 6144: 2370 -> 2346 us; at K = 2048, N = 4096, one per CU, it lost).  A row is
+  // whole wave loads either way, so the bits do not change.
+  if constexpr (XM == XM_NORM || XM == XM_ADDNORM) {
+    if (K == 4096 && N >= 3 * num_cus() * kWpg * 2)
+      return run_stream<2, 8, PG, XM>(x, w, sw, bias, y, N, gs, pp, s);
+  }
 #define CIDER_MV(RR, CC) \
   case 1024 * CC / RR: return run_stream<RR, CC, PG, XM>(x, w, sw, bias, y, N, gs, pp, s)
   switch (K) {
@@ -509,6 +534,64 @@ bool stream_k(int K) {
 }
 
 }  // namespace
+
+namespace {
+
+template <int R, int C, int XM>
+hipError_t run_pair(const uint16_t* x, const int8_t* w, const float* sw, const uint16_t* bias,
+                    uint16_t* y, int N, const MvProducer& pp, hipStream_t s) {
+  constexpr int out = kWpg * R / 2;  // outputs per workgroup
+  mv_stream_kernel<R, C, false, XM, false, true>
+      <<<(N + out - 1) / out, kWpg * 64, 0, s>>>(x, w, sw, bias, y, N, 0, pp);
+  return hipGetLastError();
+}
+
+// (R, C) of the paired kernel for K.  K % 1024 == 0 only: a row is then whole
+// wave loads, so a row's sum does not depend on which row of the wave it is and
+// equals the plain MV's.  More rows per wave mean fewer workgroups that each
+// redo the norm; three per CU have to be left (K=4096: (4, 16) against (2, 8)
+// in a Qwen3-8B-shaped decode step, I = 12288: 2405 -> 2375 us; (8, 16) at
+// K=2048, I = 6144, 1.5 workgroups per CU, lost 2 %).
+template <int XM>
+hipError_t pick_pair(int K, const uint16_t* x, const int8_t* w, const float* sw,
+                     const uint16_t* bias, uint16_t* y, int N, const MvProducer& pp,
+                     hipStream_t s) {
+#define CIDER_MVP(RR, CC) \
+  case 1024 * CC / RR: return run_pair<RR, CC, XM>(x, w, sw, bias, y, N, pp, s)
+  switch (K) {
+    CIDER_MVP(4, 4);   // 1024
+    CIDER_MVP(4, 8);   // 2048
+    CIDER_MVP(2, 6);   // 3072
+    case 4096:
+      if (N >= 3 * num_cus() * kWpg * 2) return run_pair<4, 16, XM>(x, w, sw, bias, y, N, pp, s);
+      return run_pair<2, 8, XM>(x, w, sw, bias, y, N, pp, s);
+    CIDER_MVP(2, 10);  // 5120
+    CIDER_MVP(2, 12);  // 6144
+    CIDER_MVP(2, 14);  // 7168
+    CIDER_MVP(2, 16);  // 8192
+    default: return hipErrorNotSupported;
+  }
+#undef CIDER_MVP
+}
+
+}  // namespace
+
+bool mv_pair_supported(const void* x, const void* w, int K) {
+  switch (K) {
+    case 1024: case 2048: case 3072: case 4096: case 5120: case 6144: case 7168: case 8192:
+      return (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    default: return false;
+  }
+}
+
+hipError_t launch_mv_pair(int xm, const uint16_t* x, const int8_t* w, const float* sw,
+                          const uint16_t* bias, uint16_t* y, int N, int K, const MvProducer& pp,
+                          hipStream_t s) {
+  if (xm == XM_PLAIN) return pick_pair<XM_PLAIN>(K, x, w, sw, bias, y, N, pp, s);
+  if (xm == XM_NORM) return pick_pair<XM_NORM>(K, x, w, sw, bias, y, N, pp, s);
+  if (xm == XM_ADDNORM) return pick_pair<XM_ADDNORM>(K, x, w, sw, bias, y, N, pp, s);
+  return hipErrorInvalidValue;
+}
 
 bool mv_stream_supported(const void* x, const void* w, const void* sw, int K, int gs) {
   return stream_k(K) && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 &&

@@ -304,6 +304,40 @@ def rmsnorm_mv(x: torch.Tensor, weight: torch.Tensor, eps: float, linear,
     return (x.reshape(1, K) if h is None else h), y
 
 
+def gate_up_mv(x: torch.Tensor, linear, weight: Optional[torch.Tensor] = None,
+               eps: float = 1e-6, add: Optional[torch.Tensor] = None, stream=None):
+    """Decode (one token): SwiGLU of ``linear`` (a fused gate + up projection of
+    2I outputs, gate first) on x, or on RMSNorm of x (``weight``; of fp16(x +
+    add) when ``add`` is given), in one launch.  Bit-identical to ``rmsnorm_mv``
+    (or the linear) followed by ``silu_mul_quantize``'s y.  Returns (h, y): h
+    [1, K] (a new tensor when add is given, else x) and y [1, I] fp16; None
+    where the library has no such kernel (K not a multiple of 1024 up to 8192,
+    unaligned x)."""
+    fn = "gate_up_mv"
+    dev = _require_gpu(fn, x, weight, add)
+    K = x.numel()
+    _f16(fn, "x", x)
+    for name, t in (("weight", weight), ("add", add)):
+        if t is not None:
+            _f16(fn, name, t)
+            if t.numel() != K:
+                raise ValueError(f"{fn}: {name} has {t.numel()} elements, x has {K}")
+    w, sw, bias, N = _mv_linear(fn, linear, K)
+    if N % 2:
+        raise ValueError(f"{fn}: linear must hold gate and up of equal size")
+    lib = _lib.load()
+    with _on_stream(dev, stream):
+        h = torch.empty((1, K), dtype=torch.float16, device=dev) if add is not None else None
+        y = torch.empty((1, N // 2), dtype=torch.float16, device=dev)
+        rc = lib.cider_gate_up_mv(_ptr(x), _ptr(add), _ptr(h), _ptr(weight), float(eps), _ptr(w),
+                                  _ptr(sw), _ptr(bias), _ptr(y), N // 2, K,
+                                  _stream_ptr(dev, stream))
+    if rc == _lib.CIDER_E_UNSUPPORTED:
+        return None
+    _lib.check(rc)
+    return (x.reshape(1, K) if h is None else h), y
+
+
 def swiglu_mv(gate_up: torch.Tensor, linear, stream=None) -> torch.Tensor:
     """Decode (one token): ``linear(SwiGLU(gate_up))`` in one launch, gate_up
     [1, 2I] (gate first).  Bit-identical to

@@ -218,14 +218,10 @@ class Qwen3Layer(torch.nn.Module):
         ([1] int64; RoPE row `rope_pos`, default pos), attending over
         n_valid = pos + 1 cache positions."""
         c = self.cfg
-        # RMSNorm (+ residual add) and SwiGLU run inside the x staging of the
-        # MV that consumes them (bit-identical to the separate launches; one
-        # kernel fewer each) where that pays: every workgroup of the MV redoes
-        # the producer, so only for MVs of few workgroups / short rows
-        fuse_in = self.fuse_mv and _fuse_norm_into(c.hidden_size, c.qkv_out)
-        fuse_post = self.fuse_mv and _fuse_norm_into(c.hidden_size, 2 * c.intermediate_size)
-        fuse_act = self.fuse_mv and _fuse_swiglu_into(c.intermediate_size)
-        if fuse_in:
+        # RMSNorm (+ residual add) runs inside the x staging of the MV that
+        # consumes it, and SwiGLU as the output of the gate + up MV (bit-
+        # identical to the separate launches; one kernel fewer each)
+        if self.fuse_mv and _fuse_norm_into(c.hidden_size, c.qkv_out):
             h, qkv = FK.rmsnorm_mv(x, self.input_norm, c.rms_eps, self.qkv, add=pending)
         else:
             a = self._norm(x, pending, self.input_norm, True, False)
@@ -235,12 +231,18 @@ class Qwen3Layer(torch.nn.Module):
                             c.num_heads, c.num_kv_heads)
         attn = FK.attn_decode(q, k_cache, v_cache, n_valid, 1.0 / math.sqrt(c.head_dim), ws=ws)
         o = self.o(attn.reshape(1, -1))
-        if fuse_post:
+        r = (FK.gate_up_mv(h, self.gate_up, self.post_norm, c.rms_eps, add=o)
+             if self.fuse_mv else None)
+        if r is not None:
+            return r[0], self.down(r[1])
+        # other hidden sizes: SwiGLU inside the down MV's x staging where that
+        # pays (every workgroup of the MV redoes it, so for short rows)
+        if self.fuse_mv and _fuse_norm_into(c.hidden_size, 2 * c.intermediate_size):
             h2, gu = FK.rmsnorm_mv(h, self.post_norm, c.rms_eps, self.gate_up, add=o)
         else:
             b = self._norm(h, o, self.post_norm, True, False)
             h2, gu = b.h, self.gate_up(b.y)
-        if fuse_act:
+        if self.fuse_mv and _fuse_swiglu_into(c.intermediate_size):
             return h2, FK.swiglu_mv(gu, self.down)
         hs, _, _ = FK.silu_mul_quantize(gu, want_y=True, want_q=False)
         return h2, self.down(hs)

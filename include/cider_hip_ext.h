@@ -1,9 +1,10 @@
 /*
- * cider_hip_bf16.h - the linears of cider_hip.h on bfloat16 activations
- * (libcider_hip.so; conventions as in cider_hip.h).
+ * cider_hip_ext.h - entry points of libcider_hip.so beside those of
+ * cider_hip.h (same conventions): the linears on bfloat16 activations, and
+ * longer fusions of the decode step.
  */
-#ifndef CIDER_HIP_BF16_H
-#define CIDER_HIP_BF16_H
+#ifndef CIDER_HIP_EXT_H
+#define CIDER_HIP_EXT_H
 
 #include "cider_hip.h"
 
@@ -25,8 +26,20 @@ int cider_linear_bf16(int op, const void* x_bf16, const void* w, const void* sca
                       const void* bias_f16, void* y_bf16, void* ws, size_t ws_bytes,
                       int64_t M, int64_t N, int64_t K, int group_size, void* stream);
 
+/* The MLP's first half in one decode (M == 1) launch: y [I] = SwiGLU of the
+ * fused gate + up projection w [2I, K] (gate rows first), exactly as
+ * cider_rmsnorm_mv (norm_w non-NULL; with add and sum as there) or
+ * cider_perchannel_linear at M == 1 (norm_w NULL) on w, followed by
+ * cider_silu_mul_quantize's y. Bit-identical to that pair. K a multiple of 1024
+ * up to 8192, x and w 16-byte aligned; else CIDER_E_UNSUPPORTED (use the two
+ * calls). y must not overlap any input; sum must not overlap x or add. */
+int cider_gate_up_mv(const void* x_f16, const void* add_f16, void* sum_f16,
+                     const void* norm_w_f16, float eps, const int8_t* w,
+                     const float* scale_w, const void* bias_f16, void* y_f16,
+                     int64_t I, int64_t K, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
 
-#endif /* CIDER_HIP_BF16_H */
+#endif /* CIDER_HIP_EXT_H */

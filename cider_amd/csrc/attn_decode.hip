@@ -33,6 +33,7 @@
 //     several workgroups that each read that KV head's chunk.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "norm_common.hpp"
 
 namespace cider {
 
@@ -66,11 +67,19 @@ __device__ __forceinline__ float dot8(i32x4 a, i32x4 b, float s) {
 // below hold G * 8 KB); R = (H / KV) / G workgroups share a KV head.
 // workspace layout per (head block y, chunk c): G * (kD + 2) floats:
 // o_c[G][kD], m_c[G], l_c[G]
-template <int G, int R>
+//
+// ROPE: q is the token's fused projection [q heads | k heads | v heads], and
+// each workgroup norms and rotates its G query heads itself (eight lanes per
+// head, the arithmetic of qk_norm_rope_kernel, so the same bits), from LDS; the
+// workgroup whose chunk holds the token's slot does the same for the KV head's
+// key, writes key and value to the caches and attends the values it computed
+// instead of the cache rows it loaded meanwhile.  One launch less per layer; the
+// loads of the projection run beside those of the chunk.
+template <int G, int R, bool ROPE>
 __global__ __launch_bounds__(256) void attn_chunk_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
-    const uint16_t* __restrict__ vc, const int64_t* __restrict__ n_ptr, float scale,
-    float* __restrict__ ws, int64_t T, int nchunk) {
+    const uint16_t* __restrict__ q, uint16_t* kc, uint16_t* vc,
+    const int64_t* __restrict__ n_ptr, float scale, float* __restrict__ ws, int64_t T, int nchunk,
+    const DecodeRope rp) {
   __shared__ __attribute__((aligned(16))) uint16_t qs[G][kD];
   __shared__ float part[16][G][kChunk];  // dimension / position slices
   __shared__ float ps[G][kChunk];        // scores, then probabilities
@@ -80,7 +89,11 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
   const int64_t nn = *n_ptr;
   const int64_t n = nn < T ? nn : T;
   const int64_t c0 = (int64_t)c * kChunk;
-  if (c0 >= n) return;  // uniform: nothing of this chunk is valid
+  const int64_t p = ROPE ? *rp.slot : -1;
+  const bool mine = ROPE && p >= c0 && p < c0 + kChunk && p < T;
+  // uniform: nothing of this chunk is valid (nor written)
+  if (c0 >= n && !mine) return;
+  [[maybe_unused]] __shared__ __attribute__((aligned(16))) uint16_t new_kv[2][kD];
 
   // Issue every load of the chunk first (K for the scores, V for P.V: neither
   // depends on the other), so the chunk costs one memory latency.  Positions
@@ -98,8 +111,55 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) vv[i] = ld16(vp + (int64_t)i * kD);
   }
-  for (int e = tid; e < G * kD; e += 256) qs[e / kD][e % kD] = q[(int64_t)y * G * kD + e];
-  __syncthreads();
+  if constexpr (ROPE) {
+    // threads 8r .. 8r+7: query head r; 64 .. 71: the key; 128 .. 135: the value
+    const int j8 = tid & 7, hr = tid >> 3;
+    const bool is_q = hr < G, is_k = mine && hr == 8, is_v = mine && hr == 16;
+    if (is_q || is_k || is_v) {
+      const int KV = rp.KV, H = G * R * KV;
+      const int hh = is_q ? y * G + hr : is_k ? H + j : H + KV + j;
+      const uint16_t* src = q + (int64_t)hh * kD + 8 * j8;
+      i32x4 o0 = ld16(src), o1 = ld16(src + 64);
+      const int64_t rr = *rp.rope_row;
+      const bool has_row = rr >= 0 && rr < rp.P;
+      if (!is_v) {
+        const int64_t rc = (has_row ? rr : 0) * kD + 8 * j8;
+        const uint16_t* wn = (is_q ? rp.qw : rp.kw) + 8 * j8;
+        const i32x4 x0 = o0, x1 = o1;
+        norm_rope8(x0, x1, ld16(wn), ld16(wn + 64), ld16(rp.cos_t + rc), ld16(rp.cos_t + rc + 64),
+                   ld16(rp.sin_t + rc), ld16(rp.sin_t + rc + 64), head_sumsq(x0, x1), rp.eps, o0,
+                   o1);
+      }
+      if (is_q && !has_row) {  // as qk_norm_rope: quiet NaN
+        o0 = i32x4{0x7E007E00, 0x7E007E00, 0x7E007E00, 0x7E007E00};
+        o1 = o0;
+      }
+      uint16_t* const dst = is_q ? qs[hr] : new_kv[is_v];
+      uint16_t* const row = (is_v ? vc : kc) + ((int64_t)j * T + p) * kD;
+      if (is_k && !has_row) {  // no key is written: what the cache holds stays
+        o0 = ld16(row + 8 * j8);
+        o1 = ld16(row + 8 * j8 + 64);
+      } else if (!is_q && y % R == 0) {
+        *reinterpret_cast<i32x4*>(row + 8 * j8) = o0;
+        *reinterpret_cast<i32x4*>(row + 8 * j8 + 64) = o1;
+      }
+      *reinterpret_cast<i32x4*>(dst + 8 * j8) = o0;
+      *reinterpret_cast<i32x4*>(dst + 8 * j8 + 64) = o1;
+    }
+    __syncthreads();
+    if (c0 >= n) return;  // uniform: only the write was due
+    if (mine) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (tk0 + i == p) kv[i] = *reinterpret_cast<const i32x4*>(&new_kv[0][8 * dq]);
+        if (tv0 + i == p) vv[i] = *reinterpret_cast<const i32x4*>(&new_kv[1][8 * dv]);
+      }
+    }
+  } else {
+    for (int e = tid; e < G * kD / 8; e += 256)
+      *reinterpret_cast<i32x4*>(&qs[0][8 * e]) = ld16(q + (int64_t)y * G * kD + 8 * e);
+    __syncthreads();
+  }
 
   // ---- scores: thread (dq, tq) sums dimensions 8dq..8dq+7 for positions
   // c0 + 8tq .. +7
@@ -256,11 +316,16 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float* __restrict_
 }
 
 template <int G, int R>
-hipError_t run_attn(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int64_t* n,
-                    float scale, float* ws, uint16_t* out, int KV, int64_t T, hipStream_t s) {
+hipError_t run_attn(const uint16_t* q, uint16_t* kc, uint16_t* vc, const int64_t* n, float scale,
+                    float* ws, uint16_t* out, int KV, int64_t T, const DecodeRope* rp,
+                    hipStream_t s) {
   const int nchunk = (int)((T + kChunk - 1) / kChunk);
-  attn_chunk_kernel<G, R><<<dim3(nchunk, KV * R), 256, 0, s>>>(q, kc, vc, n, scale, ws, T,
-                                                                nchunk);
+  const dim3 grid(nchunk, KV * R);
+  if (rp)
+    attn_chunk_kernel<G, R, true><<<grid, 256, 0, s>>>(q, kc, vc, n, scale, ws, T, nchunk, *rp);
+  else
+    attn_chunk_kernel<G, R, false><<<grid, 256, 0, s>>>(q, kc, vc, n, scale, ws, T, nchunk,
+                                                         DecodeRope{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   attn_merge_kernel<G><<<KV * R * G, 64, 0, s>>>(ws, n, out, nchunk, T);
@@ -277,11 +342,19 @@ size_t attn_decode_ws_floats(int H, int64_t T) {
 hipError_t launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc,
                               const int64_t* n, float scale, float* ws, uint16_t* out, int H,
                               int KV, int64_t T, hipStream_t s) {
+  // written only with rotary arguments
+  return launch_attn_decode_rope(q, const_cast<uint16_t*>(kc), const_cast<uint16_t*>(vc), n,
+                                 scale, ws, out, H, KV, T, nullptr, s);
+}
+
+hipError_t launch_attn_decode_rope(const uint16_t* q, uint16_t* kc, uint16_t* vc,
+                                   const int64_t* n, float scale, float* ws, uint16_t* out, int H,
+                                   int KV, int64_t T, const DecodeRope* rp, hipStream_t s) {
   switch (H / KV) {
-    case 1: return run_attn<1, 1>(q, kc, vc, n, scale, ws, out, KV, T, s);
-    case 2: return run_attn<2, 1>(q, kc, vc, n, scale, ws, out, KV, T, s);
-    case 4: return run_attn<4, 1>(q, kc, vc, n, scale, ws, out, KV, T, s);
-    case 8: return run_attn<4, 2>(q, kc, vc, n, scale, ws, out, KV, T, s);
+    case 1: return run_attn<1, 1>(q, kc, vc, n, scale, ws, out, KV, T, rp, s);
+    case 2: return run_attn<2, 1>(q, kc, vc, n, scale, ws, out, KV, T, rp, s);
+    case 4: return run_attn<4, 1>(q, kc, vc, n, scale, ws, out, KV, T, rp, s);
+    case 8: return run_attn<4, 2>(q, kc, vc, n, scale, ws, out, KV, T, rp, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -759,6 +759,57 @@ int cider_attn_decode(const void* q_f16, const void* k_cache_f16, const void* v_
       fn);
 }
 
+int cider_attn_decode_rope(const void* qkv_f16, const void* q_norm_w_f16,
+                           const void* k_norm_w_f16, float eps, const void* cos_f16,
+                           const void* sin_f16, int64_t P, const int64_t* rope_row,
+                           const int64_t* slot, void* k_cache_f16, void* v_cache_f16,
+                           const int64_t* n_valid, float scale, void* ws, size_t ws_bytes,
+                           void* out_f16, int64_t H, int64_t KV, int64_t D, int64_t T,
+                           void* stream) {
+  static const char* fn = "cider_attn_decode_rope";
+  if (D != 128) return fail(CIDER_E_INVALID, "%s: head_dim must be 128 (got %lld)", fn, (long long)D);
+  if (H <= 0 || KV <= 0 || H > 4096 || H % KV != 0 ||
+      (H / KV != 1 && H / KV != 2 && H / KV != 4 && H / KV != 8))
+    return fail(CIDER_E_INVALID, "%s: H/KV must be 1, 2, 4 or 8 (H=%lld KV=%lld)", fn,
+                (long long)H, (long long)KV);
+  if (T <= 0 || T > kMaxDim || T % 8 != 0)
+    return fail(CIDER_E_INVALID, "%s: cache capacity T=%lld must be a positive multiple of 8",
+                fn, (long long)T);
+  if (P <= 0 || P > kMaxDim)
+    return fail(CIDER_E_INVALID, "%s: bad table size P=%lld", fn, (long long)P);
+  if (!(eps >= 0.0f)) return fail(CIDER_E_INVALID, "%s: eps must be >= 0", fn);
+  const void* const f16[] = {qkv_f16, q_norm_w_f16, k_norm_w_f16, cos_f16,
+                             sin_f16, k_cache_f16,  v_cache_f16};
+  static const char* const names[] = {"qkv", "q_norm_w", "k_norm_w", "cos",
+                                      "sin", "k_cache",  "v_cache"};
+  for (int i = 0; i < 7; ++i) {
+    CIDER_TRY(need(fn, f16[i], names[i], true));
+    if (!aligned16(f16[i]))
+      return fail(CIDER_E_INVALID, "%s: %s must be 16-byte aligned", fn, names[i]);
+  }
+  CIDER_TRY(need(fn, rope_row, "rope_row", true));
+  CIDER_TRY(need(fn, slot, "slot", true));
+  CIDER_TRY(need(fn, n_valid, "n_valid", true));
+  CIDER_TRY(need(fn, out_f16, "out", true));
+  CIDER_TRY(check_ws(fn, ws, ws_bytes, cider_attn_decode_workspace_bytes(H, T)));
+  cider::DecodeRope rp;
+  rp.qw = reinterpret_cast<const uint16_t*>(q_norm_w_f16);
+  rp.kw = reinterpret_cast<const uint16_t*>(k_norm_w_f16);
+  rp.cos_t = reinterpret_cast<const uint16_t*>(cos_f16);
+  rp.sin_t = reinterpret_cast<const uint16_t*>(sin_f16);
+  rp.eps = eps;
+  rp.P = P;
+  rp.rope_row = rope_row;
+  rp.slot = slot;
+  rp.KV = (int)KV;
+  return hip_status(
+      cider::launch_attn_decode_rope(
+          reinterpret_cast<const uint16_t*>(qkv_f16), reinterpret_cast<uint16_t*>(k_cache_f16),
+          reinterpret_cast<uint16_t*>(v_cache_f16), n_valid, scale, reinterpret_cast<float*>(ws),
+          reinterpret_cast<uint16_t*>(out_f16), (int)H, (int)KV, T, &rp, (hipStream_t)stream),
+      fn);
+}
+
 size_t cider_attn_prefill_workspace_bytes(int64_t c, int64_t n, int64_t H) {
   if (H <= 0 || H > 4096 || c < 1 || n < c || n > ((int64_t)1 << 24) || c * H > kMaxDim)
     return 0;

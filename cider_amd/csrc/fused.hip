@@ -281,26 +281,6 @@ __global__ __launch_bounds__(256) void silu_mul_ew_kernel(const uint16_t* __rest
   *reinterpret_cast<i32x4*>(y + row * I + 8 * e) = swiglu8(ld16(g + 8 * e), ld16(g + I + 8 * e));
 }
 
-// ---------------------------------------------------------------------------
-// per-head q/k RMSNorm + RoPE + KV-cache write (head_dim 128)
-// ---------------------------------------------------------------------------
-// Eight lanes per (token, head) of the fused projection row [q heads | k
-// heads | v heads], eight heads per wave: lane j of a head holds elements
-// [8j, 8j + 8) and [64 + 8j, 64 + 8j + 8), which are the pairs the
-// rotate-half RoPE mixes, so every access is 16 bytes.  The head's sum of
-// squares: each lane's 16 squares in order, then pairs, quads and the 8-lane
-// group by DPP moves.  Per element: n = h(w * h(x * r)), out = h(h(n * cos) +
-// h(-n' * sin)) for the first half (n' its partner) and h(h(n * cos) +
-// h(n' * sin)) for the second.  (One wave per head with 2-byte lanes ran the
-// 2048-token prefill's 2048 x 48 heads in 29.5 us per call; this layout in
-// 15.6 us.)
-__device__ __forceinline__ float group8_sum(float v) {
-  v = v + __builtin_bit_cast(float, dpp_mov<kDppXor1>(__builtin_bit_cast(int32_t, v)));
-  v = v + __builtin_bit_cast(float, dpp_mov<kDppXor2>(__builtin_bit_cast(int32_t, v)));
-  v = v + __builtin_bit_cast(float, dpp_mov<kDppMirror8>(__builtin_bit_cast(int32_t, v)));
-  return v;
-}
-
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ qw,
     const uint16_t* __restrict__ kw, float eps, const uint16_t* __restrict__ cos_t,
@@ -333,10 +313,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
   const i32x4 w0 = ld16(wn + 8 * j), w1 = ld16(wn + 64 + 8 * j);
   const i32x4 c0 = ld16(cos_t + rrc * D + 8 * j), c1 = ld16(cos_t + rrc * D + 64 + 8 * j);
   const i32x4 s0 = ld16(sin_t + rrc * D + 8 * j), s1 = ld16(sin_t + rrc * D + 64 + 8 * j);
-  float ss = 0.0f;
-  ss = sumsq8(x0, ss);
-  ss = sumsq8(x1, ss);
-  ss = group8_sum(ss);  // every lane of the head's group
+  const float ss = head_sumsq(x0, x1);
   if (!has_row) {
     // No RoPE row: the k cache is left alone, and the q heads get a quiet
     // NaN, so a caller that feeds them on sees the error instead of stale
@@ -349,27 +326,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     }
     return;
   }
-  const float r = 1.0f / sqrtf(ss / (float)D + eps);
-  const i32x4 n0 = norm8(x0, w0, r), n1 = norm8(x1, w1, r);
   i32x4 o0, o1;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    uint16_t lo[2], hi[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const float a = h2f(h ? hi16(n0[e]) : lo16(n0[e]));
-      const float b = h2f(h ? hi16(n1[e]) : lo16(n1[e]));
-      const float ca = h2f(h ? hi16(c0[e]) : lo16(c0[e]));
-      const float sa = h2f(h ? hi16(s0[e]) : lo16(s0[e]));
-      const float cb = h2f(h ? hi16(c1[e]) : lo16(c1[e]));
-      const float sb = h2f(h ? hi16(s1[e]) : lo16(s1[e]));
-      // out = x * cos + rotate_half(x) * sin, rotate_half(x) = [-x[64:], x[:64]]
-      lo[h] = f2h(h2f(f2h(a * ca)) + h2f(f2h(-(b * sa))));
-      hi[h] = f2h(h2f(f2h(b * cb)) + h2f(f2h(a * sb)));
-    }
-    o0[e] = pack2(lo[0], lo[1]);
-    o1[e] = pack2(hi[0], hi[1]);
-  }
+  norm_rope8(x0, x1, w0, w1, c0, c1, s0, s1, ss, eps, o0, o1);
   uint16_t* dst;
   if (hh < H) {
     dst = q_out + (t * H + hh) * D;

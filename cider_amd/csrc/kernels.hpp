@@ -149,6 +149,19 @@ hipError_t launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint1
                               const int64_t* n, float scale, float* ws, uint16_t* out, int H,
                               int KV, int64_t T, hipStream_t s);
 
+// The same with q the fused projection [H + 2 KV, 128] of the token: q / k norm,
+// RoPE and the cache write of qk_norm_rope run inside (rp non-NULL).
+struct DecodeRope {
+  const uint16_t *qw = nullptr, *kw = nullptr, *cos_t = nullptr, *sin_t = nullptr;
+  float eps = 0.0f;
+  int64_t P = 0;
+  const int64_t *rope_row = nullptr, *slot = nullptr;
+  int KV = 0;
+};
+hipError_t launch_attn_decode_rope(const uint16_t* q, uint16_t* kc, uint16_t* vc,
+                                   const int64_t* n, float scale, float* ws, uint16_t* out, int H,
+                                   int KV, int64_t T, const DecodeRope* rp, hipStream_t s);
+
 // Causal attention of a prefill chunk over the KV cache (attn_prefill.hip):
 // c queries at cache slots n - c .. n - 1, D == 128, H % KV == 0 (n_dev: n
 // read on the device, n its upper bound).  Launches

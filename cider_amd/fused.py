@@ -171,6 +171,50 @@ def attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     return out
 
 
+def attn_decode_rope(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Tensor,
+                     eps: float, cos: torch.Tensor, sin: torch.Tensor, rope_row: torch.Tensor,
+                     slot: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                     n_valid: torch.Tensor, scale: float, num_heads: int, num_kv_heads: int,
+                     ws: Optional[torch.Tensor] = None, stream=None) -> torch.Tensor:
+    """``qk_norm_rope`` of one token's fused projection qkv [(H + 2 KV) * 128]
+    and ``attn_decode`` on its query heads, two launches instead of three and
+    bit-identical: writes the token's key and value at ``slot`` and returns
+    fp16 [H * 128], the attention over the first n_valid[0] rows."""
+    fn = "attn_decode_rope"
+    dev = _require_gpu(fn, qkv, q_norm_w, k_norm_w, cos, sin, rope_row, slot, k_cache, v_cache,
+                       n_valid, ws)
+    D = 128
+    H, KV = int(num_heads), int(num_kv_heads)
+    for name, t, size in (("qkv", qkv, (H + 2 * KV) * D), ("q_norm_w", q_norm_w, D),
+                          ("k_norm_w", k_norm_w, D)):
+        _f16(fn, name, t)
+        if t.numel() != size:
+            raise ValueError(f"{fn}: {name} must hold {size} values")
+    for name, t in (("cos", cos), ("sin", sin), ("k_cache", k_cache), ("v_cache", v_cache)):
+        _f16(fn, name, t)
+    if cos.shape != sin.shape or cos.dim() != 2 or cos.shape[1] != D:
+        raise ValueError(f"{fn}: cos and sin must be [P, {D}]")
+    if k_cache.dim() != 3 or k_cache.shape[0] != KV or k_cache.shape[2] != D:
+        raise ValueError(f"{fn}: k_cache must be [{KV}, T, {D}]")
+    T = k_cache.shape[1]
+    if v_cache.shape != k_cache.shape:
+        raise ValueError(f"{fn}: v_cache must be [{KV}, {T}, {D}]")
+    for name, t in (("rope_row", rope_row), ("slot", slot), ("n_valid", n_valid)):
+        if t.dtype != torch.int64 or t.numel() < 1:
+            raise ValueError(f"{fn}: {name} must be an int64 tensor")
+    lib = _lib.load()
+    with _on_stream(dev, stream):
+        if ws is None:
+            ws = attn_decode_workspace(H, T, dev)
+        out = torch.empty(H * D, dtype=torch.float16, device=dev)
+        _lib.check(lib.cider_attn_decode_rope(
+            _ptr(qkv), _ptr(q_norm_w), _ptr(k_norm_w), float(eps), _ptr(cos), _ptr(sin),
+            cos.shape[0], _ptr(rope_row), _ptr(slot), _ptr(k_cache), _ptr(v_cache),
+            _ptr(n_valid), float(scale), _ptr(ws), ws.numel(), _ptr(out), H, KV, D, T,
+            _stream_ptr(dev, stream)))
+    return out
+
+
 def attn_prefill_workspace(c: int, n: int, num_heads: int, device) -> Optional[torch.Tensor]:
     """The workspace a chunk of c queries over n slots splits its keys into
     (None when the launch does not split)."""

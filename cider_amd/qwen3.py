@@ -226,10 +226,10 @@ class Qwen3Layer(torch.nn.Module):
         else:
             a = self._norm(x, pending, self.input_norm, True, False)
             h, qkv = a.h, self.qkv(a.y)
-        q = FK.qk_norm_rope(qkv, self.q_norm, self.k_norm, c.rms_eps, tables[0], tables[1],
-                            pos if rope_pos is None else rope_pos, pos, k_cache, v_cache,
-                            c.num_heads, c.num_kv_heads)
-        attn = FK.attn_decode(q, k_cache, v_cache, n_valid, 1.0 / math.sqrt(c.head_dim), ws=ws)
+        attn = FK.attn_decode_rope(qkv, self.q_norm, self.k_norm, c.rms_eps, tables[0],
+                                   tables[1], pos if rope_pos is None else rope_pos, pos,
+                                   k_cache, v_cache, n_valid, 1.0 / math.sqrt(c.head_dim),
+                                   c.num_heads, c.num_kv_heads, ws=ws)
         o = self.o(attn.reshape(1, -1))
         r = (FK.gate_up_mv(h, self.gate_up, self.post_norm, c.rms_eps, add=o)
              if self.fuse_mv else None)

@@ -38,6 +38,22 @@ int cider_gate_up_mv(const void* x_f16, const void* add_f16, void* sum_f16,
                      const float* scale_w, const void* bias_f16, void* y_f16,
                      int64_t I, int64_t K, void* stream);
 
+/* cider_qk_norm_rope of one token (L == 1) and cider_attn_decode on its query
+ * heads in one call, two launches instead of three: qkv [(H + 2 KV) * 128] is
+ * the token's fused projection; its key and value go to cache row *slot as
+ * there (nothing is written for a slot outside [0, T), and no key for a
+ * *rope_row outside [0, P), which makes the output NaN), and the attention runs
+ * over the first min(*n_valid, T) rows, the written one among them.
+ * Bit-identical to the two calls. Requirements of both; every fp16 array
+ * 16-byte aligned. */
+int cider_attn_decode_rope(const void* qkv_f16, const void* q_norm_w_f16,
+                           const void* k_norm_w_f16, float eps, const void* cos_f16,
+                           const void* sin_f16, int64_t P, const int64_t* rope_row,
+                           const int64_t* slot, void* k_cache_f16, void* v_cache_f16,
+                           const int64_t* n_valid, float scale, void* ws, size_t ws_bytes,
+                           void* out_f16, int64_t H, int64_t KV, int64_t D, int64_t T,
+                           void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -71,3 +71,31 @@ def test_rmsnorm_mv_rows_per_wave(N):
     _, y = F.rmsnorm_mv(x, nw, 1e-6, lin)
     y2 = lin(F.rmsnorm_quantize(x, nw, 1e-6, want_q=False).y)
     assert torch.equal(bits(y), bits(y2))
+
+
+# slot at the edges of a 128-row chunk, at the cache's last row, past the valid
+# length (written, not attended) and outside the cache; rope_row outside the
+# tables; every grouping
+@pytest.mark.parametrize("H,KV", [(4, 4), (16, 8), (32, 8), (16, 2)])
+@pytest.mark.parametrize("n,slot,row", [(1, 0, 0), (128, 127, 127), (129, 128, 128),
+                                        (300, 299, 17), (384, 383, 383), (500, 383, 1),
+                                        (100, 200, 5), (300, -1, 3), (300, 384, 3),
+                                        (300, 299, 400), (300, 299, -1)])
+def test_attn_decode_rope(H, KV, n, slot, row):
+    T, P, D = 384, 400, 128
+    g = torch.Generator(device=DEV).manual_seed(H * 1000 + n + slot)
+
+    def rand(*s):
+        return torch.randn(*s, device=DEV, generator=g).half()
+
+    qkv, qw, kw = rand((H + 2 * KV) * D), rand(D), rand(D)
+    cos, sin, kc, vc = rand(P, D), rand(P, D), rand(KV, T, D), rand(KV, T, D)
+    i64 = dict(dtype=torch.int64, device=DEV)
+    rr, sl, nv = (torch.tensor([v], **i64) for v in (row, slot, n))
+    k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+    out = F.attn_decode_rope(qkv, qw, kw, 1e-6, cos, sin, rr, sl, k1, v1, nv, 0.09, H, KV)
+    q = F.qk_norm_rope(qkv.view(1, -1), qw, kw, 1e-6, cos, sin, rr, sl, k2, v2, H, KV)
+    e = F.attn_decode(q, k2, v2, nv, 0.09)
+    assert torch.equal(bits(k1), bits(k2)) and torch.equal(bits(v1), bits(v2))
+    assert torch.equal(out.isnan(), e.isnan())
+    assert torch.equal(bits(out)[~e.isnan()], bits(e)[~e.isnan()])

@@ -16,6 +16,8 @@ device pointers and streams from torch are valid in our calls.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -114,6 +116,35 @@ def load():
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+FAST_PATH = os.path.join(LIB_DIR, "_cider_fast.so")
+_fast_linear = None
+
+
+def fast_linear():
+    """The native common case of a linear call (``csrc/fast_linear.cpp``):
+    ``linear(op, x, w, scale, bias, group_size, any_dim)`` -> Tensor, or None
+    for a call it does not take.  RuntimeError if the extension is absent."""
+    global _fast_linear
+    if _fast_linear is not None:
+        return _fast_linear
+    load()
+    with _lock:
+        if _fast_linear is None:
+            if not os.path.exists(FAST_PATH):
+                raise RuntimeError(
+                    f"cider_amd Python extension not built: {FAST_PATH} is missing "
+                    "(run `make -C cider_amd/csrc`)")
+            loader = importlib.machinery.ExtensionFileLoader("_cider_fast", FAST_PATH)
+            try:
+                mod = importlib.util.module_from_spec(
+                    importlib.util.spec_from_loader("_cider_fast", loader))
+                loader.exec_module(mod)
+            except ImportError as e:
+                raise RuntimeError(f"cider_amd Python extension failed to load: {e}") from e
+            _fast_linear = mod.linear
+    return _fast_linear
 
 
 def check(rc: int) -> None:

@@ -70,42 +70,21 @@ class CiderLinear(torch.nn.Module):
         self.group_size = group_size
         self._in_features = in_features
         self._out_features = out_features
-        self._ws_cache = {}
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        b = self._buffers
+        op = _lib.CIDER_OP_PERGROUP if self.group_size else _lib.CIDER_OP_PERCHANNEL
+        y = ops._fast(op, x, b.get("w_int8"), b.get("scale_w"), b.get("bias"),
+                      self.group_size, None, True)
+        if y is not None:
+            return y
         orig_shape = x.shape
         x2 = x.reshape(-1, self._in_features)
-        if (self._mode == "per_channel" and x2.dtype == torch.float16 and x2.is_cuda
-                and x2.is_contiguous() and x2.device == self.w_int8.device):
-            y = self._perchannel_direct(x2)
-        elif self._mode == "per_channel":
+        if self._mode == "per_channel":
             y = ops.perchannel_linear(x2, self.w_int8, self.scale_w, self.bias)
         else:
             y = ops.pergroup_linear(x2, self.w_int8, self.scale_w, self.group_size, self.bias)
         return y.reshape(*orig_shape[:-1], self._out_features)
-
-    def _perchannel_direct(self, x2: torch.Tensor) -> torch.Tensor:
-        """Per-channel call straight into the C ABI for the common case (fp16,
-        contiguous, same device): the buffers are already in the library's
-        types, so only the output and the workspace are allocated.  The
-        launch goes to the current stream, so it can be captured in a graph."""
-        lib = _lib.load()
-        M = x2.shape[0]
-        N, K = self._out_features, self._in_features
-        dev = x2.device
-        nb = self._ws_cache.get(M)
-        if nb is None:
-            nb = _lib.workspace_bytes(_lib.CIDER_OP_PERCHANNEL, M, N, K, 0)
-            self._ws_cache[M] = nb
-        y = torch.empty((M, N), dtype=torch.float16, device=dev)
-        ws = torch.empty(nb, dtype=torch.uint8, device=dev) if nb else None
-        rc = lib.cider_perchannel_linear(
-            x2.data_ptr(), self.w_int8.data_ptr(), self.scale_w.data_ptr(), self.bias.data_ptr(),
-            y.data_ptr(), ws.data_ptr() if ws is not None else None, nb, M, N, K,
-            torch.cuda.current_stream(dev).cuda_stream)
-        if rc != 0:
-            _lib.check(rc)
-        return y
 
     def forward_quantized(self, q: torch.Tensor, scale_a: torch.Tensor) -> torch.Tensor:
         """Per-channel linear on activations already quantized per token
@@ -207,12 +186,16 @@ class W4A8Linear(torch.nn.Module):
         self._w4_sig = None
         self._w4_done = None
 
+    # the stream (handle) the copy was made on
+    _w4_stream = None
+
     def _packed_nk(self) -> torch.Tensor:
         """The library-layout copy, ordered for the current stream: a repack
-        runs on the calling stream and records an event; every use waits for
-        that event on its own stream and marks the copy as used there, so the
-        caching allocator keeps the memory until that stream's work is done
-        even after a later repack replaces the copy."""
+        runs on the calling stream and records an event; every use on another
+        stream waits for that event there and marks the copy as used there, so
+        the caching allocator keeps the memory until that stream's work is done
+        even after a later repack replaces the copy.  On the stream that made
+        the copy, and whose pool it is from, both hold by stream order."""
         w = self.packed_weight
         use = torch.cuda.current_stream(w.device)
         sig = (w._version, w.data_ptr(), tuple(w.shape), w.device)
@@ -221,7 +204,10 @@ class W4A8Linear(torch.nn.Module):
             done = torch.cuda.Event()
             done.record(use)
             self._w4_nk, self._w4_sig, self._w4_done = out, sig, done
+            self._w4_stream = use.cuda_stream
             return out
+        if use.cuda_stream == self._w4_stream:
+            return self._w4_nk
         use.wait_event(self._w4_done)
         self._w4_nk.record_stream(use)
         return self._w4_nk
@@ -230,11 +216,16 @@ class W4A8Linear(torch.nn.Module):
         self._w4_nk = None
         self._w4_sig = None
         self._w4_done = None
+        self._w4_stream = None
         super()._load_from_state_dict(*args, **kwargs)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        w4 = self._packed_nk()
+        y = ops._fast(_lib.CIDER_OP_W4A8, x, w4, self._buffers.get("scale"), None, 0, None, True)
+        if y is not None:
+            return y
         orig_shape = x.shape
-        y = ops.w4a8_linear_packed(x.reshape(-1, self._K), self._packed_nk(), self.scale)
+        y = ops.w4a8_linear_packed(x.reshape(-1, self._K), w4, self.scale)
         return y.reshape(*orig_shape[:-1], self.output_dims)
 
     @staticmethod
@@ -273,6 +264,11 @@ class W4A8GroupLinear(torch.nn.Module):
         self._K = 2 * self.packed_weight.shape[1]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        b = self._buffers
+        y = ops._fast(_lib.CIDER_OP_W4A8_PERGROUP, x, b.get("packed_weight"), b.get("scales"), self.bias,
+                      self.group_size, None, True)
+        if y is not None:
+            return y
         orig_shape = x.shape
         y = ops.w4a8_pergroup_linear(x.reshape(-1, self._K), self.packed_weight, self.scales,
                                      self.group_size, self.bias)

@@ -218,6 +218,14 @@ def _cast_out(y: torch.Tensor, dtype) -> torch.Tensor:
     return y if dtype == torch.float16 else y.to(dtype)
 
 
+def _fast(op: int, x, w, scale, bias, gs: int, stream, any_dim: bool = False):
+    """The whole linear in one native call where its operands need no
+    conversion; None sends the call through the checks and casts below."""
+    if stream is not None:
+        return None
+    return (_lib._fast_linear or _lib.fast_linear())(op, x, w, scale, bias, gs, any_dim)
+
+
 def _linear_bf16(op: int, x, w, scale, bias, M: int, N: int, K: int, gs: int, dev,
                  stream) -> Optional[torch.Tensor]:
     """A linear on bfloat16 x with a bfloat16 result in one library call (the
@@ -270,6 +278,9 @@ def perchannel_linear(x: torch.Tensor, w: torch.Tensor, scale_w: torch.Tensor,
     fp16-activation MV, M >= 2 quantizes x per token and runs the int8 GEMM
     with the fused per-channel epilogue.  Returns [M, N] in x's dtype.
     """
+    y = _fast(_lib.CIDER_OP_PERCHANNEL, x, w, scale_w, bias, 0, stream)
+    if y is not None:
+        return y
     fn = "perchannel_linear"
     dev = _require_gpu(fn, x, w, scale_w, bias)
     _check_2d(fn, "x", x, "[M,K]")
@@ -341,8 +352,11 @@ def pergroup_linear(x: torch.Tensor, w: torch.Tensor, scale_w: torch.Tensor,
     the per-group GEMM.  ``new_bias`` is accepted and ignored, as the
     reference's kernels ignore it (``cider/ops.py:151-158,197-201``).
     """
-    fn = "pergroup_linear"
     del new_bias
+    y = _fast(_lib.CIDER_OP_PERGROUP, x, w, scale_w, bias, group_size, stream)
+    if y is not None:
+        return y
+    fn = "pergroup_linear"
     dev = _require_gpu(fn, x, w, scale_w, bias)
     _check_2d(fn, "x", x, "[M,K]")
     _check_2d(fn, "w", w, "[N,K]")
@@ -470,6 +484,9 @@ _repack_cache = _RepackCache()
 def w4a8_linear_packed(x: torch.Tensor, w4_nk: torch.Tensor, scale_w: torch.Tensor,
                        stream=None) -> torch.Tensor:
     """W4A8 linear on weights already in the library layout [N, K/2]."""
+    y = _fast(_lib.CIDER_OP_W4A8, x, w4_nk, scale_w, None, 0, stream)
+    if y is not None:
+        return y
     fn = "w4a8_linear"
     dev = _require_gpu(fn, x, w4_nk, scale_w)
     _check_2d(fn, "x", x, "[M,K]")
@@ -518,6 +535,9 @@ def w4a8_pergroup_linear(x: torch.Tensor, w4_nk: torch.Tensor, scales: torch.Ten
                          stream=None) -> torch.Tensor:
     """W4A8 per-group linear (extension): w4_nk uint8 [N, K/2] low nibble first,
     scales float16 [K // group_size, N], group_size in {64, 128}."""
+    y = _fast(_lib.CIDER_OP_W4A8_PERGROUP, x, w4_nk, scales, bias, group_size, stream)
+    if y is not None:
+        return y
     fn = "w4a8_pergroup_linear"
     dev = _require_gpu(fn, x, w4_nk, scales, bias)
     _check_2d(fn, "x", x, "[M,K]")

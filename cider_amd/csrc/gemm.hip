@@ -365,6 +365,16 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
+// The conditions under which launch_gemm below reaches the one-set per-group
+// kernel with int4 weights (fp16 scales).
+bool w4_pg_wants_il(const GemmArgs& a, int gs) {
+  const bool vec = a.K % 128 == 0 && a.N % 8 == 0 && aligned16(a.x) && aligned16(a.w) &&
+                   aligned16(a.y) && aligned16(a.sw) &&
+                   (int64_t)a.K * 256 < ((int64_t)1 << 32);
+  return vec && (a.M > 64 || (a.M > 32 && (a.N + 63) / 64 >= 128)) &&
+         pg_one_set(a, gs, true, W_I4);
+}
+
 hipError_t launch_gemm(const GemmArgs& a, int wf, int epi, bool sw_half,
                        int gs, hipStream_t s) {
   // The GEMV on quantized activations for M <= 2.  At M = 3 and 4 the LDS

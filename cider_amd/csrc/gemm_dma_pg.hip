@@ -179,7 +179,8 @@ __device__ __forceinline__ bool pg_scales_tame(const GemmArgs& p, int n0, int G,
 // finite and below 2^64; real weights' scales never are, so its speed does
 // not matter, only its results.  `kbeg`, `kend`: the k range (a split-K
 // slice), `part`: fp32 partial sums [M, N] of that slice instead of y.
-template <int BM, int BN, int GS, bool SWH, int WF>
+// IL: x holds every 16 k as the even ones, then the odd ones (int4 weights).
+template <int BM, int BN, int GS, bool SWH, int WF, bool IL = false>
 __device__ __forceinline__ void pg_exact_tile(const GemmArgs& p, int m0, int n0,
                                                         int nthreads, int kbeg = 0,
                                                         int kend = -1, float* part = nullptr) {
@@ -196,9 +197,20 @@ __device__ __forceinline__ void pg_exact_tile(const GemmArgs& p, int m0, int n0,
     for (int g = kbeg / GS; g < kend / GS; ++g) {
       int32_t d = 0;
       for (int k = g * GS; k < (g + 1) * GS; k += 8) {
-        const i32x2 xv = ld8(xr + k);
+        i32x2 xv;
+        if constexpr (IL) {
+          const int8_t* const xe = xr + (k & ~15) + (k & 8) / 2;
+          xv = i32x2{*reinterpret_cast<const int32_t*>(xe),
+                     *reinterpret_cast<const int32_t*>(xe + 8)};
+        } else {
+          xv = ld8(xr + k);
+        }
         uint32_t w0, w1;
-        if constexpr (W4) {
+        if constexpr (IL) {
+          const uint32_t w = *reinterpret_cast<const uint32_t*>(wr + k / 2);
+          w0 = sext_nibbles(w & 0x0F0F0F0Fu);
+          w1 = sext_nibbles((w >> 4) & 0x0F0F0F0Fu);
+        } else if constexpr (W4) {
           unpack_w4_word(*reinterpret_cast<const uint32_t*>(wr + k / 2), w0, w1);
         } else {
           const i32x2 wv = ld8(wr + k);
@@ -811,7 +823,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_dma_pg_kernel(const 
 // A 128-k stage is two sub-steps of 64 k; in sub-step j lane l holds k in
 // [64 j + 16 (l / 16), + 16) of row l % 16 of both operands, so a group of
 // gs >= 64 never splits a sub-step (int4 weights: the 8 bytes of nibbles of
-// that k range, unpacked in the last slots of the sub-step before).  Each
+// that k range, unpacked by parity in the last slots of the sub-step before,
+// against x reordered the same way, as 16 times the weight).  Each
 // group's sum D_g lives in one int32 set; the first sub-step of group g
 // flushes each block's sum of group g-1 (in group order: the fma flush, or
 // the exact one with FL == 0) right before the MFMA that restarts the block
@@ -930,7 +943,11 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_pg16_kernel(const GemmArgs pi
                                              8 * (fq & 1));
   };
   auto unpack_w = [&](int a, i32x4 (&dst)[TN]) __attribute__((always_inline)) {
-    dst[a] = pg_unpack_w4_8((uint32_t)raw[a][0], (uint32_t)raw[a][1]);
+    // 16 times the even elements, then the odd ones (x_il = 16): 6 operations
+    // where sign extension and element order take 38
+    const uint32_t r0 = (uint32_t)raw[a][0], r1 = (uint32_t)raw[a][1];
+    dst[a] = i32x4{(int)((r0 << 4) & 0xF0F0F0F0u), (int)((r1 << 4) & 0xF0F0F0F0u),
+                   (int)(r0 & 0xF0F0F0F0u), (int)(r1 & 0xF0F0F0F0u)};
   };
   auto read_wk = [&](int slot, int j, int a, i32x4 (&dst)[TN]) __attribute__((always_inline)) {
     if constexpr (W4)
@@ -1156,7 +1173,8 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_pg16_kernel(const GemmArgs pi
     float* ssa = reinterpret_cast<float*>(smem + OUT);
     uint16_t* sbias = reinterpret_cast<uint16_t*>(ssa + BM);
     __syncthreads();  // every wave is done with the ring
-    if (tid < BM) ssa[tid] = sa_t;
+    // int4: the chain is 16 times its value (exactly: powers of two)
+    if (tid < BM) ssa[tid] = W4 ? sa_t * 0.0625f : sa_t;
     if (tid < BN) sbias[tid] = b_t;
     __syncthreads();
 #pragma unroll
@@ -1205,7 +1223,8 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_pg16_kernel(const GemmArgs pi
         const int n = n0 + wn * WN + a * 16 + 4 * fq;
         if (m < M && n < N)
           *reinterpret_cast<f32x4*>(pp + (int64_t)m * N + n) =
-              f32x4{facc[a][b][0], facc[a][b][1], facc[a][b][2], facc[a][b][3]};
+              f32x4{facc[a][b][0], facc[a][b][1], facc[a][b][2], facc[a][b][3]} *
+              (W4 ? 0.0625f : 1.0f);
       }
   };
   if constexpr (FL == 1) {
@@ -1217,7 +1236,7 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_pg16_kernel(const GemmArgs pi
         epilogue();
     } else {
       wait_vmcnt<0>();  // the prologue's DMA lands before the workgroup ends
-      pg_exact_tile<BM, BN, GS, SWH, WF>(p, m0, n0, 64 * NW, 0, KL, pp);
+      pg_exact_tile<BM, BN, GS, SWH, WF, W4>(p, m0, n0, 64 * NW, 0, KL, pp);
     }
   } else {
     body(ic<0>{});
@@ -1344,6 +1363,18 @@ PgSplit pg_split_plan(int M, int N, int K, int gs) {
 
 }  // namespace
 
+bool pg_split_one_set(int M, int N, int K, int gs) {
+  const PgSplit p = pg_split_plan(M, N, K, gs);
+  return p.S > 1 && p.one_set;
+}
+
+// launch_gemm_dma_pg's choice of the one-set kernel (its reasons there).
+bool pg_one_set(const GemmArgs& a, int gs, bool sw_half, int wf) {
+  const int64_t tiles = (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128);
+  const bool fmt = (wf == W_I8 && !sw_half) || (wf == W_I4 && sw_half && gs != 256);
+  return fmt && 2 * tiles >= 3 * (int64_t)num_cus();
+}
+
 int pg_splitk_ways(int M, int N, int K, int gs) { return pg_split_plan(M, N, K, gs).S; }
 
 size_t pg_splitk_bytes(int M, int N, int K, int gs) {
@@ -1357,6 +1388,7 @@ template <int GS, bool SWH, int WF>
 hipError_t run_pg_splitk(const GemmArgs& a, int S, float* part, hipStream_t s) {
   if constexpr (!(WF == W_I4 && GS == 256)) {
     if (pg_split_plan(a.M, a.N, a.K, GS).one_set) {
+      if (WF == W_I4 && a.x_il != 16) return hipErrorInvalidValue;
       const dim3 grid(((a.M + 127) / 128) * ((a.N + 127) / 128), S);
       gemm_dma_pg16_kernel<GS, SWH, WF, 1><<<grid, 256, 0, s>>>(a, a.K / S, part);
       return hipGetLastError();
@@ -1438,10 +1470,9 @@ hipError_t launch_gemm_dma_pg(const GemmArgs& a, int gs, bool sw_half, int wf, h
     // slower where their grid leaves a partial round; below one round of
     // 128 x 128 tiles the two-set kernel stayed ahead on some shapes (int4
     // M=512 N=12288 K=4096 gs 128: 52.3 against 55.8 us).
-    const int64_t tiles = (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128);
-    const bool fmt = (wf == W_I8 && !sw_half) || (wf == W_I4 && sw_half && gs != 256);
-    if (fmt && 2 * tiles >= 3 * (int64_t)num_cus()) {
-      const unsigned grid = (unsigned)tiles;
+    // (pg_one_set; int4 weights with x in that kernel's order only.)
+    if (pg_one_set(a, gs, sw_half, wf) && (wf == W_I8 || a.x_il == 16)) {
+      const unsigned grid = (unsigned)(((a.M + 127) / 128) * ((a.N + 127) / 128));
       if (wf == W_I4) {
         if (gs == 64)
           gemm_dma_pg16_kernel<64, true, W_I4, 1><<<grid, 256, 0, s>>>(a, 0, nullptr);

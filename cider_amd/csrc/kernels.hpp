@@ -19,19 +19,21 @@ struct GemmArgs {
   const uint16_t* bias;   // fp16 [N] or nullptr (no add)
   void* y;                // fp16 [M, N] (PC, PG) or int32 [M, N] (I32)
   int M, N, K;
-  // x holds every 32 consecutive k as the 16 even ones, then the 16 odd ones:
-  // the ping-pong kernel's order for int4 weights (w4_wants_il), no other's
-  bool x_il = false;
+  // x holds every x_il consecutive k as the even ones, then the odd ones (0: in
+  // order).  For int4 weights only, and only for the kernels that unpack nibbles
+  // by parity: 32 for the ping-pong kernel (w4_wants_il), 16 for the one-set
+  // per-group kernel (w4_pg_wants_il, pg_split_one_set).
+  int x_il = 0;
   // y (PC, PG) is bf16: the fp16 result rounded once more.  x of the GEMVs that
   // quantize it themselves is bf16, rounded to fp16 first.
   bool y_bf16 = false, x_bf16 = false;
 };
 
-// il: every 32 consecutive k of q in the order GemmArgs::x_il describes (K %
-// 32 == 0, vectorizable x and q).
+// il: the order of q's k that GemmArgs::x_il describes (K % il == 0,
+// vectorizable x and q).
 // bf: x is bf16, rounded to fp16 first.
 hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
-                           int K, hipStream_t s, bool il = false, bool bf = false);
+                           int K, hipStream_t s, int il = 0, bool bf = false);
 
 // C = epilogue(x . w^T).  wf: W_I8 / W_I4; epi: Epilogue; sw_half: PG scales
 // are fp16; gs: group size (PG only).
@@ -78,6 +80,11 @@ hipError_t launch_gemm_dma_pg(const GemmArgs& a, int gs, bool sw_half, int wf, h
 // (slices into `part`, then their sum with the epilogue into a.y).
 int pg_splitk_ways(int M, int N, int K, int gs);
 size_t pg_splitk_bytes(int M, int N, int K, int gs);
+// The same for the per-group int4 GEMM of a (with no split), and whether the
+// slices of a split run the one-set kernel.
+bool w4_pg_wants_il(const GemmArgs& a, int gs);
+bool pg_split_one_set(int M, int N, int K, int gs);
+bool pg_one_set(const GemmArgs& a, int gs, bool sw_half, int wf);
 hipError_t launch_gemm_pg_splitk(const GemmArgs& a, int gs, bool sw_half, int wf, int S,
                                  float* part, hipStream_t s);
 

@@ -21,17 +21,20 @@ namespace cider {
 
 namespace {
 
-// Vector e (8 elements) of a quantized row.  il: every 32 consecutive elements
-// are stored as the 16 of even index, then the 16 of odd index (K % 32 == 0),
-// the order the ping-pong GEMM takes for int4 weights (gemm_pp.hip).
+// Vector e (8 elements) of a quantized row.  il = 32 or 16: every il consecutive
+// elements are stored as those of even index, then those of odd index (K % il
+// == 0), the orders the int4 GEMMs take (gemm_pp.hip 32, gemm_dma_pg.hip 16).
 __device__ __forceinline__ void store_q8(int8_t* qr, int e, i32x2 v, int il) {
   if (!il) {
     *reinterpret_cast<i32x2*>(qr + 8 * e) = v;
     return;
   }
-  int32_t* const d = reinterpret_cast<int32_t*>(qr + 32 * (e >> 2) + 4 * (e & 3));
-  d[0] = (int32_t)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x06040200u);
-  d[4] = (int32_t)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x07050301u);
+  const int m = il / 8 - 1, half = il / 2;  // vectors per block - 1, bytes of the evens
+  int8_t* const d = qr + 8 * (e & ~m) + 4 * (e & m);
+  *reinterpret_cast<int32_t*>(d) =
+      (int32_t)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x06040200u);
+  *reinterpret_cast<int32_t*>(d + half) =
+      (int32_t)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x07050301u);
 }
 
 }  // namespace
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(256) void quantize_scalar_kernel(
 }
 
 hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
-                           int K, hipStream_t s, bool il, bool bf) {
+                           int K, hipStream_t s, int il, bool bf) {
   const dim3 grid((M + 3) / 4), block(256);
   const bool vec = (K % 8 == 0) && (((uintptr_t)x & 15) == 0) &&
                    (((uintptr_t)q & 7) == 0);

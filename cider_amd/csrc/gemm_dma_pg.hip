@@ -37,7 +37,7 @@
 //     4 waves (gs 128 at two workgroups per CU, gs 64 at M <= 64), and 64 x 64
 //     tiles of four 32 x 32 waves where those would leave most CUs idle (and
 //     for the split-K slices).  gemm_dma_pg16_kernel below (one group set,
-//     waves of 64 x 64) takes the grids of 512 tiles and more.
+//     waves of 64 x 64) takes the grids whose 128 x 128 tiles outnumber the CUs.
 //   * Group accumulators: two int32 sets alternate by group.  A group's first
 //     MFMA takes C = 0 (an inline constant), so starting a group costs
 //     nothing.  While group g accumulates, group g-1 is flushed into the fp32
@@ -1368,11 +1368,16 @@ bool pg_split_one_set(int M, int N, int K, int gs) {
   return p.S > 1 && p.one_set;
 }
 
-// launch_gemm_dma_pg's choice of the one-set kernel (its reasons there).
+// launch_gemm_dma_pg's choice of the one-set kernel: more tiles than CUs, so
+// that some run two workgroups.  (From 384 tiles before; at 288 and 352 tiles the
+// two-set kernel took, one-set after: M=700 N=6144 K=4096 int8 gs 64 62.8 -> 54.3
+// us, gs 128 49.4 -> 43.9, int4 gs 64 86.7 -> 62.1, gs 128 57.6 -> 49.3; M=1334
+// N=4096 K=12288 162 -> 144, 129 -> 114, 233 -> 163, 152 -> 126 us.  At 256 tiles
+// and fewer, one workgroup per CU, it is level or behind.)
 bool pg_one_set(const GemmArgs& a, int gs, bool sw_half, int wf) {
   const int64_t tiles = (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128);
   const bool fmt = (wf == W_I8 && !sw_half) || (wf == W_I4 && sw_half && gs != 256);
-  return fmt && 2 * tiles >= 3 * (int64_t)num_cus();
+  return fmt && tiles > (int64_t)num_cus();
 }
 
 int pg_splitk_ways(int M, int N, int K, int gs) { return pg_split_plan(M, N, K, gs).S; }
@@ -1454,10 +1459,8 @@ hipError_t launch_gemm_dma_pg(const GemmArgs& a, int gs, bool sw_half, int wf, h
   {
     // The one-set kernel: 128 x 128 tiles of four 64 x 64 waves, two
     // workgroups per CU, for int8 weights with fp32 scales and int4 weights
-    // with fp16 scales, once its tiles fill 384 of the 512 workgroup slots
-    // (the fma chain of the kernels below for fp32 scales; from 384 instead
-    // of 512: W4A8 gs 64 M=512 N=12288 K=4096 87.8 -> 71.6 us, gs 128 60.2
-    // -> 58.8 us).  Against the two-set
+    // with fp16 scales, where its tiles outnumber the CUs (the fma chain of
+    // the kernels below for fp32 scales).  Against the two-set
     // kernel's tiles, measured on its 32 x 32 x 32 form (the 16 x 16 x 64
     // form it runs now is 3-6 % faster again; weights from HBM where they
     // exceed the MALL): M=4096 N=10240 K=2560 gs

@@ -172,6 +172,23 @@ __device__ __forceinline__ i32x2 ld8(const void* p) {
   return *reinterpret_cast<const i32x2*>(p);
 }
 
+// Stores the first min(left, all) elements of a vector of consecutive outputs
+// of one row.  Rows of a ragged width start at any element, so the whole
+// vector's store asks for the element's alignment only (one instruction, as
+// for an aligned one); left <= 0 stores nothing.
+template <typename T, typename V>
+__device__ __forceinline__ void store_row(T* p, int left, V v) {
+  constexpr int n = sizeof(V) / sizeof(T);
+  typedef V __attribute__((aligned(alignof(T)))) VU;
+  if (left >= n) {
+    *reinterpret_cast<VU*>(p) = v;
+  } else {
+#pragma unroll
+    for (int i = 0; i < n - 1; ++i)
+      if (i < left) p[i] = reinterpret_cast<const T*>(&v)[i];
+  }
+}
+
 // Non-temporal loads (the nt cache policy) for weight streams that every
 // launch reads once: a single-launch read of 26 MB in the MV's layout ran
 // 5.78 against 5.99 us with plain loads, the M == 1 MV 6.44 -> 6.00 us.

@@ -390,8 +390,13 @@ hipError_t launch_gemm(const GemmArgs& a, int wf, int epi, bool sw_half,
   // per-lane offset of up to 256 rows * K bytes; longer rows take the
   // register-staged kernel, whose addresses are 64-bit throughout.
   const bool off32 = (int64_t)a.K * 256 < ((int64_t)1 << 32);
-  const bool dma = epi != EPI_PG && (wf == W_I8 || epi == EPI_PC) && vec && a.K % 128 == 0 &&
-                   a.N % 8 == 0 && off32;
+  // Per-channel and int32: any N, and K of whole 16-byte chunks.  Whole int8
+  // linears at N=4095 K=4096 / N=4096 K=4160, register-staged against LDS-DMA:
+  // M=96 107 / 90 -> 15 us, M=400 123 / 103 -> 24, M=1500 127 / 106 -> 39 / 41
+  // (N=509 K=5952, M=96: 147 -> 19); int4 M=1500 123 / 104 -> 61 / 63.
+  const bool dma = epi != EPI_PG && (wf == W_I8 || epi == EPI_PC) &&
+                   a.K % (wf == W_I4 ? 32 : 16) == 0 && a.K >= 128 && aligned16(a.x) &&
+                   aligned16(a.w) && off32;
   const bool dma_pg = epi == EPI_PG && (gs == 64 || gs == 128 || (gs == 256 && wf == W_I8)) &&
                       vec && a.K % 128 == 0 && a.K % gs == 0 && a.N % 8 == 0 && off32;
   if (a.M <= 64) {

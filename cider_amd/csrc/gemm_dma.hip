@@ -1,7 +1,7 @@
 // Tiled int8 GEMM for shapes with few rows or columns, where the 256-column
 // tiles of the ping-pong kernel (gemm_pp.hip) would leave CUs idle: int8
 // weights (int32 and per-channel epilogues) and int4 weights (per-channel, the
-// reference W4A8) with K % 128 == 0 and N % 8 == 0.  Operands stream global ->
+// reference W4A8) with K >= 128 of whole 16-byte chunks and any N.  Operands stream global ->
 // LDS by gfx950's 16-byte LDS-DMA loads through a ring of k-stages, the MFMAs
 // are v_mfma_i32_32x32x32_i8, and the fp16 tile is staged through LDS so the
 // output is written in whole rows.
@@ -66,7 +66,9 @@
 //     on k 64p + 32h + [0, 32), identically for both operands, so the int32
 //     dot products are exact.
 //   * Rows past M or N are loaded from the last valid row (their results are
-//     never stored); K % 128 == 0 is required, so there is no K tail.
+//     never stored).  Where K is no multiple of 128 the last stage is the
+//     row's last 128 k, and the x chunks that it shares with the stage before
+//     are zeroed: no load is masked and the loop does not change.
 #include "common.hpp"
 #include "dma_common.hpp"
 #include "kernels.hpp"
@@ -163,14 +165,21 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
   }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)smem);
+  // The last stage ends with K: where K is no multiple of BK it starts inside
+  // the stage before, and the X chunks that it shares with that stage are
+  // zeroed as they are multiplied (k_skip k values, 0 for whole stages).
+  const int klen = kloop > 0 ? kloop : K;  // this tile's K (a split-K slice: kloop of K)
+  const int nk = (klen + BK - 1) / BK;     // k-stages
+  const int xlast = klen - BK, wlast = W4 ? xlast / 2 : xlast;
+  const int k_skip = nk * BK - klen;
   // DMA instruction d (0 .. PS-1) of this wave for stage st into ring slot
   // `slot`: W rows first, then X rows.
   auto dma_one = [&](int st, int slot, int d) {
     const uint32_t sb = lds0 + (uint32_t)(slot * STAGE);
     if (d < WI)
-      dma16s(wbase + (int64_t)st * WB, woff[d < WI ? d : 0], sb + (wave * WI + d) * 1024);
+      dma16s(wbase + min(st * WB, wlast), woff[d < WI ? d : 0], sb + (wave * WI + d) * 1024);
     else
-      dma16s(xbase + (int64_t)st * BK, xoff[d >= WI ? d - WI : 0],
+      dma16s(xbase + min(st * BK, xlast), xoff[d >= WI ? d - WI : 0],
              sb + W_BYTES + (wave * XI + d - WI) * 1024);
   };
 
@@ -279,7 +288,6 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
     }
   };
 
-  const int nk = (kloop > 0 ? kloop : K) / BK;  // k-stages (a split-K slice: kloop of K)
   i32x4 wf[2][TN], xf[2][TM];
   // Prologue: stages 0 .. NS-2 into slots 0 .. NS-2, and part 0 of stage
   // NS-1 into slot NS-1; stage 0's first sub-steps issue its other parts as
@@ -313,11 +321,18 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
   // slot of stage kt, which receives stage kt+NS from that sub-step on.  The
   // first DS-1 sub-steps issue the rest of the loads the previous stage began
   // (in the first stage, the rest of the prologue's stage NS-1).
+  auto drop_shared = [&](int j, i32x4 (&x)[TM]) {
+    if (16 * x_chunk(j) < k_skip) {
+#pragma unroll
+      for (int b = 0; b < TM; ++b) x[b] = i32x4{0, 0, 0, 0};
+    }
+  };
   auto stage_body = [&](int kt, auto lastc) {
     constexpr bool LAST = decltype(lastc)::value != 0;
     const int sl = kt % NS;
     const int pdst = min(kt - 1 + NS, nk - 1), psl = (kt + NS - 1) % NS;
 #define DMA_SUB(J)                                                                          \
+  if constexpr (LAST) drop_shared((J), xf[(J) & 1]);                                        \
   if constexpr ((J) < SUBS - 1) {                                                           \
     step(icst<(J) + 1>{}, icst<1>{}, icst<((J) + 1 < DS) ? (J) + 2 : 0>{},                   \
          wf[(J) & 1], xf[(J) & 1], sl, wf[((J) + 1) & 1], xf[((J) + 1) & 1], pdst, psl);     \
@@ -363,10 +378,9 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int n = n0 + wn * WN + a * 32 + 8 * g + 4 * h;
-          if (n < N)
-            *reinterpret_cast<i32x4*>(reinterpret_cast<int32_t*>(p.y) + (int64_t)m * N + n) =
-                i32x4{acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2],
-                      acc[a][b][4 * g + 3]};
+          store_row(reinterpret_cast<int32_t*>(p.y) + (int64_t)m * N + n, N - n,
+                    i32x4{acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2],
+                          acc[a][b][4 * g + 3]});
         }
     }
   } else {
@@ -458,9 +472,9 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
 #pragma unroll 4
     for (int rr = wave * RPS + lane / LPR; rr < BM; rr += NWV * RPS) {
       const int m = m0 + rr;
-      if (m < M && n < N)
-        *reinterpret_cast<i32x4*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + n) =
-            *reinterpret_cast<const i32x4*>(smem + rr * C::OUT_LD + cl * 2);
+      if (m < M)  // n may lie past N
+        store_row(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + n, N - n,
+                  *reinterpret_cast<const i32x4*>(smem + rr * C::OUT_LD + cl * 2));
     }
   }
 }
@@ -534,7 +548,7 @@ bool pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N], const 
   *best = nullptr;
   for (const TileCost& c : cands) {
     if (c.bn == 256 && (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus) continue;
-    const double cost = tile_cost(c, a.M, a.N, a.K / 128, cus);
+    const double cost = tile_cost(c, a.M, a.N, (a.K + 127) / 128, cus);
     if (cost < best_cost) {
       best_cost = cost;
       *best = &c;
@@ -691,7 +705,7 @@ bool w4_wants_il(const GemmArgs& a) {
 }
 
 // Eligible: EPI_I32 or EPI_PC with int8 weights, EPI_PC with int4 weights;
-// K % 128 == 0, N % 8 == 0, 16-byte aligned operands (launch_gemm checks).
+// K >= 128, K % 16 == 0 (int4: 32), x and w 16-byte aligned (launch_gemm checks).
 hipError_t launch_gemm_dma(const GemmArgs& a, int epi, int wf, hipStream_t s) {
   if (wf == W_I4) return launch_i4(a, s);
   if (epi == EPI_I32) return launch_i8<EPI_I32>(a, s);

@@ -471,11 +471,11 @@ double plan_cost(const PpCost& c, const PpPlan& pl, int nk, int cus) {
 }  // namespace
 
 bool pp_supported(const GemmArgs& a, int epi, int wf) {
-  // 32-bit element offsets within a tile of the output; the DMA of the bias
-  // moves 16 bytes per lane; 16 times the int4 weights' sums fit int32
+  // 32-bit element offsets within a tile of the output; the DMA of the scales
+  // and the bias and the stores move 16 bytes per lane; 16 times the int4 weights' sums fit int32
   return a.M >= 64 && a.N >= 256 && a.N % 8 == 0 && a.N <= (1 << 22) && a.K >= 512 &&
          a.K % 128 == 0 && (wf == W_I8 ? epi != EPI_PG : epi == EPI_PC && a.K < (1 << 17)) &&
-         (a.bias == nullptr || ((uintptr_t)a.bias & 15) == 0);
+         (((uintptr_t)a.y | (uintptr_t)a.sw | (uintptr_t)a.bias) & 15) == 0;
 }
 
 // The cheapest of: one tile height throughout; the rows below the last whole

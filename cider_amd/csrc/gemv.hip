@@ -59,10 +59,15 @@ __device__ __forceinline__ float dot8(uint32_t w0, uint32_t w1, uint32_t x0, uin
 
 }  // namespace
 
-// PG: per-group scales; VEC: K % 256 == 0 and 16-byte aligned w (full blocks,
-// vector loads); otherwise the weight tail is loaded bytewise with bounds.
+// PG: per-group scales; VEC: how the weights load.  kFull: K % 256 == 0 and
+// 16-byte aligned w and x.  kChunks: K % 16 == 0, 16-byte aligned w, x in LDS:
+// the same loads, clamped to the row's last chunk in a part-filled last block,
+// where the staged x is zero (N=4096 K=4160: 32.8 us bytewise, 10.2 so).  kBytes:
+// anything else, bytewise with bounds.
 // XLDS: x staged in LDS (K <= kMaxLdsK); otherwise read from global.
-template <bool PG, bool VEC, bool XLDS, int U>
+enum MvLoad { kBytes, kChunks, kFull };
+
+template <bool PG, int VEC, bool XLDS, int U>
 __global__ __launch_bounds__(256) void mv_kernel(
     const uint16_t* __restrict__ x, const int8_t* __restrict__ w,
     const float* __restrict__ sw, const uint16_t* __restrict__ bias,
@@ -86,7 +91,11 @@ __global__ __launch_bounds__(256) void mv_kernel(
 
   // weight slice of block b for this lane (16 bytes at 256 b + 16 j)
   auto load_w = [&](int b, i32x4& v) {
-    if (VEC) {
+    if constexpr (VEC == kChunks) {
+      v = ld16_nt(wr + min(min(b, nb - 1) * 256 + 16 * j, K - 16));
+      return;
+    }
+    if constexpr (VEC == kFull) {
       // branch-free: a block index past the end re-reads the last block (its
       // value is never consumed), so every load is issued unconditionally and
       // the compiler can count outstanding loads exactly
@@ -115,7 +124,7 @@ __global__ __launch_bounds__(256) void mv_kernel(
   const int nchunk = kp / 8;
   auto load_x = [&](int e) -> i32x4 {
     const int k = 8 * e;
-    if (VEC || (k + 8 <= K && (((uintptr_t)(x + k) & 15) == 0))) return ld16(x + k);
+    if (VEC == kFull || (k + 8 <= K && (((uintptr_t)(x + k) & 15) == 0))) return ld16(x + k);
     uint32_t t[4] = {0u, 0u, 0u, 0u};
     for (int i = 0; i < 8; ++i)
       if (k + i < K) t[i >> 1] |= (uint32_t)x[k + i] << (16 * (i & 1));
@@ -131,7 +140,7 @@ __global__ __launch_bounds__(256) void mv_kernel(
 #pragma unroll
     for (int q = 0; q < XR; ++q) {
       const int e = tid + q * nthr;
-      if (VEC)
+      if (VEC == kFull)
         xr[q] = ld16(x + 8 * min(e, nchunk - 1));  // unconditional, stored only if e < nchunk
       else if (e < nchunk)
         xr[q] = load_x(e);
@@ -149,7 +158,7 @@ __global__ __launch_bounds__(256) void mv_kernel(
   for (int u = 0; u < U; ++u) load_w(u, wa[u]);
   // VEC loads are unconditional (a branch here lets the compiler sink them
   // past the staging barrier); the scalar path loads only what exists
-  if (VEC || U < nb) {
+  if (VEC != kBytes || U < nb) {
 #pragma unroll
     for (int u = 0; u < U; ++u) load_w(U + u, wb[u]);
   }
@@ -434,19 +443,26 @@ constexpr int kMaxLdsK = 32768;  // x staged in LDS up to 64 KB
 
 template <bool PG, bool XLDS, int U>
 hipError_t run_mv(const uint16_t* x, const int8_t* w, const float* sw, const uint16_t* bias,
-                  uint16_t* y, int N, int K, int gs, bool vec, int rows, size_t lds,
+                  uint16_t* y, int N, int K, int gs, int vec, int rows, size_t lds,
                   hipStream_t s) {
   const dim3 grid((N + rows - 1) / rows), block(rows * kLanesPerRow);
-  if (vec)
-    mv_kernel<PG, true, XLDS, U><<<grid, block, lds, s>>>(x, w, sw, bias, y, N, K, gs, rows);
-  else
-    mv_kernel<PG, false, XLDS, U><<<grid, block, lds, s>>>(x, w, sw, bias, y, N, K, gs, rows);
+  if (vec == kFull) {
+    mv_kernel<PG, kFull, XLDS, U><<<grid, block, lds, s>>>(x, w, sw, bias, y, N, K, gs, rows);
+    return hipGetLastError();
+  }
+  if constexpr (XLDS) {
+    if (vec == kChunks) {
+      mv_kernel<PG, kChunks, XLDS, U><<<grid, block, lds, s>>>(x, w, sw, bias, y, N, K, gs, rows);
+      return hipGetLastError();
+    }
+  }
+  mv_kernel<PG, kBytes, XLDS, U><<<grid, block, lds, s>>>(x, w, sw, bias, y, N, K, gs, rows);
   return hipGetLastError();
 }
 
 template <bool PG, bool XLDS>
 hipError_t pick_u(const uint16_t* x, const int8_t* w, const float* sw, const uint16_t* bias,
-                  uint16_t* y, int N, int K, int gs, bool vec, int rows, size_t lds,
+                  uint16_t* y, int N, int K, int gs, int vec, int rows, size_t lds,
                   hipStream_t s) {
   // the prologue requests 2U blocks: U = ceil(nb / 2) up to 8 puts the whole
   // row of a short-K shape in flight at once with no redundant loads
@@ -557,7 +573,10 @@ hipError_t launch_mv_lanes(const uint16_t* x, const int8_t* w, const float* sw,
   const int G = gs > 0 ? K / gs : 0;
   const size_t lds = (xlds ? (size_t)nb * 256 * 2 : 0) + (size_t)G * rows * sizeof(float);
   if (lds > 160 * 1024) return hipErrorInvalidValue;
-  const bool vec = (K % 256 == 0) && (((uintptr_t)w & 15) == 0) && (((uintptr_t)x & 15) == 0);
+  const bool wal = ((uintptr_t)w & 15) == 0;
+  const int vec = K % 256 == 0 && wal && ((uintptr_t)x & 15) == 0 ? kFull
+                  : K % 16 == 0 && K > 0 && wal && xlds           ? kChunks
+                                                                  : kBytes;
   if (gs > 0) {
     if (xlds) return pick_u<true, true>(x, w, sw, bias, y, N, K, gs, vec, rows, lds, s);
     return pick_u<true, false>(x, w, sw, bias, y, N, K, gs, vec, rows, lds, s);

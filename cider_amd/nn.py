@@ -195,7 +195,9 @@ class W4A8Linear(torch.nn.Module):
         stream waits for that event there and marks the copy as used there, so
         the caching allocator keeps the memory until that stream's work is done
         even after a later repack replaces the copy.  On the stream that made
-        the copy, and whose pool it is from, both hold by stream order."""
+        the copy, and whose pool it is from, both hold by stream order, but not
+        where it was made under capture: nothing has run there yet, and the
+        wait is what refuses an eager call."""
         w = self.packed_weight
         use = torch.cuda.current_stream(w.device)
         sig = (w._version, w.data_ptr(), tuple(w.shape), w.device)
@@ -203,8 +205,10 @@ class W4A8Linear(torch.nn.Module):
             out = ops.repack_w4_ref(w)
             done = torch.cuda.Event()
             done.record(use)
-            self._w4_nk, self._w4_sig, self._w4_done = out, sig, done
-            self._w4_stream = use.cuda_stream
+            self._w4_stream = (None if torch.cuda.is_current_stream_capturing()
+                               else use.cuda_stream)
+            # sig last: it is what lets another thread use the rest
+            self._w4_nk, self._w4_done, self._w4_sig = out, done, sig
             return out
         if use.cuda_stream == self._w4_stream:
             return self._w4_nk

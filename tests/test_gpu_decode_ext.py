@@ -99,3 +99,27 @@ def test_attn_decode_rope(H, KV, n, slot, row):
     assert torch.equal(bits(k1), bits(k2)) and torch.equal(bits(v1), bits(v2))
     assert torch.equal(out.isnan(), e.isnan())
     assert torch.equal(bits(out)[~e.isnan()], bits(e)[~e.isnan()])
+
+
+@pytest.mark.parametrize("sub", ["keys", "queries", "values"])
+def test_attn_decode_subnormal(sub):
+    # fp16 subnormals are operands as good as any: flushed, every score (or the
+    # output) would be 0.  Bound: 128 products summed in fp32 (2^-24 each, scores
+    # up to ~8) and one fp16 rounding of the result (2^-11; subnormal: 2^-25).
+    T, D, n, H = 256, 128, 200, 4
+    g = torch.Generator(device=DEV).manual_seed(3)
+
+    def rand(*s):
+        return torch.randn(*s, device=DEV, generator=g)
+
+    tiny = 2.0 ** -17
+    q = (rand(H, D) * (tiny if sub == "queries" else 2.0 ** 12)).half()
+    k = (rand(1, T, D) * (tiny if sub == "keys" else 2.0 ** 12)).half()
+    v = (rand(1, T, D) * (tiny if sub == "values" else 1.0)).half()
+    scale = {"values": 2.0 ** -27}.get(sub, 1.0)
+    nv = torch.tensor([n], dtype=torch.int64, device=DEV)
+    out = F.attn_decode(q, k, v, nv, scale).double().view(H, D).cpu()
+    s = q.double().cpu() @ k[0, :n].double().cpu().T * scale
+    e = torch.softmax(s, -1) @ v[0, :n].double().cpu()
+    bound = 1e-3 * e.abs() + (2.0 ** -24 if sub == "values" else 2.0 ** -13)
+    assert ((out - e).abs() <= bound).all()

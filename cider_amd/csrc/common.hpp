@@ -176,8 +176,13 @@ __device__ __forceinline__ i32x2 ld8(const void* p) {
 // of one row.  Rows of a ragged width start at any element, so the whole
 // vector's store asks for the element's alignment only (one instruction, as
 // for an aligned one); left <= 0 stores nothing.
-template <typename T, typename V>
+// RAG = false: rows of whole, aligned vectors, so left is never a part of one.
+template <bool RAG = true, typename T, typename V>
 __device__ __forceinline__ void store_row(T* p, int left, V v) {
+  if constexpr (!RAG) {
+    if (left > 0) *reinterpret_cast<V*>(p) = v;
+    return;
+  }
   constexpr int n = sizeof(V) / sizeof(T);
   typedef V __attribute__((aligned(alignof(T)))) VU;
   if (left >= n) {

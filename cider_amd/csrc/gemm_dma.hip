@@ -122,7 +122,13 @@ using icst = std::integral_constant<int, V>;
 // One BM x BN output tile over the whole K.  smem: DmaCfg::SMEM bytes of LDS.
 // WF = W_I8: weights int8 [N, K]; W_I4: packed int4 [N, K/2] (element k in
 // byte k/2, low nibble first, two's complement), unpacked in registers.
-template <int BM, int BN, int BK, int EPI, int WF = W_I8, int NWV = 4>
+// RAG: K is no multiple of BK, N none of 8, or y not 16-byte aligned.  A
+// template argument, not a test: the clamped addresses, the zeroing and the
+// cut-off stores cost whole shapes about 1 % (M=512 N=4096 K=2048 linear 13.22
+// -> 13.05 us without them; Qwen3-VL-2B-shaped chunk layer of 300 tokens 100.98
+// -> 99.96, of 120 81.09 -> 80.46); ragged ones are level (M=500 N=4095 K=4160
+// 21.7 us).
+template <int BM, int BN, int BK, int EPI, int WF = W_I8, int NWV = 4, bool RAG = false>
 __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const int n0,
                                          int8_t* __restrict__ smem, const int kloop = 0) {
   static_assert((BM == 64 || BM == 128) && (BN == 64 || BN == 128 || BN == 256), "tile shape");
@@ -169,7 +175,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
   // the stage before, and the X chunks that it shares with that stage are
   // zeroed as they are multiplied (k_skip k values, 0 for whole stages).
   const int klen = kloop > 0 ? kloop : K;  // this tile's K (a split-K slice: kloop of K)
-  const int nk = (klen + BK - 1) / BK;     // k-stages
+  const int nk = (klen + (RAG ? BK - 1 : 0)) / BK;  // k-stages
   const int xlast = klen - BK, wlast = W4 ? xlast / 2 : xlast;
   const int k_skip = nk * BK - klen;
   // DMA instruction d (0 .. PS-1) of this wave for stage st into ring slot
@@ -177,9 +183,9 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
   auto dma_one = [&](int st, int slot, int d) {
     const uint32_t sb = lds0 + (uint32_t)(slot * STAGE);
     if (d < WI)
-      dma16s(wbase + min(st * WB, wlast), woff[d < WI ? d : 0], sb + (wave * WI + d) * 1024);
+      dma16s(wbase + (RAG ? min(st * WB, wlast) : st * WB), woff[d < WI ? d : 0], sb + (wave * WI + d) * 1024);
     else
-      dma16s(xbase + min(st * BK, xlast), xoff[d >= WI ? d - WI : 0],
+      dma16s(xbase + (RAG ? min(st * BK, xlast) : st * BK), xoff[d >= WI ? d - WI : 0],
              sb + W_BYTES + (wave * XI + d - WI) * 1024);
   };
 
@@ -332,7 +338,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
     const int sl = kt % NS;
     const int pdst = min(kt - 1 + NS, nk - 1), psl = (kt + NS - 1) % NS;
 #define DMA_SUB(J)                                                                          \
-  if constexpr (LAST) drop_shared((J), xf[(J) & 1]);                                        \
+  if constexpr (LAST && RAG) drop_shared((J), xf[(J) & 1]);                                        \
   if constexpr ((J) < SUBS - 1) {                                                           \
     step(icst<(J) + 1>{}, icst<1>{}, icst<((J) + 1 < DS) ? (J) + 2 : 0>{},                   \
          wf[(J) & 1], xf[(J) & 1], sl, wf[((J) + 1) & 1], xf[((J) + 1) & 1], pdst, psl);     \
@@ -378,7 +384,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int n = n0 + wn * WN + a * 32 + 8 * g + 4 * h;
-          store_row(reinterpret_cast<int32_t*>(p.y) + (int64_t)m * N + n, N - n,
+          store_row<RAG>(reinterpret_cast<int32_t*>(p.y) + (int64_t)m * N + n, N - n,
                     i32x4{acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2],
                           acc[a][b][4 * g + 3]});
         }
@@ -473,19 +479,19 @@ __device__ __forceinline__ void dma_tile(const GemmArgs& p, const int m0, const 
     for (int rr = wave * RPS + lane / LPR; rr < BM; rr += NWV * RPS) {
       const int m = m0 + rr;
       if (m < M)  // n may lie past N
-        store_row(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + n, N - n,
+        store_row<RAG>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + n, N - n,
                   *reinterpret_cast<const i32x4*>(smem + rr * C::OUT_LD + cl * 2));
     }
   }
 }
 
 // Uniform grid: one BM x BN tile per workgroup.
-template <int BM, int BN, int BK, int EPI, int WF, int NWV = 4>
+template <int BM, int BN, int BK, int EPI, int WF, int NWV, bool RAG>
 __global__ __launch_bounds__(64 * NWV, 1) void gemm_dma_kernel(const GemmArgs p) {
   __shared__ __attribute__((aligned(1024))) int8_t smem[DmaCfg<BM, BN, BK, WF, NWV>::SMEM];
   int m0, n0;
   tile_coords<BM, BN>(xcd_remap(blockIdx.x, gridDim.x), p.M, 0, p.N, m0, n0);
-  dma_tile<BM, BN, BK, EPI, WF, NWV>(p, m0, n0, smem);
+  dma_tile<BM, BN, BK, EPI, WF, NWV, RAG>(p, m0, n0, smem);
 }
 
 namespace {
@@ -495,7 +501,11 @@ template <int BM, int BN, int BK, int EPI, int WF = W_I8>
 hipError_t run_dma(const GemmArgs& a, hipStream_t s) {
   constexpr int NWV = BN == 256 ? 8 : 4;
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  gemm_dma_kernel<BM, BN, BK, EPI, WF, NWV><<<tiles, 64 * NWV, 0, s>>>(a);
+  // whole rows are stored 16 bytes aligned, ragged ones at element alignment
+  if (a.K % BK == 0 && a.N % 8 == 0 && ((uintptr_t)a.y & 15) == 0)
+    gemm_dma_kernel<BM, BN, BK, EPI, WF, NWV, false><<<tiles, 64 * NWV, 0, s>>>(a);
+  else
+    gemm_dma_kernel<BM, BN, BK, EPI, WF, NWV, true><<<tiles, 64 * NWV, 0, s>>>(a);
   return hipGetLastError();
 }
 

@@ -123,3 +123,47 @@ def test_attn_decode_subnormal(sub):
     e = torch.softmax(s, -1) @ v[0, :n].double().cpu()
     bound = 1e-3 * e.abs() + (2.0 ** -24 if sub == "values" else 2.0 ** -13)
     assert ((out - e).abs() <= bound).all()
+
+
+# The decode attention's partial results of a chunk (its largest score, and P.V
+# before the division) against the stated arithmetic, bit for bit: fp32, every
+# product and every sum rounded once, ascending order inside and over the slices
+# of 8.  The probabilities are read from a first call whose values are one-hot.
+# n: one position, a part of a slice, whole slices, a whole chunk.
+@pytest.mark.parametrize("H,KV", [(1, 1), (2, 1), (4, 1), (8, 1)])
+@pytest.mark.parametrize("n", [1, 5, 100, 104, 128])
+def test_attn_decode_rounding(H, KV, n):
+    np = pytest.importorskip("numpy")
+    D = T = 128
+    g = torch.Generator(device=DEV).manual_seed(H + n)
+    q = torch.randn(H, D, device=DEV, generator=g).half()
+    k = torch.randn(KV, T, D, device=DEV, generator=g).half()
+    v = torch.randn(KV, T, D, device=DEV, generator=g).half()
+    nv = torch.tensor([n], dtype=torch.int64, device=DEV)
+    scale = np.float32(0.0883883461356163)
+    G = min(H, 4)
+
+    def partials(values):
+        ws = F.attn_decode_workspace(H, T, DEV)
+        F.attn_decode(q, k, values, nv, float(scale), ws=ws)
+        f = ws.view(torch.float32)[:H * (D + 2)].cpu().numpy().reshape(H // G, G * (D + 2))
+        return f[:, :G * D].reshape(H, D), f[:, G * D:G * D + G].reshape(H)
+
+    def summed(terms):  # [..., 128, x]: slices of 8 in order, then their sums in order
+        t = terms.reshape(*terms.shape[:-2], 16, 8, terms.shape[-1])
+        part = np.zeros(t.shape[:-2] + t.shape[-1:], np.float32)
+        for i in range(8):
+            part = part + t[..., i, :]
+        out = np.zeros(part.shape[:-2] + part.shape[-1:], np.float32)
+        for i in range(16):
+            out = out + part[..., i, :]
+        return out
+
+    qf, kf, vf = (t.float().cpu().numpy() for t in (q, k[0], v[0]))
+    scores = summed(qf[:, :, None] * kf.T[None]) * scale  # [H, T]
+    p, m = partials(torch.eye(T, device=DEV).half()[None].contiguous())
+    assert np.array_equal(m, scores[:, :n].max(1))
+    assert (p[:, n:] == 0).all()
+    o, _ = partials(v)
+    expected = summed(p[:, :, None] * vf[None])  # positions past n: p is 0
+    assert np.array_equal(o, expected)

@@ -1,0 +1,24 @@
+"""The Python extension of the linears (csrc/fast_linear.cpp) as a library."""
+
+import os
+import struct
+
+import pytest
+
+from cider_amd import _lib
+
+PT_TLS = 7
+
+
+def test_no_thread_local_storage():
+    # thread-local storage in a library loaded late slows every other library's
+    # thread-local access (see the Makefile's -DNDEBUG)
+    if not os.path.exists(_lib.FAST_PATH):
+        pytest.skip("extension not built")
+    with open(_lib.FAST_PATH, "rb") as f:
+        elf = f.read()
+    assert elf[:5] == b"\x7fELF\x02"
+    phoff, = struct.unpack_from("<Q", elf, 32)
+    size, count = struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, phoff + i * size)[0] for i in range(count)]
+    assert PT_TLS not in kinds

@@ -73,11 +73,15 @@ class CiderLinear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         b = self._buffers
-        op = _lib.CIDER_OP_PERGROUP if self.group_size else _lib.CIDER_OP_PERCHANNEL
-        y = ops._fast(op, x, b.get("w_int8"), b.get("scale_w"), b.get("bias"),
-                      self.group_size, None, True)
-        if y is not None:
-            return y
+        bias = b.get("bias")
+        if bias is None:
+            bias = self.bias  # a Parameter in the buffer's place
+        if bias is not None:  # None would be the native call's "no bias"
+            op = _lib.CIDER_OP_PERGROUP if self.group_size else _lib.CIDER_OP_PERCHANNEL
+            y = ops._fast(op, x, b.get("w_int8"), b.get("scale_w"), bias, self.group_size, None,
+                          True)
+            if y is not None:
+                return y
         orig_shape = x.shape
         x2 = x.reshape(-1, self._in_features)
         if self._mode == "per_channel":

@@ -183,15 +183,23 @@ class W4A8Linear(torch.nn.Module):
         self.register_buffer("scale", torch.as_tensor(scale, dtype=torch.float32, device=dev)
                              .contiguous())
         self._K = K
-        # library layout, made on first use on the GPU; valid for the
-        # (version, address, shape, device) of packed_weight it was made from.
-        # _w4_done: event recorded after the repack on the stream that made it
-        self._w4_nk = None
-        self._w4_sig = None
-        self._w4_done = None
 
-    # the stream (handle) the copy was made on
-    _w4_stream = None
+    # (signature, copy, event, stream) of the copy in the library layout, or None.
+    # Made on first use on the GPU; the signature is the (version, address, shape,
+    # device) of packed_weight that it was made from, the event recorded after the
+    # repack on the stream that made it, the stream that stream's handle where
+    # stream order alone serves (see _packed_nk).  One attribute, so that a
+    # thread that reads it while another repacks has one copy's four parts.
+    _w4 = None
+
+    @property
+    def _w4_done(self):
+        """The event of the copy in use; set to None, it drops the copy."""
+        return self._w4[2] if self._w4 is not None else None
+
+    @_w4_done.setter
+    def _w4_done(self, none):
+        self._w4 = none
 
     def _packed_nk(self) -> torch.Tensor:
         """The library-layout copy, ordered for the current stream: a repack
@@ -200,31 +208,32 @@ class W4A8Linear(torch.nn.Module):
         the caching allocator keeps the memory until that stream's work is done
         even after a later repack replaces the copy.  On the stream that made
         the copy, and whose pool it is from, both hold by stream order, but not
-        where it was made under capture: nothing has run there yet, and the
-        wait is what refuses an eager call."""
+        where it was made under capture (nothing has run there yet, and the
+        wait is what refuses an eager call) or on a stream of another library,
+        whose handle may come back for a new stream once it is destroyed (torch's
+        own are never destroyed; the id of another library's is its handle)."""
         w = self.packed_weight
         use = torch.cuda.current_stream(w.device)
         sig = (w._version, w.data_ptr(), tuple(w.shape), w.device)
-        if self._w4_nk is None or self._w4_sig != sig:
+        have = self._w4
+        if have is None or have[0] != sig:
             out = ops.repack_w4_ref(w)
             done = torch.cuda.Event()
             done.record(use)
-            self._w4_stream = (None if torch.cuda.is_current_stream_capturing()
-                               else use.cuda_stream)
-            # sig last: it is what lets another thread use the rest
-            self._w4_nk, self._w4_done, self._w4_sig = out, done, sig
+            handle = use.cuda_stream
+            if torch.cuda.is_current_stream_capturing() or (
+                    handle != 0 and getattr(use, "stream_id", None) == handle):
+                handle = None
+            self._w4 = (sig, out, done, handle)
             return out
-        if use.cuda_stream == self._w4_stream:
-            return self._w4_nk
-        use.wait_event(self._w4_done)
-        self._w4_nk.record_stream(use)
-        return self._w4_nk
+        _, copy, done, handle = have
+        if use.cuda_stream != handle:
+            use.wait_event(done)
+            copy.record_stream(use)
+        return copy
 
     def _load_from_state_dict(self, *args, **kwargs):
-        self._w4_nk = None
-        self._w4_sig = None
-        self._w4_done = None
-        self._w4_stream = None
+        self._w4 = None
         super()._load_from_state_dict(*args, **kwargs)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

@@ -2,6 +2,7 @@
 
 import os
 import struct
+import warnings
 
 import pytest
 
@@ -22,3 +23,18 @@ def test_no_thread_local_storage():
     size, count = struct.unpack_from("<HH", elf, 54)
     kinds = [struct.unpack_from("<I", elf, phoff + i * size)[0] for i in range(count)]
     assert PT_TLS not in kinds
+
+
+@pytest.mark.parametrize("there", [False, True])
+def test_linears_run_without_the_extension(monkeypatch, tmp_path, there):
+    path = tmp_path / "_cider_fast.so"
+    if there:
+        path.write_bytes(b"built against another torch")
+    monkeypatch.setattr(_lib, "FAST_PATH", str(path))
+    monkeypatch.setattr(_lib, "_fast_linear", None)
+    with pytest.warns(RuntimeWarning, match="make -C cider_amd/csrc"):
+        f = _lib.fast_linear()
+    assert f(0, None, None, None, None, 0, True) is None  # the general path
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.fast_linear() is f  # said once

@@ -2,9 +2,11 @@
 
 import os
 import struct
+import subprocess
 import warnings
 
 import pytest
+import torch
 
 from cider_amd import _lib
 
@@ -38,3 +40,26 @@ def test_linears_run_without_the_extension(monkeypatch, tmp_path, there):
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         assert _lib.fast_linear() is f  # said once
+
+
+def test_build_follows_torch(tmp_path):
+    # the extension's build: the C++ ABI of the torch that will load it, and built
+    # again where torch, Python or a flag differs from the last build
+    make = ["make", "-n", "-C", os.path.join(os.path.dirname(_lib.LIB_DIR), "csrc"),
+            f"STAMP={tmp_path}/stamp", f"OUT={tmp_path}"]
+
+    def planned(*more):
+        out = subprocess.run([*make, *more], capture_output=True, text=True, check=True).stdout
+        return [line for line in out.splitlines() if "fast_linear.cpp" in line]
+
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    first, = planned()
+    assert f"-D_GLIBCXX_USE_CXX11_ABI={abi} " in first
+    assert torch.__version__ in (tmp_path / "stamp").read_text()
+    for name in ("libcider_hip.so", "libcider_probe.so", "_cider_fast.so"):
+        (tmp_path / name).touch()
+    objects = ["-o", "libcider_hip.so", "-o", f"{tmp_path}/libcider_hip.so"]
+    assert not planned(*objects)
+    assert planned(*objects, "TORCH_VERSION=0.0")
+    os.utime(tmp_path / "_cider_fast.so")
+    assert planned(*objects, "PYINC=/elsewhere")

@@ -408,7 +408,7 @@ static int linear_w4(bool bf, const void* x_f16, const uint8_t* w4_nk, const flo
   if (try_fused_gemv(fn, x_f16, gf, cider::W_I4, cider::EPI_PC, 0, s, &rc)) return rc;
   int8_t* q;
   float* sa;
-  const int il = aligned16(x_f16) && cider::w4_wants_il(gf) ? 32 : 0;
+  const int il = cider::w4_wants_il(gf) ? 32 : 0;
   CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, bf, il));
   cider::GemmArgs g{q, w4_nk, sa, sw, nullptr, y_f16, (int)M, (int)N, (int)K, il};
   g.y_bf16 = bf;
@@ -473,13 +473,11 @@ static int linear_w4pg(bool bf, const void* x_f16, const uint8_t* w4_nk,
   cider::GemmArgs g{q, w4_nk, nullptr, scale_gn_f16, reinterpret_cast<const uint16_t*>(bias_f16),
                     y_f16, (int)M, (int)N, (int)K};
   g.y_bf16 = bf;
-  // the one-set kernel takes x reordered by parity; a scalar quantize (x not
-  // aligned) writes it in order, for the other kernels
+  // the one-set kernel takes x reordered by parity
   float* part = pg_splitk_part(g, ws, ws_bytes, group_size);
-  const bool split_il =
-      part && cider::pg_split_one_set((int)M, (int)N, (int)K, group_size);
-  if (split_il && !aligned16(x_f16)) part = nullptr;
-  if (aligned16(x_f16) && (part ? split_il : cider::w4_pg_wants_il(g, group_size))) g.x_il = 16;
+  if (part ? cider::pg_split_one_set((int)M, (int)N, (int)K, group_size)
+           : cider::w4_pg_wants_il(g, group_size))
+    g.x_il = 16;
   CIDER_TRY(quantize_into_ws(fn, x_f16, ws, M, K, s, &q, &sa, bf, g.x_il));
   g.sa = sa;
   if (part)

@@ -29,8 +29,7 @@ struct GemmArgs {
   bool y_bf16 = false, x_bf16 = false;
 };
 
-// il: the order of q's k that GemmArgs::x_il describes (K % il == 0,
-// vectorizable x and q).
+// il: the order of q's k that GemmArgs::x_il describes (K % il == 0).
 // bf: x is bf16, rounded to fp16 first.
 hipError_t launch_quantize(const uint16_t* x, int8_t* q, float* sa, int M,
                            int K, hipStream_t s, int il = 0, bool bf = false);

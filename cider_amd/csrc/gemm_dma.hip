@@ -534,7 +534,11 @@ double tile_cost(const TileCost& c, int M, int N, int nk, int cus) {
 // the ping-pong kernel was ahead everywhere.  The measured operands stayed in
 // the caches between calls; on weights that do not, the deeper rings of the
 // other tiles gain some 3 % on the ping-pong kernel (M=512 N=12288 K=2048
-// inside a model layer), hence the margin.
+// inside a model layer), hence the margin.  Where the ping-pong kernel does not
+// take the operands (a ragged shape, unaligned y or scales), 128 x 256 tiles are a
+// candidate in any number of rounds (128 x 128 tiles before; linears: M=4096
+// N=10239 K=2560 int8 156 -> 128 us, int4 187 -> 152; M=3000 N=4100 K=1040 46.3 ->
+// 35.8; M=1500 N=4095 K=4096 int4 56.7 -> 43.6).
 constexpr TileCost kTilesI8[] = {{128, 256, 0.545, 3.30, 1.685, 7.53},
                                  {128, 128, 0.326, 5.73, 2.164, 1.74},
                                  {128, 64, 0.286, 3.60, 2.427, 2.79},
@@ -542,8 +546,11 @@ constexpr TileCost kTilesI8[] = {{128, 256, 0.545, 3.30, 1.685, 7.53},
                                  {64, 64, 0.197, 2.85, 2.468, 3.36}};
 
 // int4 weights: the same rule; over 190 measured shapes 0.2 % off the best in
-// the geometric mean.  128 x 256 tiles were not ahead anywhere.
-constexpr TileCost kTilesI4[] = {{128, 128, 0.655, 4.75, 2.328, 4.35},
+// the geometric mean.  128 x 256 tiles (times of theirs not fitted, but scaled
+// from int8's) were not ahead anywhere, and are a candidate only where the
+// ping-pong kernel does not take the operands.
+constexpr TileCost kTilesI4[] = {{128, 256, 0.900, 4.00, 1.900, 7.50},
+                                 {128, 128, 0.655, 4.75, 2.328, 4.35},
                                  {128, 64, 0.373, 3.48, 2.612, 3.63},
                                  {64, 128, 0.484, 3.40, 3.137, 4.08},
                                  {64, 64, 0.348, 2.62, 3.034, 3.98}};
@@ -554,17 +561,20 @@ template <int N>
 bool pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N], const TileCost** best,
           PpPlan* pl) {
   const int cus = num_cus();
+  const bool pp = pp_supported(a, epi, wf);
   double best_cost = 1e300;
   *best = nullptr;
   for (const TileCost& c : cands) {
-    if (c.bn == 256 && (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus) continue;
+    if (c.bn == 256 && pp &&
+        (wf == W_I4 || (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus))
+      continue;
     const double cost = tile_cost(c, a.M, a.N, (a.K + 127) / 128, cus);
     if (cost < best_cost) {
       best_cost = cost;
       *best = &c;
     }
   }
-  return pp_supported(a, epi, wf) && pp_plan(a.M, a.N, a.K, wf, *pl) < 0.96 * best_cost;
+  return pp && pp_plan(a.M, a.N, a.K, wf, *pl) < 0.96 * best_cost;
 }
 
 template <int EPI>
@@ -585,6 +595,7 @@ hipError_t launch_i4(const GemmArgs& a, hipStream_t s) {
   PpPlan pl;
   const bool pp = pick(a, EPI_PC, W_I4, kTilesI4, &c, &pl);
   if (a.x_il) return pp ? launch_gemm_pp(a, EPI_PC, W_I4, pl, s) : hipErrorInvalidValue;
+  if (c->bn == 256) return run_dma<128, 256, 128, EPI_PC, W_I4>(a, s);
   if (c->bm == 128 && c->bn == 128) return run_dma<128, 128, 128, EPI_PC, W_I4>(a, s);
   if (c->bm == 128) return run_dma<128, 64, 128, EPI_PC, W_I4>(a, s);
   if (c->bn == 128) return run_dma<64, 128, 128, EPI_PC, W_I4>(a, s);

@@ -497,6 +497,13 @@ int cider_w4a8_pergroup_linear(const void* x_f16, const uint8_t* w4_nk,
                      group_size, stream);
 }
 
+int cider_linear_bf16_supported(int op, const void* x_bf16, const void* w, const void* scale,
+                                int64_t M, int64_t K, int group_size) {
+  if (M != 1 || K > kMaxDim || (op != CIDER_OP_PERCHANNEL && op != CIDER_OP_PERGROUP)) return 1;
+  return cider::mv_stream_supported(x_bf16, w, scale, (int)K,
+                                    op == CIDER_OP_PERGROUP ? group_size : 0);
+}
+
 int cider_linear_bf16(int op, const void* x_bf16, const void* w, const void* scale,
                       const void* bias_f16, void* y_bf16, void* ws, size_t ws_bytes, int64_t M,
                       int64_t N, int64_t K, int group_size, void* stream) {

@@ -79,6 +79,12 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (w.device() != dev || s.device() != dev || (has_bias && bias_in.device() != dev))
     Py_RETURN_NONE;
 
+  // before anything is allocated (and a zero bias filled) for a call that the
+  // library would turn down
+  if (bf && !cider_linear_bf16_supported((int)op, x.const_data_ptr(), w.const_data_ptr(),
+                                         s.const_data_ptr(), M, K, (int)gs))
+    Py_RETURN_NONE;
+
   at::Tensor y;
   int rc = CIDER_OK;
   bool taken = true;

@@ -84,10 +84,14 @@ class CiderLinear(torch.nn.Module):
                 return y
         orig_shape = x.shape
         x2 = x.reshape(-1, self._in_features)
+        # a contiguous copy of x may be one that the native call takes; x itself is not
+        again = bias is None or not x.is_contiguous()
         if self._mode == "per_channel":
-            y = ops.perchannel_linear(x2, self.w_int8, self.scale_w, self.bias)
+            f = ops.perchannel_linear if again else ops._perchannel_linear
+            y = f(x2, self.w_int8, self.scale_w, bias)
         else:
-            y = ops.pergroup_linear(x2, self.w_int8, self.scale_w, self.group_size, self.bias)
+            f = ops.pergroup_linear if again else ops._pergroup_linear
+            y = f(x2, self.w_int8, self.scale_w, self.group_size, bias)
         return y.reshape(*orig_shape[:-1], self._out_features)
 
     def forward_quantized(self, q: torch.Tensor, scale_a: torch.Tensor) -> torch.Tensor:

@@ -231,15 +231,18 @@ def _linear_bf16(op: int, x, w, scale, bias, M: int, N: int, K: int, gs: int, de
     """A linear on bfloat16 x with a bfloat16 result in one library call (the
     values of casting around the fp16 entry, without the cast kernels); None
     where the library has no such path (some M == 1 shapes)."""
+    if M == 1 and (K % 256 or not 1024 <= K <= 16384) and op in (_lib.CIDER_OP_PERCHANNEL,
+                                                                 _lib.CIDER_OP_PERGROUP):
+        return None  # as the library says of these, without the call
+    lib = _lib.load()
     xb = x.contiguous()
+    if not lib.cider_linear_bf16_supported(op, _ptr(xb), _ptr(w), _ptr(scale), M, K, gs):
+        return None
     y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     ws = _workspace(op, M, N, K, gs, dev)
-    rc = _lib.load().cider_linear_bf16(op, _ptr(xb), _ptr(w), _ptr(scale), _ptr(bias), _ptr(y),
-                                       _ptr(ws), _nbytes(ws), M, N, K, gs,
-                                       _stream_ptr(dev, stream))
-    if rc == _lib.CIDER_E_UNSUPPORTED:
-        return None
-    _lib.check(rc)
+    _lib.check(lib.cider_linear_bf16(op, _ptr(xb), _ptr(w), _ptr(scale), _ptr(bias), _ptr(y),
+                                     _ptr(ws), _nbytes(ws), M, N, K, gs,
+                                     _stream_ptr(dev, stream)))
     return y
 
 
@@ -279,8 +282,11 @@ def perchannel_linear(x: torch.Tensor, w: torch.Tensor, scale_w: torch.Tensor,
     with the fused per-channel epilogue.  Returns [M, N] in x's dtype.
     """
     y = _fast(_lib.CIDER_OP_PERCHANNEL, x, w, scale_w, bias, 0, stream)
-    if y is not None:
-        return y
+    return _perchannel_linear(x, w, scale_w, bias, stream) if y is None else y
+
+
+def _perchannel_linear(x, w, scale_w, bias, stream=None) -> torch.Tensor:
+    """``perchannel_linear`` of a call that ``_fast`` did not take."""
     fn = "perchannel_linear"
     dev = _require_gpu(fn, x, w, scale_w, bias)
     _check_2d(fn, "x", x, "[M,K]")
@@ -354,8 +360,11 @@ def pergroup_linear(x: torch.Tensor, w: torch.Tensor, scale_w: torch.Tensor,
     """
     del new_bias
     y = _fast(_lib.CIDER_OP_PERGROUP, x, w, scale_w, bias, group_size, stream)
-    if y is not None:
-        return y
+    return _pergroup_linear(x, w, scale_w, group_size, bias, stream) if y is None else y
+
+
+def _pergroup_linear(x, w, scale_w, group_size, bias, stream=None) -> torch.Tensor:
+    """``pergroup_linear`` of a call that ``_fast`` did not take."""
     fn = "pergroup_linear"
     dev = _require_gpu(fn, x, w, scale_w, bias)
     _check_2d(fn, "x", x, "[M,K]")

@@ -26,6 +26,11 @@ int cider_linear_bf16(int op, const void* x_bf16, const void* w, const void* sca
                       const void* bias_f16, void* y_bf16, void* ws, size_t ws_bytes,
                       int64_t M, int64_t N, int64_t K, int group_size, void* stream);
 
+/* Whether it takes such a call (1) or answers CIDER_E_UNSUPPORTED (0); asked
+ * before the result and the workspace are allocated. Reads no memory. */
+int cider_linear_bf16_supported(int op, const void* x_bf16, const void* w, const void* scale,
+                                int64_t M, int64_t K, int group_size);
+
 /* The MLP's first half in one decode (M == 1) launch: y [I] = SwiGLU of the
  * fused gate + up projection w [2I, K] (gate rows first), exactly as
  * cider_rmsnorm_mv (norm_w non-NULL; with add and sum as there) or

@@ -25,8 +25,8 @@ def test_native_call_gets_the_bias(monkeypatch, group_size, form):
     lin.bias = {"buffer": b, "parameter": torch.nn.Parameter(b), "none": None}[form]
     given = []
     monkeypatch.setattr(ops, "_fast", lambda op, x, w, s, bias, *a: given.append(bias) or x)
-    monkeypatch.setattr(ops, "perchannel_linear", lambda x, *a: x[:, :N])
-    monkeypatch.setattr(ops, "pergroup_linear", lambda x, *a: x[:, :N])
+    for general in ("perchannel_linear", "pergroup_linear"):
+        monkeypatch.setattr(ops, general, lambda x, *a: x[:, :N])
     lin(torch.zeros(2, K).half())
     assert len(given) == (form != "none")
     assert all(t is lin.bias for t in given)

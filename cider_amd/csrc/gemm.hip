@@ -377,6 +377,15 @@ bool w4_pg_wants_il(const GemmArgs& a, int gs) {
 
 hipError_t launch_gemm(const GemmArgs& a, int wf, int epi, bool sw_half,
                        int gs, hipStream_t s) {
+  // x in the order of one kernel goes to that kernel's launcher, which takes no
+  // other order, or nowhere: the kernels below would multiply the wrong k.
+  if (a.x_il != 0) {
+    if (wf == W_I4 && epi == EPI_PC && a.x_il == 32 && aligned16(a.x) && w4_wants_il(a))
+      return launch_gemm_dma(a, epi, wf, s);
+    if (wf == W_I4 && epi == EPI_PG && a.x_il == 16 && sw_half && w4_pg_wants_il(a, gs))
+      return launch_gemm_dma_pg(a, gs, sw_half, wf, s);
+    return hipErrorInvalidValue;
+  }
   // The GEMV on quantized activations for M <= 2.  At M = 3 and 4 the LDS
   // weight stream below was ahead on every shape measured (whole linears in
   // HIP graphs: per-channel N=10240 K=2560 M=4 9.9 against 13.5 us, per-group

@@ -594,7 +594,8 @@ hipError_t launch_i4(const GemmArgs& a, hipStream_t s) {
   const TileCost* c;
   PpPlan pl;
   const bool pp = pick(a, EPI_PC, W_I4, kTilesI4, &c, &pl);
-  if (a.x_il) return pp ? launch_gemm_pp(a, EPI_PC, W_I4, pl, s) : hipErrorInvalidValue;
+  if (a.x_il)
+    return pp && a.x_il == 32 ? launch_gemm_pp(a, EPI_PC, W_I4, pl, s) : hipErrorInvalidValue;
   if (c->bn == 256) return run_dma<128, 256, 128, EPI_PC, W_I4>(a, s);
   if (c->bm == 128 && c->bn == 128) return run_dma<128, 128, 128, EPI_PC, W_I4>(a, s);
   if (c->bm == 128) return run_dma<128, 64, 128, EPI_PC, W_I4>(a, s);

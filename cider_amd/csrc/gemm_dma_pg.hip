@@ -1393,12 +1393,13 @@ template <int GS, bool SWH, int WF>
 hipError_t run_pg_splitk(const GemmArgs& a, int S, float* part, hipStream_t s) {
   if constexpr (!(WF == W_I4 && GS == 256)) {
     if (pg_split_plan(a.M, a.N, a.K, GS).one_set) {
-      if (WF == W_I4 && a.x_il != 16) return hipErrorInvalidValue;
+      if (a.x_il != (WF == W_I4 ? 16 : 0)) return hipErrorInvalidValue;
       const dim3 grid(((a.M + 127) / 128) * ((a.N + 127) / 128), S);
       gemm_dma_pg16_kernel<GS, SWH, WF, 1><<<grid, 256, 0, s>>>(a, a.K / S, part);
       return hipGetLastError();
     }
   }
+  if (a.x_il != 0) return hipErrorInvalidValue;
   const PgSplitTile t = pg_split_tile(a.M, GS);
   const int bm = t.bm, bn = t.bn;
   const dim3 grid(((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn), S);
@@ -1436,6 +1437,9 @@ hipError_t launch_gemm_pg_splitk(const GemmArgs& a, int gs, bool sw_half, int wf
 }
 
 hipError_t launch_gemm_dma_pg(const GemmArgs& a, int gs, bool sw_half, int wf, hipStream_t s) {
+  // only the one-set kernel's int4 form takes reordered x
+  if (a.x_il != 0 && !(a.x_il == 16 && wf == W_I4 && pg_one_set(a, gs, sw_half, wf)))
+    return hipErrorInvalidValue;
   {
     // Mid M on small N: when the tiles below would fill at most half the
     // CUs, 64 x 64 tiles give four times as many workgroups (the group chain

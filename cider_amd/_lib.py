@@ -82,6 +82,7 @@ SIGNATURES_EXT = {
     "cider_attn_decode_rope": (_I, [_P, _P, _P, _F, _P, _P, _I64, _P, _P, _P, _P, _P, _F, _P, _SZ,
                                     _P, _I64, _I64, _I64, _I64, _P]),
     "cider_gate_up_mv": (_I, [_P, _P, _P, _P, _F, _P, _P, _P, _P, _I64, _I64, _P]),
+    "cider_gemm_tiles": (_I, [_I, _I64, _I64, _I64, _P]),
     "cider_linear_bf16_supported": (_I, [_I, _P, _P, _P, _I64, _I64, _I]),
     "cider_linear_bf16": (_I, [_I, _P, _P, _P, _P, _P, _P, _SZ, _I64, _I64, _I64, _I, _P]),
 }

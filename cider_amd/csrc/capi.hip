@@ -497,6 +497,26 @@ int cider_w4a8_pergroup_linear(const void* x_f16, const uint8_t* w4_nk,
                      group_size, stream);
 }
 
+int cider_gemm_tiles(int op, int64_t M, int64_t N, int64_t K, int tiles[4]) {
+  static const char* fn = "cider_gemm_tiles";
+  CIDER_TRY(check_dims(fn, M, N, K));
+  CIDER_TRY(need(fn, tiles, "tiles", true));
+  if (op != CIDER_OP_PERCHANNEL && op != CIDER_OP_W4A8)
+    return fail(CIDER_E_INVALID, "%s: op %d has no such GEMM", fn, op);
+  const int wf = op == CIDER_OP_W4A8 ? cider::W_I4 : cider::W_I8;
+  const cider::GemmArgs a{nullptr, nullptr, nullptr, nullptr, nullptr,
+                          nullptr, (int)M,  (int)N,  (int)K};
+  if (M <= 64 || N == 0 || !cider::gemm_dma_supported(a, cider::EPI_PC, wf))
+    return fail(CIDER_E_UNSUPPORTED, "%s: M=%lld N=%lld K=%lld runs another kernel", fn,
+                (long long)M, (long long)N, (long long)K);
+  const cider::GemmTiles t = cider::gemm_tiles(a, cider::EPI_PC, wf);
+  tiles[0] = t.pp;
+  tiles[1] = t.pp ? 64 * t.plan.mb : t.bm;
+  tiles[2] = t.pp ? 256 : t.bn;
+  tiles[3] = t.pp && t.plan.nsmall > 0 ? 64 * t.plan.ms : 0;
+  return ok();
+}
+
 int cider_linear_bf16_supported(int op, const void* x_bf16, const void* w, const void* scale,
                                 int64_t M, int64_t K, int group_size) {
   if (M != 1 || K > kMaxDim || (op != CIDER_OP_PERCHANNEL && op != CIDER_OP_PERGROUP)) return 1;

@@ -375,6 +375,20 @@ bool w4_pg_wants_il(const GemmArgs& a, int gs) {
          pg_one_set(a, gs, true, W_I4);
 }
 
+// The LDS-DMA kernels address a tile's rows as a 64-bit base plus a 32-bit
+// per-lane offset of up to 256 rows * K bytes; longer rows take the
+// register-staged kernel, whose addresses are 64-bit throughout.
+static bool off32(const GemmArgs& a) { return (int64_t)a.K * 256 < ((int64_t)1 << 32); }
+
+// Per-channel and int32: any N, and K of whole 16-byte chunks.  Whole int8
+// linears at N=4095 K=4096 / N=4096 K=4160, register-staged against LDS-DMA:
+// M=96 107 / 90 -> 15 us, M=400 123 / 103 -> 24, M=1500 127 / 106 -> 39 / 41
+// (N=509 K=5952, M=96: 147 -> 19); int4 M=1500 123 / 104 -> 61 / 63.
+bool gemm_dma_supported(const GemmArgs& a, int epi, int wf) {
+  return epi != EPI_PG && (wf == W_I8 || epi == EPI_PC) && a.K % (wf == W_I4 ? 32 : 16) == 0 &&
+         a.K >= 128 && aligned16(a.x) && aligned16(a.w) && off32(a);
+}
+
 hipError_t launch_gemm(const GemmArgs& a, int wf, int epi, bool sw_half,
                        int gs, hipStream_t s) {
   // x in the order of one kernel goes to that kernel's launcher, which takes no
@@ -395,19 +409,9 @@ hipError_t launch_gemm(const GemmArgs& a, int wf, int epi, bool sw_half,
   const bool vec = (wf == W_I4 ? a.K % 32 == 0 : a.K % 16 == 0) && a.N % 4 == 0 &&
                    aligned16(a.x) && aligned16(a.w) && aligned16(a.y) &&
                    (a.sw == nullptr || aligned16(a.sw));
-  // The LDS-DMA kernels address a tile's rows as a 64-bit base plus a 32-bit
-  // per-lane offset of up to 256 rows * K bytes; longer rows take the
-  // register-staged kernel, whose addresses are 64-bit throughout.
-  const bool off32 = (int64_t)a.K * 256 < ((int64_t)1 << 32);
-  // Per-channel and int32: any N, and K of whole 16-byte chunks.  Whole int8
-  // linears at N=4095 K=4096 / N=4096 K=4160, register-staged against LDS-DMA:
-  // M=96 107 / 90 -> 15 us, M=400 123 / 103 -> 24, M=1500 127 / 106 -> 39 / 41
-  // (N=509 K=5952, M=96: 147 -> 19); int4 M=1500 123 / 104 -> 61 / 63.
-  const bool dma = epi != EPI_PG && (wf == W_I8 || epi == EPI_PC) &&
-                   a.K % (wf == W_I4 ? 32 : 16) == 0 && a.K >= 128 && aligned16(a.x) &&
-                   aligned16(a.w) && off32;
+  const bool dma = gemm_dma_supported(a, epi, wf);
   const bool dma_pg = epi == EPI_PG && (gs == 64 || gs == 128 || (gs == 256 && wf == W_I8)) &&
-                      vec && a.K % 128 == 0 && a.K % gs == 0 && a.N % 8 == 0 && off32;
+                      vec && a.K % 128 == 0 && a.K % gs == 0 && a.N % 8 == 0 && off32(a);
   if (a.M <= 64) {
     // The LDS-DMA kernel's 64 x 64 tiles load whole weight rows (one 16-byte
     // lane after another) and beat the skinny kernel, whose MFMA operand loads

@@ -555,15 +555,12 @@ constexpr TileCost kTilesI4[] = {{128, 256, 0.900, 4.00, 1.900, 7.50},
                                  {64, 128, 0.484, 3.40, 3.137, 4.08},
                                  {64, 64, 0.348, 2.62, 3.034, 3.98}};
 
-// The best small tile and, where the ping-pong kernel takes the operands and
-// is ahead, its plan (returns true).
 template <int N>
-bool pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N], const TileCost** best,
-          PpPlan* pl) {
+GemmTiles pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N]) {
   const int cus = num_cus();
   const bool pp = pp_supported(a, epi, wf);
   double best_cost = 1e300;
-  *best = nullptr;
+  GemmTiles t;
   for (const TileCost& c : cands) {
     if (c.bn == 256 && pp &&
         (wf == W_I4 || (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus))
@@ -571,36 +568,27 @@ bool pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N], const 
     const double cost = tile_cost(c, a.M, a.N, (a.K + 127) / 128, cus);
     if (cost < best_cost) {
       best_cost = cost;
-      *best = &c;
+      t.bm = c.bm;
+      t.bn = c.bn;
     }
   }
-  return pp && pp_plan(a.M, a.N, a.K, wf, *pl) < 0.96 * best_cost;
+  t.pp = pp && pp_plan(a.M, a.N, a.K, wf, t.plan) < 0.96 * best_cost;
+  return t;
 }
 
-template <int EPI>
-hipError_t launch_i8(const GemmArgs& a, hipStream_t s) {
-  const TileCost* c;
-  PpPlan pl;
-  if (pick(a, EPI, W_I8, kTilesI8, &c, &pl)) return launch_gemm_pp(a, EPI, W_I8, pl, s);
-  if (c->bn == 256) return run_dma<128, 256, 128, EPI>(a, s);
-  if (c->bm == 128 && c->bn == 128) return run_dma<128, 128, 128, EPI>(a, s);
-  if (c->bm == 128) return run_dma<128, 64, 128, EPI>(a, s);
-  if (c->bn == 128) return run_dma<64, 128, 128, EPI>(a, s);
-  return run_dma<64, 64, 128, EPI>(a, s);
-}
-
-// x_il says that w4_wants_il chose the ping-pong kernel for this call.
-hipError_t launch_i4(const GemmArgs& a, hipStream_t s) {
-  const TileCost* c;
-  PpPlan pl;
-  const bool pp = pick(a, EPI_PC, W_I4, kTilesI4, &c, &pl);
-  if (a.x_il)
-    return pp && a.x_il == 32 ? launch_gemm_pp(a, EPI_PC, W_I4, pl, s) : hipErrorInvalidValue;
-  if (c->bn == 256) return run_dma<128, 256, 128, EPI_PC, W_I4>(a, s);
-  if (c->bm == 128 && c->bn == 128) return run_dma<128, 128, 128, EPI_PC, W_I4>(a, s);
-  if (c->bm == 128) return run_dma<128, 64, 128, EPI_PC, W_I4>(a, s);
-  if (c->bn == 128) return run_dma<64, 128, 128, EPI_PC, W_I4>(a, s);
-  return run_dma<64, 64, 128, EPI_PC, W_I4>(a, s);
+template <int EPI, int WF>
+hipError_t run_tiles(const GemmArgs& a, hipStream_t s) {
+  const GemmTiles t = gemm_tiles(a, EPI, WF);
+  // int4 weights: the ping-pong kernel takes x in its own order only, which says
+  // that w4_wants_il chose it for this call
+  const bool il = WF == W_I4 && a.x_il == 32;
+  if (a.x_il != 0 && !(il && t.pp)) return hipErrorInvalidValue;
+  if (t.pp && (il || WF == W_I8)) return launch_gemm_pp(a, EPI, WF, t.plan, s);
+  if (t.bn == 256) return run_dma<128, 256, 128, EPI, WF>(a, s);
+  if (t.bm == 128 && t.bn == 128) return run_dma<128, 128, 128, EPI, WF>(a, s);
+  if (t.bm == 128) return run_dma<128, 64, 128, EPI, WF>(a, s);
+  if (t.bn == 128) return run_dma<64, 128, 128, EPI, WF>(a, s);
+  return run_dma<64, 64, 128, EPI, WF>(a, s);
 }
 
 }  // namespace
@@ -716,22 +704,24 @@ hipError_t launch_gemm_splitk(const GemmArgs& a, int S, int32_t* part, hipStream
   return hipGetLastError();
 }
 
+GemmTiles gemm_tiles(const GemmArgs& a, int epi, int wf) {
+  return wf == W_I4 ? pick(a, epi, wf, kTilesI4) : pick(a, epi, wf, kTilesI8);
+}
+
 bool w4_wants_il(const GemmArgs& a) {
-  const TileCost* c;
-  PpPlan pl;
   // launch_gemm's conditions for the LDS-DMA kernels, above its M <= 64 rules
   if (a.M <= 64 || a.K % 128 != 0 || a.N % 8 != 0 || (int64_t)a.K * 256 >= ((int64_t)1 << 32) ||
       (((uintptr_t)a.w | (uintptr_t)a.y | (uintptr_t)a.sw) & 15) != 0)
     return false;
-  return pick(a, EPI_PC, W_I4, kTilesI4, &c, &pl);
+  return gemm_tiles(a, EPI_PC, W_I4).pp;
 }
 
 // Eligible: EPI_I32 or EPI_PC with int8 weights, EPI_PC with int4 weights;
 // K >= 128, K % 16 == 0 (int4: 32), x and w 16-byte aligned (launch_gemm checks).
 hipError_t launch_gemm_dma(const GemmArgs& a, int epi, int wf, hipStream_t s) {
-  if (wf == W_I4) return launch_i4(a, s);
-  if (epi == EPI_I32) return launch_i8<EPI_I32>(a, s);
-  return launch_i8<EPI_PC>(a, s);
+  if (wf == W_I4) return run_tiles<EPI_PC, W_I4>(a, s);
+  if (epi == EPI_I32) return run_tiles<EPI_I32, W_I8>(a, s);
+  return run_tiles<EPI_PC, W_I8>(a, s);
 }
 
 }  // namespace cider

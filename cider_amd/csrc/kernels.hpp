@@ -62,6 +62,16 @@ struct PpPlan {
 // Whether the per-channel int4 GEMM of a runs the ping-pong kernel, so that its
 // x has to be quantized with il (a.x need not hold anything yet).
 bool w4_wants_il(const GemmArgs& a);
+// The tiles launch_gemm_dma runs: the ping-pong kernel's plan, where it takes the
+// operands and is ahead (pp), else bm x bn ones.
+struct GemmTiles {
+  bool pp = false;
+  int bm = 0, bn = 0;
+  PpPlan plan{};
+};
+GemmTiles gemm_tiles(const GemmArgs& a, int epi, int wf);
+// Whether launch_gemm_dma takes a (any M).
+bool gemm_dma_supported(const GemmArgs& a, int epi, int wf);
 // Shapes and alignments it takes, the best plan for a shape (returns its
 // estimated time in us), and the launch.
 bool pp_supported(const GemmArgs& a, int epi, int wf);

@@ -19,8 +19,8 @@ DEV = "cuda"
 
 # (M, N, K); on 256 compute units, tile rows (big, small):
 SHAPES = [
-    (64, 256, 512),       # one tile of 64 rows
-    (100, 520, 640),      # 64 rows, the last tile row and column moved inside
+    (64, 256, 512),       # the smallest it takes; these three run LDS-DMA tiles
+    (100, 520, 640),
     (193, 2056, 1152),
     (1000, 6152, 512),    # 128 rows
     (1334, 6152, 640),    # 192 rows, one round
@@ -36,6 +36,11 @@ SHAPES = [
     (4096, 12296, 640),   # 256 rows, the last columns in tiles of 128 rows
 ]
 
+# 64-row tiles: rows moved inside, whole and ragged columns; int8 and int4 weights
+# (tests/test_gemm_tiles.py holds which kernel and tiles every shape here selects)
+NARROW = [(257, 12288, 512), (319, 12280, 640), (320, 12296, 2048), (129, 18944, 3584),
+          (192, 18936, 1152)]
+
 
 def ints(shape, seed):
     g = torch.Generator(device=DEV).manual_seed(seed)
@@ -46,7 +51,7 @@ def exact_product(a, b):
     return a.double() @ b.double().t().contiguous()
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("M,N,K", SHAPES + NARROW)
 def test_int32_product(M, N, K):
     a, b = ints((M, K), 1), ints((N, K), 2)
     a[0], b[-1] = -128, -128  # the largest sums
@@ -55,7 +60,7 @@ def test_int32_product(M, N, K):
 
 
 @pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("M,N,K", SHAPES + NARROW)
 def test_perchannel_epilogue(M, N, K, bias):
     g = torch.Generator(device=DEV).manual_seed(3)
     q, w = ints((M, K), 4), ints((N, K), 5)
@@ -73,7 +78,7 @@ def test_perchannel_epilogue(M, N, K, bias):
     assert torch.equal(y.isnan(), e.isnan())
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES + [(65, 256, 512), (777, 4104, 4096)])
+@pytest.mark.parametrize("M,N,K", SHAPES + NARROW + [(65, 256, 512), (777, 4104, 4096)])
 def test_int4_weights(M, N, K):
     g = torch.Generator(device=DEV).manual_seed(6)
     x = torch.randn(M, K, device=DEV, generator=g).half()
@@ -88,4 +93,21 @@ def test_int4_weights(M, N, K):
     q, sa = C.quantize_per_token(x)  # pinned to the oracle elsewhere
     e = exact_product(q, w).float() * sa[:, None]
     e = (e * sw).half()
+    assert torch.equal(y.view(torch.int16), e.view(torch.int16))
+
+
+# bf16: the fp16 result rounded once more, on every tile height
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K", NARROW + SHAPES[3:])
+def test_bf16(M, N, K, bias):
+    g = torch.Generator(device=DEV).manual_seed(7)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    w = ints((N, K), 8)
+    sw = torch.rand(N, device=DEV, generator=g) * 1e-2 + 1e-4
+    b = torch.randn(N, device=DEV, generator=g).half() if bias else None
+    y = C.perchannel_linear(x, w, sw, b)
+    q, sa = C.quantize_per_token(x.half())
+    e = exact_product(q, w).float() * sa[:, None]
+    e = e * sw
+    e = (e + (b.float() if bias else 0.0)).half().bfloat16()
     assert torch.equal(y.view(torch.int16), e.view(torch.int16))

@@ -86,9 +86,18 @@ __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
       for (int i = 0; i < QV; ++i) {
         const int e = tid + 1024 * i;
         xv[m][i] = (m < M && e < nv8) ? ld16(x16 + (size_t)m * K + 8 * e) : i32x4{0, 0, 0, 0};
-        if (p.x_bf16) xv[m][i] = bf16x8_to_f16(xv[m][i]);
-        am[m] = absmax8(xv[m][i], am[m]);
       }
+    }
+    if (p.x_bf16) {  // one test behind all loads: one per load waits for each
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < QV; ++i) xv[m][i] = bf16x8_to_f16(xv[m][i]);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int i = 0; i < QV; ++i) am[m] = absmax8(xv[m][i], am[m]);
       am[m] = wave_max(am[m]);
       if (lane == 0) red[m][wave] = am[m];
     }
@@ -292,13 +301,12 @@ hipError_t run_m(const GemmArgs& a, int wf, int epi, int gs, hipStream_t s) {
 // group order, then y = h(f32(chain * sa) (+ bias)), as the kernel above.
 // Per-channel (GS == 0): each lane sums its chunks per row (exact int32), the
 // rows' sums meet in xor butterflies, y = h(f32(f32(acc) * sa) * sw[n] (+ bias)).
-template <int R, int C, int GS, int NW>
+template <int R, int C, int GS, int NW, bool BF>
 __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __restrict__ x16,
                                                           const uint8_t* __restrict__ w,
                                                           const void* __restrict__ sw_,
                                                           const uint16_t* __restrict__ bias,
-                                                          uint16_t* __restrict__ y, int N,
-                                                          bool bf) {
+                                                          uint16_t* __restrict__ y, int N) {
   constexpr bool PG = GS > 0;
   constexpr int NT = 64 * NW;
   constexpr int RB = 1024 * C / R, K = 2 * RB;  // bytes per weight row, k per row
@@ -340,7 +348,7 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
   __builtin_amdgcn_sched_barrier(0);
 
   // per-token quantization of x (one row; bf16 is rounded to fp16 first)
-  if (bf) {
+  if constexpr (BF) {
 #pragma unroll
     for (int q = 0; q < XV; ++q) xv[q] = bf16x8_to_f16(xv[q]);
   }
@@ -416,7 +424,7 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
       float v = (float)av * sa;
       v = v * reinterpret_cast<const float*>(sw_)[n0 + lane];
       if (bias) v = v + h2f(bias[n0 + lane]);
-      y[n0 + lane] = f2o(v, bf);
+      y[n0 + lane] = f2o(v, BF);
     }
     return;
   }
@@ -431,7 +439,7 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
     for (int g = 0; g < G; ++g) chain = chain + tm[g];
     float v = chain * sa;
     if (bias) v = v + h2f(bias[n0 + lane]);
-    y[n0 + lane] = f2o(v, bf);
+    y[n0 + lane] = f2o(v, BF);
   }
 }
 
@@ -442,14 +450,14 @@ __global__ __launch_bounds__(64 * NW) void gemv1_w4_kernel(const uint16_t* __res
 // us, gs 64 10.8 -> 8.1 us; N=4096 K=12288 gs 128 11.1 -> 9.6 us, gs 64 11.9
 // -> 11.0 us; per-channel N=12288 K=4096 9.3 -> 7.4 us, N=4096 K=12288 9.2 ->
 // 8.0 us.
-template <int GS>
+template <int GS, bool BF>
 hipError_t run_gemv1_w4(const uint16_t* x, const GemmArgs& a, hipStream_t s) {
   const uint8_t* w = reinterpret_cast<const uint8_t*>(a.w);
   uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
-#define CIDER_G1(RR, CC, NWW)                                                                 \
-  case 1024 * (CC) / (RR) * 2:                                                                \
-    gemv1_w4_kernel<RR, CC, GS, NWW><<<(a.N + (NWW) * (RR) - 1) / ((NWW) * (RR)), 64 * (NWW), \
-                                       0, s>>>(x, w, a.sw, a.bias, y, a.N, a.x_bf16);         \
+#define CIDER_G1(RR, CC, NWW)                                                                      \
+  case 1024 * (CC) / (RR) * 2:                                                                     \
+    gemv1_w4_kernel<RR, CC, GS, NWW, BF><<<(a.N + (NWW) * (RR) - 1) / ((NWW) * (RR)), 64 * (NWW),  \
+                                           0, s>>>(x, w, a.sw, a.bias, y, a.N);                    \
     return hipGetLastError();
   switch (a.K) {
     CIDER_G1(4, 4, 4)   // 2048
@@ -466,6 +474,12 @@ hipError_t run_gemv1_w4(const uint16_t* x, const GemmArgs& a, hipStream_t s) {
     default: return hipErrorNotSupported;
   }
 #undef CIDER_G1
+}
+
+template <bool BF>
+hipError_t pick_gemv1_w4(const uint16_t* x, const GemmArgs& a, int epi, int gs, hipStream_t s) {
+  if (epi == EPI_PC) return run_gemv1_w4<0, BF>(x, a, s);
+  return gs == 64 ? run_gemv1_w4<64, BF>(x, a, s) : run_gemv1_w4<128, BF>(x, a, s);
 }
 
 bool gemv1_w4_supported(const GemmArgs& a, int wf, int epi, int gs) {
@@ -491,8 +505,8 @@ hipError_t launch_gemv_q(const GemmArgs& a, int wf, int epi, int gs, hipStream_t
 hipError_t launch_gemv_qx(const uint16_t* x, const GemmArgs& a, int wf, int epi, int gs,
                           hipStream_t s) {
   if (gemv1_w4_supported(a, wf, epi, gs) && ((uintptr_t)x & 15) == 0) {
-    if (epi == EPI_PC) return run_gemv1_w4<0>(x, a, s);
-    return gs == 64 ? run_gemv1_w4<64>(x, a, s) : run_gemv1_w4<128>(x, a, s);
+    if (a.x_bf16) return pick_gemv1_w4<true>(x, a, epi, gs, s);
+    return pick_gemv1_w4<false>(x, a, epi, gs, s);
   }
   GemmArgs b = a;
   b.x = reinterpret_cast<const int8_t*>(x);

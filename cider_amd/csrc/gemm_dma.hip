@@ -538,7 +538,9 @@ double tile_cost(const TileCost& c, int M, int N, int nk, int cus) {
 // take the operands (a ragged shape, unaligned y or scales), 128 x 256 tiles are a
 // candidate in any number of rounds (128 x 128 tiles before; linears: M=4096
 // N=10239 K=2560 int8 156 -> 128 us, int4 187 -> 152; M=3000 N=4100 K=1040 46.3 ->
-// 35.8; M=1500 N=4095 K=4096 int4 56.7 -> 43.6).
+// 35.8; M=1500 N=4095 K=4096 int4 56.7 -> 43.6).  Fewer than four k-stages were not
+// in the fit; there 128 x 256 tiles of one round are ahead of the ping-pong kernel
+// (M=1000 N=6152 K=256 int32: 10.9 against 13.4 us).
 constexpr TileCost kTilesI8[] = {{128, 256, 0.545, 3.30, 1.685, 7.53},
                                  {128, 128, 0.326, 5.73, 2.164, 1.74},
                                  {128, 64, 0.286, 3.60, 2.427, 2.79},
@@ -558,13 +560,12 @@ constexpr TileCost kTilesI4[] = {{128, 256, 0.900, 4.00, 1.900, 7.50},
 template <int N>
 GemmTiles pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N]) {
   const int cus = num_cus();
-  const bool pp = pp_supported(a, epi, wf);
+  const bool one_round = (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) <= cus;
+  const bool pp = pp_supported(a, epi, wf) && !(a.K < 512 && one_round);
   double best_cost = 1e300;
   GemmTiles t;
   for (const TileCost& c : cands) {
-    if (c.bn == 256 && pp &&
-        (wf == W_I4 || (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256) > cus))
-      continue;
+    if (c.bn == 256 && pp && (wf == W_I4 || !one_round)) continue;
     const double cost = tile_cost(c, a.M, a.N, (a.K + 127) / 128, cus);
     if (cost < best_cost) {
       best_cost = cost;
@@ -572,7 +573,7 @@ GemmTiles pick(const GemmArgs& a, int epi, int wf, const TileCost (&cands)[N]) {
       t.bn = c.bn;
     }
   }
-  t.pp = pp && pp_plan(a.M, a.N, a.K, wf, t.plan) < 0.96 * best_cost;
+  t.pp = pp && pp_plan(a.M, a.N, a.K, wf, epi, t.plan) < 0.96 * best_cost;
   return t;
 }
 

@@ -1,6 +1,6 @@
 // Persistent ping-pong int8 GEMM, the main path for M > 64 or so: int8 weights
 // (int32 and per-channel epilogues) and int4 weights (per-channel, the
-// reference W4A8), K % 128 == 0 and >= 512, N % 8 == 0 and >= 256.
+// reference W4A8), K % 128 == 0, N % 8 == 0 and >= 256.
 //
 // Reference semantics are those of gemm.hip (same epilogues, same fp32
 // operation order, bit-identical results):
@@ -76,7 +76,11 @@ namespace {
 constexpr int kStageBytes = 64 * 1024;   // W 32 KB (int4: 16), X up to 32 KB
 constexpr int kXBase = 32 * 1024;
 constexpr int kSclBytes = 3 * 1024;      // sw 1 KB, bias 512 B (1 KB written), sa 1 KB
-constexpr int kPpSmem = 2 * kStageBytes + 2 * kSclBytes;
+// Scale buffers: the cursor is two stages ahead and takes a tile's scales as it
+// reaches the tile, before the epilogue of the one being computed: at K = 128,
+// one stage per tile, four tiles' scales are held at once.
+constexpr int kSclBufs = 4;
+constexpr int kPpSmem = 2 * kStageBytes + kSclBufs * kSclBytes;
 
 __device__ __forceinline__ void pp_bar() { asm volatile("s_barrier" ::: "memory"); }
 __device__ __forceinline__ void pp_lgkm0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
@@ -175,17 +179,17 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
   coords(wg, m0, n0);
 
   // Load cursor: tile lt, stage lk; lx1 is the X pointer of the stage before.
-  int lt = wg, lk = 0, lpar = 0, lm0 = m0, ln0 = n0;
+  int lt = wg, lk = 0, lbuf = 0, lm0 = m0, ln0 = n0;
   const int8_t* const wp = reinterpret_cast<const int8_t*>(p.w);
   const int8_t* lw = wp + ln0 * ldw;
   const int8_t* lx = p.x + (int64_t)lm0 * K;
   const int8_t* lx1 = lx;
-  // The scales of the cursor's tile, into the scale buffer of its parity.
-  // Extra loads of some waves only make those waves' counted waits stricter.
+  // The scales of the cursor's tile, into the next scale buffer.  Extra loads of
+  // some waves only make those waves' counted waits stricter.
   auto dma_scales = [&]() {
     if constexpr (EPI == EPI_PC) {
       const uint32_t sb =
-          __builtin_amdgcn_readfirstlane(lds0 + 2 * kStageBytes + lpar * kSclBytes);
+          __builtin_amdgcn_readfirstlane(lds0 + 2 * kStageBytes + lbuf * kSclBytes);
       if (wave == 0) dma16s(reinterpret_cast<const float*>(p.sw) + ln0, lane * 16, sb);
       if (wave == 1 && p.bias) dma16s(p.bias + ln0, (lane & 31) * 16, sb + 1024);
       if (wave >= 4 && wave < 4 + MB)
@@ -203,7 +207,7 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
     } else if (lt + nwg < ntiles) {
       lt += nwg;
       lk = 0;
-      lpar ^= 1;
+      lbuf = (lbuf + 1) % kSclBufs;
       coords(lt, lm0, ln0);
       lw = wp + ln0 * ldw;
       lx = p.x + (int64_t)lm0 * K;
@@ -307,7 +311,7 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  int par = 0, b = 0;
+  int buf = 0, b = 0;
   for (int t = wg; t < ntiles; t += nwg) {
     for (int kt = 0; kt < nk; ++kt) {
       stage(b, kt == 0 && t != wg);
@@ -319,7 +323,7 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
     asm volatile("" : "+v"(le));
     const int er = wr * 16 * MB + (le & 15), ec = wc * 64 + 8 * (le >> 4);
     if constexpr (EPI == EPI_PC) {
-      const int8_t* const sc = smem + 2 * kStageBytes + par * kSclBytes;
+      const int8_t* const sc = smem + 2 * kStageBytes + buf * kSclBytes;
       const float* const ssw = reinterpret_cast<const float*>(sc) + ec;
       const uint16_t* const sbi = reinterpret_cast<const uint16_t*>(sc + 1024) + ec;
       const float* const ssa = reinterpret_cast<const float*>(sc + 2048) + er;
@@ -383,7 +387,7 @@ __device__ __forceinline__ void pp_run(const GemmArgs& p, int8_t* __restrict__ s
       }
     }
     zero_acc();
-    par ^= 1;
+    buf = (buf + 1) % kSclBufs;
     __builtin_amdgcn_sched_barrier(0);
     if (t + nwg < ntiles) coords(t + nwg, m0, n0);
   }
@@ -473,15 +477,20 @@ double plan_cost(const PpCost& c, const PpPlan& pl, int nk, int cus) {
 bool pp_supported(const GemmArgs& a, int epi, int wf) {
   // 32-bit element offsets within a tile of the output; the DMA of the scales
   // and the bias and the stores move 16 bytes per lane; 16 times the int4 weights' sums fit int32
-  return a.M >= 64 && a.N >= 256 && a.N % 8 == 0 && a.N <= (1 << 22) && a.K >= 512 &&
+  return a.M >= 64 && a.N >= 256 && a.N % 8 == 0 && a.N <= (1 << 22) && a.K >= 128 &&
          a.K % 128 == 0 && (wf == W_I8 ? epi != EPI_PG : epi == EPI_PC && a.K < (1 << 17)) &&
          (((uintptr_t)a.y | (uintptr_t)a.sw | (uintptr_t)a.bias) & 15) == 0;
 }
 
 // The cheapest of: one tile height throughout; the rows below the last whole
 // big tile in small ones; and as many whole tile columns of big tiles as fill
-// whole rounds of the CUs, the columns right of them in small ones.
-double pp_plan(int M, int N, int K, int wf, PpPlan& best) {
+// whole rounds of the CUs, the columns right of them in small ones.  One or two
+// k-stages are mostly stores: for fp16 results tiles of 128 rows then, if there is
+// more than one round, so that a tile's stores run beside the next one's loads
+// (linears, int8 / int4: M=N=8192 K=256 256 rows 60.4 / 60.0, 128 rows 45.1 / 44.1 us;
+// M=4096 N=10240 K=128 64 rows 31.5 / -, 256 rows - / 32.0, 128 rows 26.9 / 26.9).
+// int32 results were split: M=N=8192 82 -> 62 us, but M=2048 N=12288 26.4 -> 29.9.
+double pp_plan(int M, int N, int K, int wf, int epi, PpPlan& best) {
   const PpCost& c = wf == W_I4 ? kCostI4 : kCostI8;
   const int cus = num_cus(), nk = K / 128, tn = (N + 255) / 256;
   auto ceil_div = [](int x, int y) { return (x + y - 1) / y; };
@@ -500,6 +509,7 @@ double pp_plan(int M, int N, int K, int wf, PpPlan& best) {
   for (int mb = 1; mb <= 4; ++mb) {
     const int bm = 64 * mb, tm = ceil_div(M, bm);
     if (M < bm) continue;
+    if (epi == EPI_PC && nk < 3 && mb != 2 && M >= 128 && tm * tn > cus) continue;
     offer(mb, mb > 2 ? 2 : 1, tm * tn, 0, M, N);
     if (mb < 3) continue;
     const int rows = M / bm, rest = M - rows * bm;

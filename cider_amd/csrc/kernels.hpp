@@ -75,7 +75,7 @@ bool gemm_dma_supported(const GemmArgs& a, int epi, int wf);
 // Shapes and alignments it takes, the best plan for a shape (returns its
 // estimated time in us), and the launch.
 bool pp_supported(const GemmArgs& a, int epi, int wf);
-double pp_plan(int M, int N, int K, int wf, PpPlan& best);
+double pp_plan(int M, int N, int K, int wf, int epi, PpPlan& best);
 hipError_t launch_gemm_pp(const GemmArgs& a, int epi, int wf, const PpPlan& pl, hipStream_t s);
 // Split-K per-channel GEMM for shapes with few tiles (gemm_dma.hip): K slices
 // (1 = no split), the int32 partial bytes they need, and the launch (split

@@ -31,13 +31,14 @@ int cider_linear_bf16(int op, const void* x_bf16, const void* w, const void* sca
 int cider_linear_bf16_supported(int op, const void* x_bf16, const void* w, const void* scale,
                                 int64_t M, int64_t K, int group_size);
 
-/* The tiles of the GEMM that cider_perchannel_gemm and cider_int8_matmul_int32
- * (op CIDER_OP_PERCHANNEL), or cider_w4a8_linear after its quantization (op
- * CIDER_OP_W4A8), run on 16-byte aligned operands at M > 64: tiles[0] 1 for the
+/* The tiles of the GEMM that cider_perchannel_gemm (op CIDER_OP_PERCHANNEL), or
+ * cider_w4a8_linear after its quantization (op CIDER_OP_W4A8), run on 16-byte
+ * aligned operands at M > 64: tiles[0] 1 for the
  * ping-pong kernel and 0 for the LDS-DMA tiles, tiles[1] x tiles[2] rows x columns
  * of a tile, tiles[3] rows of the ping-pong kernel's small tiles beside those
  * (0: none). CIDER_E_UNSUPPORTED for a shape that runs neither. The per-channel
- * linear runs the same where it does not split K. Launches nothing. */
+ * linear runs the same where it does not split K, cider_int8_matmul_int32 from K =
+ * 384 on. Launches nothing. */
 int cider_gemm_tiles(int op, int64_t M, int64_t N, int64_t K, int tiles[4]);
 
 /* The MLP's first half in one decode (M == 1) launch: y [I] = SwiGLU of the

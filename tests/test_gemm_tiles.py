@@ -10,7 +10,7 @@ import torch
 
 from cider_amd import _lib
 
-from .test_gpu_pp import NARROW, SHAPES
+from .test_gpu_pp import NARROW, SHAPES, SHORT
 
 PC, W4 = _lib.CIDER_OP_PERCHANNEL, _lib.CIDER_OP_W4A8
 
@@ -19,7 +19,9 @@ BIG = {(1000, 6152, 512): (128, 0), (1334, 6152, 640): (192, 0), (3455, 6152, 51
        (1000, 12296, 640): (256, 0), (2500, 10248, 1152): (256, 0), (4096, 2056, 640): (192, 64),
        (1601, 6152, 640): (192, 128), (1601, 12296, 512): (192, 128), (2049, 6152, 640): (256, 64),
        (2049, 12296, 512): (256, 64), (3455, 12288, 640): (256, 128),
-       (4096, 12296, 640): (256, 128), **{s: (64, 0) for s in NARROW}}
+       (4096, 12296, 640): (256, 128), **{s: (64, 0) for s in NARROW},
+       (2500, 10248, 128): (128, 0), (4096, 4096, 128): (256, 0), (2049, 12296, 256): (128, 0),
+       (4000, 8200, 384): (192, 0), (100, 65544, 256): (64, 0)}
 LDS_DMA = [(100, 520, 640), (193, 2056, 1152)]
 
 
@@ -32,7 +34,7 @@ def tiles(op, shape):
 
 
 @pytest.mark.parametrize("op", [PC, W4])
-@pytest.mark.parametrize("shape", [s for s in SHAPES + NARROW if s in BIG])
+@pytest.mark.parametrize("shape", [s for s in SHAPES + NARROW + SHORT if s in BIG])
 def test_ping_pong(op, shape):
     assert tiles(op, shape) == (1, BIG[shape][0], 256, BIG[shape][1])
 
@@ -41,7 +43,7 @@ def test_every_height_of_the_ping_pong_kernel_is_there():
     # (4, 2), (4, 1), (3, 2), (3, 1): big and small tiles; 2 and 1 alone
     assert set(BIG.values()) == {(256, 128), (256, 64), (256, 0), (192, 128), (192, 64), (192, 0),
                                  (128, 0), (64, 0)}
-    assert set(SHAPES) == set(BIG) - set(NARROW) | set(LDS_DMA) | {(64, 256, 512)}
+    assert set(SHAPES + NARROW + SHORT) == set(BIG) | set(LDS_DMA) | {(64, 256, 512)}
 
 
 @pytest.mark.parametrize("op", [PC, W4])
@@ -51,13 +53,14 @@ def test_lds_dma(op):
     assert tiles(op, (64, 256, 512)) == _lib.CIDER_E_UNSUPPORTED
 
 
-# the headline shape, and shapes shorter than the ping-pong kernel takes
+# the headline shape, shapes that the ping-pong kernel does not take, and a short K in
+# one round of tiles
 @pytest.mark.parametrize("op,shape,expected", [
     (PC, (4096, 10240, 2560), (1, 256, 256, 128)),
-    (PC, (4096, 4096, 256), (0, 128, 256, 0)),
-    (PC, (4096, 10240, 128), (0, 128, 256, 0)),
-    (W4, (4096, 4096, 256), (0, 128, 256, 0)),
-    (W4, (4096, 10240, 128), (0, 128, 256, 0)),
+    (PC, (4096, 10239, 2560), (0, 128, 256, 0)),
+    (PC, (4096, 10240, 2576), (0, 128, 256, 0)),
+    (W4, (4096, 10239, 2560), (0, 128, 256, 0)),
+    (PC, (1000, 6152, 256), (0, 128, 256, 0)),
 ])
 def test_selected(op, shape, expected):
     assert tiles(op, shape) == expected

@@ -41,6 +41,11 @@ SHAPES = [
 NARROW = [(257, 12288, 512), (319, 12280, 640), (320, 12296, 2048), (129, 18944, 3584),
           (192, 18936, 1152)]
 
+# one, two and three k-stages per tile, several tiles per workgroup: the scales of
+# up to four tiles are held at once
+SHORT = [(2500, 10248, 128), (4096, 4096, 128), (2049, 12296, 256), (4000, 8200, 384),
+         (100, 65544, 256)]
+
 
 def ints(shape, seed):
     g = torch.Generator(device=DEV).manual_seed(seed)
@@ -51,7 +56,7 @@ def exact_product(a, b):
     return a.double() @ b.double().t().contiguous()
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES + NARROW)
+@pytest.mark.parametrize("M,N,K", SHAPES + NARROW + SHORT)
 def test_int32_product(M, N, K):
     a, b = ints((M, K), 1), ints((N, K), 2)
     a[0], b[-1] = -128, -128  # the largest sums
@@ -60,7 +65,7 @@ def test_int32_product(M, N, K):
 
 
 @pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("M,N,K", SHAPES + NARROW)
+@pytest.mark.parametrize("M,N,K", SHAPES + NARROW + SHORT)
 def test_perchannel_epilogue(M, N, K, bias):
     g = torch.Generator(device=DEV).manual_seed(3)
     q, w = ints((M, K), 4), ints((N, K), 5)
@@ -78,7 +83,7 @@ def test_perchannel_epilogue(M, N, K, bias):
     assert torch.equal(y.isnan(), e.isnan())
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES + NARROW + [(65, 256, 512), (777, 4104, 4096)])
+@pytest.mark.parametrize("M,N,K", SHAPES + NARROW + SHORT + [(65, 256, 512), (777, 4104, 4096)])
 def test_int4_weights(M, N, K):
     g = torch.Generator(device=DEV).manual_seed(6)
     x = torch.randn(M, K, device=DEV, generator=g).half()
@@ -98,7 +103,7 @@ def test_int4_weights(M, N, K):
 
 # bf16: the fp16 result rounded once more, on every tile height
 @pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("M,N,K", NARROW + SHAPES[3:])
+@pytest.mark.parametrize("M,N,K", NARROW + SHORT + SHAPES[3:])
 def test_bf16(M, N, K, bias):
     g = torch.Generator(device=DEV).manual_seed(7)
     x = torch.randn(M, K, device=DEV, generator=g).bfloat16()

@@ -10,6 +10,7 @@ pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
     import cider_amd as C
+    from cider_amd import _lib
 
 DEV = "cuda"
 
@@ -53,3 +54,67 @@ def test_x(fmt, M, N, K, dtype):
         s = (torch.rand(K // gs, N, device=DEV, generator=g) * 0.1 + 1e-3).half()
         layer = C.W4A8GroupLinear(w, s, gs)
     assert torch.equal(bits(layer(off_by_one(x))), bits(layer(x)))
+
+
+def guarded(shape, dtype):
+    """An empty result one element past an aligned address, and its buffer."""
+    n = shape[0] * shape[1]
+    buf = torch.full((n + 33,), 77, dtype=dtype, device=DEV)
+    return buf[1:1 + n].view(shape), buf
+
+
+def untouched(buf, n):
+    return bool((buf[:1] == 77).all() and (buf[1 + n:] == 77).all())
+
+
+# y and the weight scales at element alignment, N and K whole: GEMV, few rows,
+# 64 x 64 LDS-DMA tiles, larger ones, a split-K shape, a shape of the ping-pong kernel
+SHAPES = [(2, 512, 1024), (16, 4096, 512), (40, 512, 1024), (56, 1024, 512), (96, 2048, 512),
+          (300, 4096, 512), (128, 512, 8192), (1000, 6144, 512), (2500, 10248, 128)]
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_y_and_scales(M, N, K, bias):
+    g = torch.Generator(device=DEV).manual_seed(M)
+    lib = _lib.load()
+    x = torch.randn(M, K, device=DEV, generator=g).half()
+    w = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=DEV, generator=g)
+    sw = torch.rand(N, device=DEV, generator=g) * 1e-2 + 1e-4
+    b = torch.randn(N, device=DEV, generator=g).half() if bias else None
+    q, sa = C.quantize_per_token(x)
+    nb = lib.cider_workspace_bytes(_lib.CIDER_OP_PERCHANNEL, M, N, K, 0)
+    ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    expected = C.perchannel_gemm(q, sa, w, sw, b)
+
+    def run(linear, scales, bias_):
+        y, buf = guarded((M, N), torch.float16)
+        bp = bias_.data_ptr() if bias else None
+        if linear:
+            rc = lib.cider_perchannel_linear(x.data_ptr(), w.data_ptr(), scales.data_ptr(), bp,
+                                             y.data_ptr(), ws.data_ptr(), nb, M, N, K, st)
+        else:
+            rc = lib.cider_perchannel_gemm(q.data_ptr(), sa.data_ptr(), w.data_ptr(),
+                                           scales.data_ptr(), bp, y.data_ptr(), M, N, K, st)
+        assert rc == 0
+        assert torch.equal(bits(y.clone()), bits(expected)) and untouched(buf, M * N)
+
+    for linear in (False, True):
+        for scales in (sw, off_by_one(sw)):
+            run(linear, scales, b)
+        if bias:
+            run(linear, sw, off_by_one(b))
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_int32_y(M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a, b = (torch.randint(-128, 128, (n, K), dtype=torch.int8, device=DEV, generator=g)
+            for n in (M, N))
+    y, buf = guarded((M, N), torch.int32)
+    rc = _lib.load().cider_int8_matmul_int32(a.data_ptr(), b.data_ptr(), y.data_ptr(), M, N, K,
+                                             torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(y.double(), a.double() @ b.double().t().contiguous())
+    assert untouched(buf, M * N)

@@ -437,16 +437,27 @@ template <bool PG, int XM>
 hipError_t pick_stream(int K, const uint16_t* x, const int8_t* w, const float* sw,
                        const uint16_t* bias, uint16_t* y, int N, int gs, const MvProducer& pp,
                        hipStream_t s) {
-  // RMSNorm in the staging: two rows per wave at K = 4096 halve the workgroups
-  // that redo it, where three per CU are left (Qwen3-8B-shaped decode step, N =
-  // 6144: 2370 -> 2346 us; at K = 2048, N = 4096, one per CU, it lost).  A row is
-  // whole wave loads either way, so the bits do not change.
-  if constexpr (XM == XM_NORM || XM == XM_ADDNORM) {
-    if (K == 4096 && N >= 3 * num_cus() * kWpg * 2)
-      return run_stream<2, 8, PG, XM>(x, w, sw, bias, y, N, gs, pp, s);
-  }
+  // RMSNorm in the staging: two rows per wave, where the table below has one, halve
+  // the workgroups that redo it, if three per CU are left: N=6144 at K=3072 / 5120 /
+  // 8192 7.2 -> 6.5, 10.3 -> 8.9 and 14.0 -> 12.8 us (with an add; four layers' weights
+  // in turn), N=24576 20.8 -> 16.0, 31.3 -> 24.3 and 44.4 -> 37.5; Qwen3-8B-shaped
+  // decode step (K=4096, N=6144) 2370 -> 2346 us.  (One per CU, K=2048 N=4096, lost.)
+  // A row is whole wave loads either way, so the bits do not change.
 #define CIDER_MV(RR, CC) \
   case 1024 * CC / RR: return run_stream<RR, CC, PG, XM>(x, w, sw, bias, y, N, gs, pp, s)
+  if constexpr (XM == XM_NORM || XM == XM_ADDNORM) {
+    if (N >= 3 * num_cus() * kWpg * 2) {
+      switch (K) {
+        CIDER_MV(2, 6);   // 3072
+        CIDER_MV(2, 8);   // 4096
+        CIDER_MV(2, 10);  // 5120
+        CIDER_MV(2, 12);  // 6144
+        CIDER_MV(2, 14);  // 7168
+        CIDER_MV(2, 16);  // 8192
+        default: break;
+      }
+    }
+  }
   switch (K) {
     CIDER_MV(4, 4);   // 1024
     CIDER_MV(4, 5);   // 1280

@@ -73,6 +73,22 @@ def test_rmsnorm_mv_rows_per_wave(N):
     assert torch.equal(bits(y), bits(y2))
 
 
+# every K with two rows per wave, from the N where they begin (24 per compute unit)
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("K", [3072, 5120, 6144, 7168, 8192])
+@pytest.mark.parametrize("N", [6143, 6144, 6149])
+def test_rmsnorm_mv_two_rows(N, K, add):
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    lin = linear(N, K, g, True)
+    x = torch.randn(1, K, device=DEV, generator=g).half()
+    a = torch.randn(1, K, device=DEV, generator=g).half() if add else None
+    nw = torch.rand(K, device=DEV, generator=g).half() + 0.5
+    h, y = F.rmsnorm_mv(x, nw, 1e-6, lin, add=a)
+    e = F.rmsnorm_quantize(x, nw, 1e-6, add=a, want_q=False)
+    assert torch.equal(bits(h), bits(e.h))
+    assert torch.equal(bits(y), bits(lin(e.y)))
+
+
 # slot at the edges of a 128-row chunk, at the cache's last row, past the valid
 # length (written, not attended) and outside the cache; rope_row outside the
 # tables; every grouping

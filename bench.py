@@ -235,10 +235,10 @@ def main():
                     "host_wall_ms_per_step": round(wall_ms, 4),
                     "gemm_tops": round(gemm_tops, 2),
                     "frac_of_int8_peak_whole_step": round(value_tops / INT8_PEAK_TOPS, 4)},
-        "roofline": {"bound": "mfma", "kernel": gemm_kernel_name(M, N, K, dev),
+        "roofline": {"bound": "mfma", "kernel": gemm_kernel_name(M, N, K),
                      "achieved": round(gemm_tops, 2), "peak": INT8_PEAK_TOPS,
                      "unit": "TOPS", "frac": round(gemm_tops / INT8_PEAK_TOPS, 4),
-                     "traffic": load_traffic()},
+                     "traffic": load_traffic(gemm_kernel_name(M, N, K), M, N, K)},
     }
 
     if not args.no_decode:
@@ -999,47 +999,37 @@ def bench_qwen3vl(torch, args, dev):
     }), flush=True)
 
 
-# (bm, bn, rate) for int8 weights, as pick_tile in cider_amd/csrc/gemm_dma.hip
-_TILES_I8 = [(256, 256, 1.0), (128, 256, 0.87), (128, 128, 0.75), (128, 64, 0.517),
-             (64, 128, 0.508), (64, 64, 0.40), (192, 256, 0.90)]
+def gemm_kernel_name(M, N, K):
+    """The GEMM kernel that the library says it launches for this shape (int8
+    weights, per-channel), as a kernel trace names it, with its tiles."""
+    import ctypes
+
+    from cider_amd import _lib
+    t = (ctypes.c_int * 4)()
+    if _lib.load().cider_gemm_tiles(_lib.CIDER_OP_PERCHANNEL, M, N, K, t) != 0:
+        return "per-channel GEMM of few rows or long ones (launch_gemm, cider_amd/csrc/gemm.hip)"
+    pp, bm, bn, small = t
+    if pp:
+        ms = small // 64 if small else 2 if bm > 128 else 1
+        beside = " and %dx%d" % (small, bn) if small else ""
+        return "gemm_pp_kernel<%d, %d, 1, 0> (%dx%d%s tiles, persistent, 8 waves)" % (
+            bm // 64, ms, bm, bn, beside)
+    waves = 8 if bn == 256 else 4
+    return "gemm_dma_kernel<%d, %d, 128, 1, 0, %d, %s> (%dx%d tiles, %d waves)" % (
+        bm, bn, waves, "false" if K % 128 == 0 and N % 8 == 0 else "true", bm, bn, waves)
 
 
-def gemm_kernel_name(M, N, K, dev):
-    """The GEMM kernel the library's dispatcher launches for this shape
-    (int8 weights, per-channel; cider_amd/csrc/gemm_dma.hip, pick_tile)."""
-    import torch
-    cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    if K % 128 == 0 and N % 8 == 0 and M > 64:
-        best, best_cost = None, None
-        for bm, bn, rate in _TILES_I8:
-            tiles = -(-M // bm) * -(-N // bn)
-            full, rest = divmod(tiles, cus)
-            rounds = full + (0.6 + 0.4 * rest / cus if rest else 0.0)
-            cost = rounds * bm * bn / rate
-            if best_cost is None or cost < best_cost * 0.999:
-                best, best_cost = (bm, bn), cost
-        tm, tn = -(-M // 256), -(-N // 256)
-        T = tm * tn
-        R = T % cus
-        if T > cus and 0 < R and 2 * R <= cus and R % tm == 0:
-            tail = (0.6 + 0.4 * 2 * R / cus) * 128 * 256 / 0.87
-            if (T // cus) * 256 * 256 + tail < best_cost * 0.999:
-                return ("gemm_dma_mixed_kernel<PC, I8, 8> (256x256 tiles + 128x256 tiles, "
-                        "half of them first and half last, 8 waves)")
-        waves = 8 if best[1] == 256 else 4
-        return "gemm_dma_kernel<%d, %d, 128, PC, I8, %d> (%dx%d tiles, %d waves)" % (
-            best[0], best[1], waves, best[0], best[1], waves)
-    return "gemm_kernel<PC>"
-
-
-def load_traffic():
-    """HBM bytes per GEMM launch from the committed rocprofv3 PMC summary, if any."""
+def load_traffic(kernel, M, N, K):
+    """HBM bytes per launch of this kernel at this shape from the committed
+    rocprofv3 PMC summary; None where that holds another."""
     p = os.path.join(ROOT, "profiles", "gemm_pc_m4096_traffic.json")
     try:
         with open(p) as f:
-            return json.load(f).get("bytes_per_launch")
+            d = json.load(f)
     except (OSError, ValueError):
         return None
+    same = kernel.startswith(str(d.get("kernel"))) and [M, N, K] == d.get("shape")
+    return d.get("bytes_per_launch") if same else None
 
 
 if __name__ == "__main__":

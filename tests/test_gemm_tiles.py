@@ -8,6 +8,7 @@ import ctypes
 import pytest
 import torch
 
+import bench
 from cider_amd import _lib
 
 from .test_gpu_pp import NARROW, SHAPES, SHORT
@@ -64,3 +65,21 @@ def test_lds_dma(op):
 ])
 def test_selected(op, shape, expected):
     assert tiles(op, shape) == expected
+
+
+# the kernel that bench.py's line names, and the traffic it attaches to that kernel only
+@pytest.mark.parametrize("shape,kernel", [
+    ((4096, 10240, 2560), "gemm_pp_kernel<4, 2, 1, 0> (256x256 and 128x256 tiles"),
+    ((8192, 10240, 2560), "gemm_pp_kernel<4, 2, 1, 0> (256x256 tiles"),
+    ((1024, 10240, 2560), "gemm_pp_kernel<3, 1, 1, 0> (192x256 and 64x256 tiles"),
+    ((128, 10240, 2560), "gemm_dma_kernel<128, 64, 128, 1, 0, 4, false> (128x64 tiles"),
+    ((4096, 10239, 2560), "gemm_dma_kernel<128, 256, 128, 1, 0, 8, true> (128x256 tiles"),
+    ((16, 10240, 2560), "per-channel GEMM of few rows"),
+])
+def test_bench_names_the_kernel(shape, kernel):
+    tiles(PC, shape)  # skips on another number of compute units
+    name = bench.gemm_kernel_name(*shape)
+    assert name.startswith(kernel)
+    headline = shape == (4096, 10240, 2560)
+    assert (bench.load_traffic(name, *shape) is not None) == headline
+    assert bench.load_traffic("gemm_dma_mixed_kernel<1, 0, 8>", *shape) is None

@@ -10,9 +10,9 @@
 //
 // What bounds it: power.  Under a random int8 load the part lowers its clock
 // until the chip fits its power limit, so what counts is energy per product.
-// M=8192 N=10240 K=2560: the MFMAs are busy 63 % of the cycles at 1.93 GHz
-// (the 32x32x32 tiles of gemm_dma.hip that this kernel replaced: 61 % at 1.74
-// GHz); v_mfma_i32_16x16x64_i8 alone, all operands in registers, holds 1.96
+// M=8192 N=10240 K=2560: the MFMAs are busy 62 % of the cycles at 2.00 GHz
+// (the 32x32x32 tiles of gemm_dma.hip that this kernel replaced: 58 % at 1.90
+// GHz); v_mfma_i32_16x16x64_i8 alone, all operands in registers, holds 2.00
 // GHz.  Kernel times before and after, same box, outputs bit-identical:
 //   M=4096 N=10240 K=2560   100.4 ->  93.3 us (2301 TOPS)
 //   M=8192 N=10240 K=2560   196   -> 169   us (2540 TOPS)

@@ -17,19 +17,23 @@
 //     scores, its max m_c, sum l_c and unnormalised output o_c (fp32) and
 //     writes them to a workspace; a second kernel merges the chunks with the
 //     usual max-rescaling.  Each K / V byte is read once for all G heads.
-//   * scores: a thread owns 8 consecutive positions and 8 of the 128
+//   * scores: a thread owns 4 consecutive positions and 8 of the 128
 //     dimensions (one 16-byte K load per position); the 16 dimension slices
 //     are summed through LDS.
-//     What bounds a chunk once its loads are in is VALU issue at one wave per
-//     SIMD, so both products take as few operations as their roundings allow:
-//     v_fma_mix_f32 widens its fp16 operands in place.  A score's term is one
-//     of them (the product of two fp16 is exact in fp32, so the fused add
-//     rounds as a multiply and an add do); a term of P.V is one for the rounded
-//     product and an add.  v_dot2_f32_f16 and a fused P.V would be half the
-//     operations, in another rounding: the logits of a whole model move by
-//     0.5 %, and their error against 64 bits from 0.00574 to 0.00596.
-//   * P.V: a thread owns 8 dimensions (one 16-byte V load per position) and
+//   * P.V: a thread owns 4 dimensions (one 8-byte V load per position) and
 //     8 positions; the 16 position slices are summed through LDS.
+//   * What bounds a chunk once its loads are in is VALU issue, so both products
+//     take as few operations as their roundings allow: v_fma_mix_f32 widens its
+//     fp16 operands in place.  A score's term is one of them (the product of two
+//     fp16 is exact in fp32, so the fused add rounds as a multiply and an add
+//     do); a term of P.V is one for the rounded product and an add.
+//     v_dot2_f32_f16 and a fused P.V would be half the operations, in another
+//     rounding: the logits of a whole model move by 0.5 %, and their error
+//     against 64 bits from 0.00574 to 0.00596.
+//   * eight waves, two per SIMD, issue them at twice the rate of four with the
+//     same sums in the same order: Qwen3-8B-shaped decode step 2313 -> 2257 us
+//     (2252 with four waves in that other rounding, 2545 before fma_mix), 32
+//     heads at n = 2112 10.5 us (10.9, 11.9), at n = 32000 51.1 (50.4, 54.6).
 //   * the grid covers the cache capacity T; chunks at or past n exit at once
 //     (n is clamped to T).
 //   * with more than 4 query heads per KV head, the heads are split over
@@ -44,6 +48,7 @@ namespace {
 
 constexpr int kD = 128;      // head dimension
 constexpr int kChunk = 128;  // positions per workgroup
+constexpr int kThreads = 512;  // per workgroup
 
 __device__ __forceinline__ float wave_max_f(float v) {
 #pragma unroll
@@ -57,8 +62,9 @@ __device__ __forceinline__ float wave_sum_f(float v) {
   return v;
 }
 
-// element i of a vector of 8 fp16
-__device__ __forceinline__ float elem8(i32x4 v, int i) {
+// element i of a vector of fp16
+template <typename V>
+__device__ __forceinline__ float elem(V v, int i) {
   const uint32_t w = (uint32_t)v[i / 2];
   return h2f((uint16_t)(i & 1 ? w >> 16 : w & 0xffffu));
 }
@@ -67,7 +73,7 @@ __device__ __forceinline__ float elem8(i32x4 v, int i) {
 __device__ __forceinline__ float dot8(i32x4 a, i32x4 b) {
   float s = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) s = __builtin_fmaf(elem8(a, j), elem8(b, j), s);
+  for (int j = 0; j < 8; ++j) s = __builtin_fmaf(elem(a, j), elem(b, j), s);
   return s;
 }
 
@@ -84,7 +90,7 @@ __device__ __forceinline__ float dot8(i32x4 a, i32x4 b) {
 // instead of the cache rows it loaded meanwhile.  One launch less per layer; the
 // loads of the projection run beside those of the chunk.
 template <int G, int R, bool ROPE>
-__global__ __launch_bounds__(256) void attn_chunk_kernel(
+__global__ __launch_bounds__(kThreads) void attn_chunk_kernel(
     const uint16_t* __restrict__ q, uint16_t* kc, uint16_t* vc,
     const int64_t* __restrict__ n_ptr, float scale, float* __restrict__ ws, int64_t T, int nchunk,
     const DecodeRope rp) {
@@ -107,17 +113,18 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
   // depends on the other), so the chunk costs one memory latency.  Positions
   // past n (within T) are loaded and never used; 8-position groups wholly
   // past n re-load group 0 of the chunk (always valid).
-  const int tq = tid & 15, dq = tid >> 4;  // scores: 8 positions x 8 dimensions
-  const int dv = tid & 15, ts = tid >> 4;  // P.V: 8 dimensions x 8 positions
-  const int64_t tk0 = c0 + 8 * tq, tv0 = c0 + 8 * ts;
-  i32x4 kv[8], vv[8];
+  const int tq = tid & 31, dq = tid >> 5;  // scores: 4 positions x 8 dimensions
+  const int dv = tid & 31, ts = tid >> 5;  // P.V: 4 dimensions x 8 positions
+  const int64_t tk0 = c0 + 4 * tq, tv0 = c0 + 8 * ts;
+  i32x4 kv[4];
+  i32x2 vv[8];
   {
     const uint16_t* kp = kc + ((int64_t)j * T + (tk0 < n ? tk0 : c0)) * kD + 8 * dq;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) kv[i] = ld16(kp + (int64_t)i * kD);
-    const uint16_t* vp = vc + ((int64_t)j * T + (tv0 < n ? tv0 : c0)) * kD + 8 * dv;
+    for (int i = 0; i < 4; ++i) kv[i] = ld16(kp + (int64_t)i * kD);
+    const uint16_t* vp = vc + ((int64_t)j * T + (tv0 < n ? tv0 : c0)) * kD + 4 * dv;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) vv[i] = ld16(vp + (int64_t)i * kD);
+    for (int i = 0; i < 8; ++i) vv[i] = ld8(vp + (int64_t)i * kD);
   }
   if constexpr (ROPE) {
     // threads 8r .. 8r+7: query head r; 64 .. 71: the key; 128 .. 135: the value
@@ -159,34 +166,34 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
     if (mine) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        if (tk0 + i == p) kv[i] = *reinterpret_cast<const i32x4*>(&new_kv[0][8 * dq]);
-        if (tv0 + i == p) vv[i] = *reinterpret_cast<const i32x4*>(&new_kv[1][8 * dv]);
+        if (i < 4 && tk0 + i == p) kv[i % 4] = *reinterpret_cast<const i32x4*>(&new_kv[0][8 * dq]);
+        if (tv0 + i == p) vv[i] = *reinterpret_cast<const i32x2*>(&new_kv[1][4 * dv]);
       }
     }
   } else {
-    for (int e = tid; e < G * kD / 8; e += 256)
+    for (int e = tid; e < G * kD / 8; e += kThreads)
       *reinterpret_cast<i32x4*>(&qs[0][8 * e]) = ld16(q + (int64_t)y * G * kD + 8 * e);
     __syncthreads();
   }
 
   // ---- scores: thread (dq, tq) sums dimensions 8dq..8dq+7 for positions
-  // c0 + 8tq .. +7
+  // c0 + 4tq .. +3
   {
     const int64_t t0 = tk0;
-    float acc[G][8];
+    float acc[G][4];
 #pragma unroll
     for (int r = 0; r < G; ++r) {
       const i32x4 qv = *reinterpret_cast<const i32x4*>(&qs[r][8 * dq]);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[r][i] = t0 < n ? dot8(kv[i], qv) : 0.0f;
+      for (int i = 0; i < 4; ++i) acc[r][i] = t0 < n ? dot8(kv[i], qv) : 0.0f;
     }
 #pragma unroll
     for (int r = 0; r < G; ++r)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) part[dq][r][8 * tq + i] = acc[r][i];
+      for (int i = 0; i < 4; ++i) part[dq][r][4 * tq + i] = acc[r][i];
   }
   __syncthreads();
-  for (int e = tid; e < G * kChunk; e += 256) {
+  for (int e = tid; e < G * kChunk; e += kThreads) {
     const int r = e / kChunk, t = e % kChunk;
     float s = 0.0f;
 #pragma unroll
@@ -195,10 +202,10 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
   }
   __syncthreads();
 
-  // ---- chunk softmax statistics: wave w handles heads w, w + 4, ...
+  // ---- chunk softmax statistics: wave w handles head w
   {
     const int wave = tid >> 6, lane = tid & 63;
-    for (int r = wave; r < G; r += 4) {
+    for (int r = wave; r < G; r += kThreads / 64) {
       const float a = ps[r][lane], b = ps[r][lane + 64];
       const float m = wave_max_f(fmaxf(a, b));  // finite: position c0 < n is valid
       const float pa = expf(a - m), pb = expf(b - m);
@@ -214,13 +221,13 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
   __syncthreads();
 
   // ---- P.V: thread (ts, dv) sums positions 8ts..8ts+7 for dimensions
-  // 8dv..8dv+7
+  // 4dv..4dv+3
   {
-    float acc[G][8];
+    float acc[G][4];
 #pragma unroll
     for (int r = 0; r < G; ++r)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[r][i] = 0.0f;
+      for (int i = 0; i < 4; ++i) acc[r][i] = 0.0f;
     const int64_t t0 = tv0;
     if (t0 < n) {
 #pragma unroll
@@ -230,8 +237,8 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
         for (int r = 0; r < G; ++r) {
           const float p = ps[r][8 * ts + i];
 #pragma unroll
-          for (int d = 0; d < 8; ++d)  // the product rounded, then the sum
-            acc[r][d] = acc[r][d] + __builtin_fmaf(p, elem8(vv[i], d), 0.0f);
+          for (int d = 0; d < 4; ++d)  // the product rounded, then the sum
+            acc[r][d] = acc[r][d] + __builtin_fmaf(p, elem(vv[i], d), 0.0f);
         }
       }
     }
@@ -239,11 +246,11 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
 #pragma unroll
     for (int r = 0; r < G; ++r)
 #pragma unroll
-      for (int d = 0; d < 8; ++d) part[ts][r][8 * dv + d] = acc[r][d];
+      for (int d = 0; d < 4; ++d) part[ts][r][4 * dv + d] = acc[r][d];
   }
   __syncthreads();
   float* out = ws + ((int64_t)y * nchunk + c) * G * (kD + 2);
-  for (int e = tid; e < G * kD; e += 256) {
+  for (int e = tid; e < G * kD; e += kThreads) {
     const int r = e / kD, d = e % kD;
     float o = 0.0f;
 #pragma unroll
@@ -327,9 +334,9 @@ hipError_t run_attn(const uint16_t* q, uint16_t* kc, uint16_t* vc, const int64_t
   const int nchunk = (int)((T + kChunk - 1) / kChunk);
   const dim3 grid(nchunk, KV * R);
   if (rp)
-    attn_chunk_kernel<G, R, true><<<grid, 256, 0, s>>>(q, kc, vc, n, scale, ws, T, nchunk, *rp);
+    attn_chunk_kernel<G, R, true><<<grid, kThreads, 0, s>>>(q, kc, vc, n, scale, ws, T, nchunk, *rp);
   else
-    attn_chunk_kernel<G, R, false><<<grid, 256, 0, s>>>(q, kc, vc, n, scale, ws, T, nchunk,
+    attn_chunk_kernel<G, R, false><<<grid, kThreads, 0, s>>>(q, kc, vc, n, scale, ws, T, nchunk,
                                                          DecodeRope{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

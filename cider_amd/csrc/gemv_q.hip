@@ -49,7 +49,7 @@ __device__ __forceinline__ float scale1(const void* base, int64_t idx) {
 // FQ: p.x holds the fp16 activations and the workgroup quantizes them per
 // token while staging them (bit-identical to quantize_per_token: the same
 // absmax, scale and rounding helpers), so no separate quantize launch.
-template <int MT, int WF, int EPI, bool SWH, int GS, int JM, bool FQ>
+template <int MT, int WF, int EPI, bool SWH, int GS, int JM, bool FQ, bool BF>
 __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
   __shared__ float red[MT][16];
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
         xv[m][i] = (m < M && e < nv8) ? ld16(x16 + (size_t)m * K + 8 * e) : i32x4{0, 0, 0, 0};
       }
     }
-    if (p.x_bf16) {  // one test behind all loads: one per load waits for each
+    if constexpr (BF) {
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
       for (; g < G; ++g) chain = chain + tm[g];
       float v = chain * (FQ ? srow[m] : p.sa[m]);
       if (p.bias) v = v + h2f(p.bias[n]);
-      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
+      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, BF);
     }
   } else {
 #pragma unroll
@@ -225,21 +225,21 @@ __global__ __launch_bounds__(1024) void gemv_q_kernel(const GemmArgs p) {
           float v = (float)acc[m] * (FQ ? srow[m] : p.sa[m]);
           v = v * reinterpret_cast<const float*>(p.sw)[n];
           if (p.bias) v = v + h2f(p.bias[n]);
-          reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
+          reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, BF);
         }
       }
     }
   }
 }
 
-template <int MT, int WF, int EPI, bool SWH, int GS, bool FQ>
-hipError_t run_jm(const GemmArgs& a, hipStream_t s) {
+template <int MT, int WF, int EPI, bool SWH, int GS, bool FQ, bool BF>
+hipError_t run_jm_as(const GemmArgs& a, hipStream_t s) {
   const int rb = (WF == W_I4) ? a.K / 2 : a.K;
   const int per_lane = (rb / 16 + 63) / 64;
   const int GP = (EPI == EPI_PG) ? ((a.K / GS + 3) & ~3) : 0;
   const size_t lds = (size_t)MT * a.K + (size_t)kRowsPerWg * MT * GP * sizeof(float);
   const dim3 grid((a.N + kRowsPerWg - 1) / kRowsPerWg), block(64 * kRowsPerWg);
-#define CIDER_GQ(J) gemv_q_kernel<MT, WF, EPI, SWH, GS, J, FQ><<<grid, block, lds, s>>>(a)
+#define CIDER_GQ(J) gemv_q_kernel<MT, WF, EPI, SWH, GS, J, FQ, BF><<<grid, block, lds, s>>>(a)
   if (per_lane <= 2)
     CIDER_GQ(2);
   else if (per_lane <= 3)
@@ -258,6 +258,15 @@ hipError_t run_jm(const GemmArgs& a, hipStream_t s) {
     return hipErrorInvalidValue;
 #undef CIDER_GQ
   return hipGetLastError();
+}
+
+// bf16 y; with FQ bf16 x too (the callers set both)
+template <int MT, int WF, int EPI, bool SWH, int GS, bool FQ>
+hipError_t run_jm(const GemmArgs& a, hipStream_t s) {
+  if (FQ && a.x_bf16 != a.y_bf16) return hipErrorInvalidValue;
+  if constexpr (EPI != EPI_I32)
+    if (a.y_bf16) return run_jm_as<MT, WF, EPI, SWH, GS, FQ, true>(a, s);
+  return run_jm_as<MT, WF, EPI, SWH, GS, FQ, false>(a, s);
 }
 
 template <int MT, bool FQ>

@@ -40,7 +40,7 @@ __device__ __forceinline__ float load_scale1(const void* base, int64_t idx) {
 
 }  // namespace
 
-template <int TM, int WF, int EPI, bool SWH, int GS, bool VEC, int KW>
+template <int TM, int WF, int EPI, bool SWH, int GS, bool VEC, int KW, bool BF>
 __global__ __launch_bounds__(KW * 64) void skinny_kernel(const GemmArgs p) {
   // k-steps per batch: two batches in flight per lane; 16-wave workgroups
   // have 128 VGPRs per lane, which holds two batches of 6 (int4) or 4 (int8)
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_kernel(const GemmArgs p) {
         v[r] = v[r] * swn;
         if (p.bias) v[r] = v[r] + (n < N ? h2f(p.bias[n]) : 0.0f);
       }
-      const uint32_t o01 = f2o2(v[0], v[1], p.y_bf16), o23 = f2o2(v[2], v[3], p.y_bf16);
+      const uint32_t o01 = f2o2(v[0], v[1], BF), o23 = f2o2(v[2], v[3], BF);
       uint16_t* yp = reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + ncol;
       store_row(yp, N - ncol, i32x2{(int)o01, (int)o23});
     }
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_kernel(const GemmArgs p) {
 // terms in group order.  Weights and x are prefetched across rounds (two
 // register batches of RB rounds), so the barriers do not drain the stream.
 // ---------------------------------------------------------------------------
-template <int TM, int WF, bool SWH, int GS, bool VEC, int KW>
+template <int TM, int WF, bool SWH, int GS, bool VEC, int KW, bool BF>
 __global__ __launch_bounds__(KW * 64) void skinny_pg_kernel(const GemmArgs p) {
   constexpr int kThreads = KW * 64;
   constexpr int SUB = GS / 64;  // k-steps per group
@@ -333,30 +333,43 @@ __global__ __launch_bounds__(KW * 64) void skinny_pg_kernel(const GemmArgs p) {
     if (m >= M || n >= N) continue;
     float v = facc[o] * p.sa[m];
     if (p.bias) v = v + h2f(p.bias[n]);
-    reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
+    reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, BF);
   }
 }
 
 namespace {
 
-template <int TM, int WF, int EPI, bool SWH, int GS, int KW>
-hipError_t run_skinny_kw(const GemmArgs& a, bool vec, size_t lds, hipStream_t s) {
+template <int TM, int WF, int EPI, bool SWH, int GS, int KW, bool BF>
+hipError_t run_skinny_as(const GemmArgs& a, bool vec, size_t lds, hipStream_t s) {
   const int grid = (a.N + 15) / 16;
   if (vec)
-    skinny_kernel<TM, WF, EPI, SWH, GS, true, KW><<<grid, KW * 64, lds, s>>>(a);
+    skinny_kernel<TM, WF, EPI, SWH, GS, true, KW, BF><<<grid, KW * 64, lds, s>>>(a);
   else
-    skinny_kernel<TM, WF, EPI, SWH, GS, false, KW><<<grid, KW * 64, lds, s>>>(a);
+    skinny_kernel<TM, WF, EPI, SWH, GS, false, KW, BF><<<grid, KW * 64, lds, s>>>(a);
+  return hipGetLastError();
+}
+
+template <int TM, int WF, int EPI, bool SWH, int GS, int KW>
+hipError_t run_skinny_kw(const GemmArgs& a, bool vec, size_t lds, hipStream_t s) {
+  if constexpr (EPI != EPI_I32)
+    if (a.y_bf16) return run_skinny_as<TM, WF, EPI, SWH, GS, KW, true>(a, vec, lds, s);
+  return run_skinny_as<TM, WF, EPI, SWH, GS, KW, false>(a, vec, lds, s);
+}
+
+template <int TM, int WF, bool SWH, int GS, int KW, bool BF>
+hipError_t run_skinny_pg_as(const GemmArgs& a, bool vec, size_t lds, hipStream_t s) {
+  const int grid = (a.N + 15) / 16;
+  if (vec)
+    skinny_pg_kernel<TM, WF, SWH, GS, true, KW, BF><<<grid, KW * 64, lds, s>>>(a);
+  else
+    skinny_pg_kernel<TM, WF, SWH, GS, false, KW, BF><<<grid, KW * 64, lds, s>>>(a);
   return hipGetLastError();
 }
 
 template <int TM, int WF, bool SWH, int GS, int KW>
 hipError_t run_skinny_pg_kw(const GemmArgs& a, bool vec, size_t lds, hipStream_t s) {
-  const int grid = (a.N + 15) / 16;
-  if (vec)
-    skinny_pg_kernel<TM, WF, SWH, GS, true, KW><<<grid, KW * 64, lds, s>>>(a);
-  else
-    skinny_pg_kernel<TM, WF, SWH, GS, false, KW><<<grid, KW * 64, lds, s>>>(a);
-  return hipGetLastError();
+  return a.y_bf16 ? run_skinny_pg_as<TM, WF, SWH, GS, KW, true>(a, vec, lds, s)
+                  : run_skinny_pg_as<TM, WF, SWH, GS, KW, false>(a, vec, lds, s);
 }
 
 // Waves per workgroup: 4, raised to 8 or 16 while the grid has fewer than 16

@@ -97,7 +97,9 @@ __device__ __forceinline__ void wait_stage(int rem) {
 
 }  // namespace
 
-template <int RB, int MB, int NS, int WF, int EPI, int GS, bool SWH>
+// BF: y is bf16 (a template argument, here and in the other kernels of few rows: a test
+// in the epilogue costs the fp16 ones 2-3 %: int4 M=5 N=2560 K=10240 10.65 -> 10.28 us).
+template <int RB, int MB, int NS, int WF, int EPI, int GS, bool SWH, bool BF>
 __global__ __launch_bounds__((EPI == EPI_PG ? kSdKW + kSdCW : kSdKW) * 64) void skinny_dma_kernel(
     const GemmArgs p) {
   using C = SdCfg<RB, MB, NS, WF, EPI, GS, SWH>;
@@ -259,7 +261,7 @@ __global__ __launch_bounds__((EPI == EPI_PG ? kSdKW + kSdCW : kSdKW) * 64) void 
         if (p.bias) v[r] = v[r] + h2f(e_b[r]);
       }
       *reinterpret_cast<i32x2*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + ncol) =
-          i32x2{(int)f2o2(v[0], v[1], p.y_bf16), (int)f2o2(v[2], v[3], p.y_bf16)};
+          i32x2{(int)f2o2(v[0], v[1], BF), (int)f2o2(v[2], v[3], BF)};
     }
   } else {
     // ---- per-group.  Parts of a stage (int32 sums in LDS, [part][output],
@@ -352,7 +354,7 @@ __global__ __launch_bounds__((EPI == EPI_PG ? kSdKW + kSdCW : kSdKW) * 64) void 
       if (m >= M || n >= N) continue;
       float v = facc[o] * p.sa[m];
       if (p.bias) v = v + h2f(p.bias[n]);
-      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
+      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, BF);
     }
   }
 }
@@ -362,8 +364,14 @@ namespace {
 template <int RB, int MB, int WF, int EPI, int GS, bool SWH, int NS>
 hipError_t run_sd_ns(const GemmArgs& a, hipStream_t s) {
   const int rows = 16 * RB;
-  skinny_dma_kernel<RB, MB, NS, WF, EPI, GS, SWH>
-      <<<(a.N + rows - 1) / rows, (EPI == EPI_PG ? kSdKW + kSdCW : kSdKW) * 64, 0, s>>>(a);
+  const dim3 grid((a.N + rows - 1) / rows), block((EPI == EPI_PG ? kSdKW + kSdCW : kSdKW) * 64);
+  if constexpr (EPI != EPI_I32) {
+    if (a.y_bf16) {
+      skinny_dma_kernel<RB, MB, NS, WF, EPI, GS, SWH, true><<<grid, block, 0, s>>>(a);
+      return hipGetLastError();
+    }
+  }
+  skinny_dma_kernel<RB, MB, NS, WF, EPI, GS, SWH, false><<<grid, block, 0, s>>>(a);
   return hipGetLastError();
 }
 

@@ -70,7 +70,7 @@ constexpr int phase_groups(int TM, int WF, int EPI, int GS, int KW, int NB, int 
 
 }  // namespace
 
-template <int TM, int WF, int EPI, bool SWH, int GS, int KW, int NB, int RB>
+template <int TM, int WF, int EPI, bool SWH, int GS, int KW, int NB, int RB, bool BF>
 __global__ __launch_bounds__(KW * 64) void skinny_stream_kernel(const GemmArgs p) {
   constexpr int kThreads = KW * 64;
   constexpr bool PG = EPI == EPI_PG;
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_stream_kernel(const GemmArgs p
             if (p.bias) v[r] = v[r] + h2f(p.bias[ncol + r]);
           }
           *reinterpret_cast<i32x2*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)m * N + ncol) =
-              i32x2{(int)f2o2(v[0], v[1], p.y_bf16), (int)f2o2(v[2], v[3], p.y_bf16)};
+              i32x2{(int)f2o2(v[0], v[1], BF), (int)f2o2(v[2], v[3], BF)};
         }
       }
     }
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(KW * 64) void skinny_stream_kernel(const GemmArgs p
       if (m >= M || n >= N) continue;
       float v = facc[o] * p.sa[m];
       if (p.bias) v = v + h2f(p.bias[n]);
-      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, p.y_bf16);
+      reinterpret_cast<uint16_t*>(p.y)[(int64_t)m * N + n] = f2o(v, BF);
     }
   }
 }
@@ -307,8 +307,14 @@ namespace {
 
 template <int TM, int WF, int EPI, bool SWH, int GS, int KW, int NB, int RB = 1>
 hipError_t run_ss(const GemmArgs& a, hipStream_t s) {
-  skinny_stream_kernel<TM, WF, EPI, SWH, GS, KW, NB, RB>
-      <<<(a.N + 16 * RB - 1) / (16 * RB), KW * 64, 0, s>>>(a);
+  const int grid = (a.N + 16 * RB - 1) / (16 * RB);
+  if constexpr (EPI != EPI_I32) {
+    if (a.y_bf16) {
+      skinny_stream_kernel<TM, WF, EPI, SWH, GS, KW, NB, RB, true><<<grid, KW * 64, 0, s>>>(a);
+      return hipGetLastError();
+    }
+  }
+  skinny_stream_kernel<TM, WF, EPI, SWH, GS, KW, NB, RB, false><<<grid, KW * 64, 0, s>>>(a);
   return hipGetLastError();
 }
 
